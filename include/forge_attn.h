@@ -219,6 +219,26 @@ int forge_attn_prefill_docs(int dtype, int B, int T, int H, int K, int D, const 
                             const int32_t* doc_start, int64_t s_doc_b, void* out, int64_t sob,
                             int64_t sot, int64_t soh, void* stream);
 
+/*
+ * forge_attn_prefill (doc_start NULL) or forge_attn_prefill_docs with a caller-owned workspace
+ * (no counterpart in the reference): where the call's query tiles leave CUs idle -- a chunk of a
+ * long prompt, a short batch -- each tile's keys are split over several blocks, whose fp32
+ * partials meet in the workspace. forge_attn_prefill_workspace_bytes (pure host function) says
+ * how much a shape needs; 0: it is not split and the workspace may be NULL. With a NULL workspace
+ * nothing is split, nor is it with documents, whose extents the host does not know. Results
+ * differ from the unsplit call's by the order of the fp32 sums only.
+ */
+size_t forge_attn_prefill_workspace_bytes(int dtype, int B, int T, int H, int K, int D,
+                                          int64_t offset, int window);
+int forge_attn_prefill_ws(int dtype, int B, int T, int H, int K, int D, const void* q,
+                          int64_t sqb, int64_t sqh, int64_t sqt, const float* q_weight,
+                          float eps, int flags, const float* cos, const float* sin,
+                          int64_t s_cos_t, const void* k, const void* v, int64_t skb,
+                          int64_t skh, int64_t sks, int64_t offset, int window, float scale,
+                          const int32_t* doc_start, int64_t s_doc_b, void* out, int64_t sob,
+                          int64_t sot, int64_t soh, void* workspace, size_t workspace_bytes,
+                          void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -22,6 +22,14 @@ int check_launch() {
   return (int)e;
 }
 
+int device_cus() {
+  int ncu = 0, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0)
+    ncu = 256;
+  return ncu;
+}
+
 }  // namespace forge
 
 extern "C" int forge_abi_version(void) { return FORGE_ABI_VERSION; }

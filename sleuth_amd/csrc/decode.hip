@@ -2220,15 +2220,6 @@ static int64_t chunk_span(int64_t max_kv_len, int window) {
   return window > 0 && window + kMaxVerifyT < max_kv_len ? window + kMaxVerifyT : max_kv_len;
 }
 
-// CUs of the current device (256 where no device answers, e.g. a host-only build check).
-static int device_cus() {
-  int ncu = 0, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0)
-    ncu = 256;
-  return ncu;
-}
-
 // MFMA verify path: the smallest multiple of 32 keys that puts every unit into one round of
 // the device's block slots (CUs x blocks per CU): with one more unit than slots, the last
 // few full units run as a second round and double the kernel's time. (rows of T = 1, as

@@ -78,7 +78,47 @@ struct PrefillParams {
   // position doc_lo[b * sdb + t], the first of its document (non-decreasing in t); or null.
   const int32_t* doc_lo;
   int64_t sdb;
+  // Key split (launches whose query tiles leave CUs idle): a query tile's key tiles go to
+  // ceil(tiles / split_tiles) blocks, at most nsplit of them, each writing an fp32 partial
+  // (m, l, o) that prefill_combine_kernel merges. nsplit 1: no split.
+  int nsplit, split_tiles;
+  float2* ws_ml;  // [nsplit][B*H*T]
+  float* ws_o;    // [nsplit][B*H*T][D]
 };
+
+// First document position of a row's query tile (its first query's: starts do not decrease).
+__device__ __forceinline__ int first_doc(const PrefillParams& p, int b, int qt, int BM) {
+  return p.doc_lo ? p.doc_lo[b * p.sdb + (int64_t)qt * BM] : 0;
+}
+
+// Key tiles [begin, end] of query tile qt (BM queries, BN keys per tile): from its first
+// query's window or document start to its last query.
+__host__ __device__ __forceinline__ void tile_span(int64_t offset, int T, int window, int doc0, int qt, int BM,
+                                                   int BN, int& begin, int& end) {
+  const int64_t i0 = (int64_t)qt * BM;
+  const int64_t i1 = i0 + BM < T ? i0 + BM - 1 : T - 1;
+  int64_t kmin = window > 0 ? offset + i0 - window + 1 : 0;
+  if (kmin < doc0) kmin = doc0;
+  begin = (int)(kmin / BN);
+  end = (int)((offset + i1) / BN);
+}
+
+// Blocks that share a query tile of n key tiles.
+__device__ __forceinline__ int split_count(const PrefillParams& p, int n) {
+  const int c = (n + p.split_tiles - 1) / p.split_tiles;
+  return c < p.nsplit ? c : p.nsplit;
+}
+
+// This block's share of its query tile's key tiles: part `part` of split_count. False (the
+// same for the whole block) where the query tile has fewer parts.
+__device__ __forceinline__ bool take_part(const PrefillParams& p, int part, int& begin, int& end, int& parts) {
+  const int n = end - begin + 1;
+  parts = split_count(p, n);
+  if (part >= parts) return false;
+  end = begin + (int)((int64_t)(part + 1) * n / parts) - 1;
+  begin += (int)((int64_t)part * n / parts);
+  return true;
+}
 
 constexpr float kLazyLog2 = 8.0f;
 
@@ -180,7 +220,8 @@ __device__ __forceinline__ void load_q(const PrefillParams& p, int b, int h, int
     for (int e = 0; e < 8; ++e) qreg[s][e] = from_f32<T>(qf[s][e]);
 }
 
-template <typename T, int D>
+// SPLIT: the key-split launch (PrefillParams::nsplit > 1); otherwise one block per query tile.
+template <typename T, int D, bool SPLIT>
 __global__ __launch_bounds__(Tile<D>::WAVES * 64) __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2)))
 void prefill_kernel(PrefillParams p) {
   using V8 = typename Mfma<T>::vec;
@@ -202,26 +243,36 @@ void prefill_kernel(PrefillParams p) {
 
   // ---- block -> (query tile, head, batch). Heavy (late) causal tiles first. With
   // xcd_map, block i runs on XCD i % 8 and all blocks of one (b, kv head) pair share an
-  // XCD, so the K/V they all read stays in that XCD's L2.
-  int qt, b, kvh, gq;
+  // XCD, so the K/V they all read stays in that XCD's L2. A split launch does the same with
+  // (pair, part) in place of the pair: the blocks of one part read the same keys.
+  int qt, b, kvh, gq, part = 0;
   {
     const int bid = blockIdx.x;
-    const int P = p.B * p.K;
+    const int NS = SPLIT ? p.nsplit : 1;
+    const int P = p.B * p.K * NS;
     if (p.xcd_map) {
       const int x = bid & 7, local = bid >> 3;
       const int per = (P >> 3) * p.G;  // (pair, head) combinations per XCD
       const int rank = local / per, rest = local % per;
       qt = p.nqt - 1 - rank;
-      const int pair = (rest / p.G) * 8 + x;
+      int pair = (rest / p.G) * 8 + x;
       gq = rest % p.G;
+      if (SPLIT) {
+        part = pair % NS;
+        pair /= NS;
+      }
       b = pair / p.K;
       kvh = pair % p.K;
     } else {
-      const int HB = p.H * p.B;
+      const int HB = p.H * p.B * NS;
       qt = p.nqt - 1 - bid / HB;
       const int hb = bid % HB;
-      const int pair = hb % P;
+      int pair = hb % P;
       gq = hb / P;
+      if (SPLIT) {
+        part = pair % NS;
+        pair /= NS;
+      }
       b = pair / p.K;
       kvh = pair % p.K;
     }
@@ -234,20 +285,11 @@ void prefill_kernel(PrefillParams p) {
   const int64_t S = p.offset + p.T;
 
   // ---- key tiles of the block, and the first stage's loads (issued before the Q math)
-  const int64_t q_first = p.offset + (int64_t)qt * kBM;
-  const int64_t q_last_idx =
-      (int64_t)qt * kBM + kBM - 1 < p.T - 1 ? (int64_t)qt * kBM + kBM - 1 : p.T - 1;
-  const int64_t blk_kmax = p.offset + q_last_idx;
-  int64_t blk_kmin = p.window > 0 ? q_first - p.window + 1 : 0;
-  if (blk_kmin < 0) blk_kmin = 0;
-  // with documents: the block's first query starts the earliest document of the block
   const int32_t* dl = p.doc_lo ? p.doc_lo + b * p.sdb : nullptr;
-  if (dl) {
-    const int64_t d0 = __builtin_amdgcn_readfirstlane(dl[(int64_t)qt * kBM]);
-    if (d0 > blk_kmin) blk_kmin = d0;
-  }
-  const int kt_begin = (int)(blk_kmin / BN);
-  const int kt_end = (int)(blk_kmax / BN);
+  int kt_begin, kt_end, parts = 1;
+  tile_span(p.offset, p.T, p.window, __builtin_amdgcn_readfirstlane(first_doc(p, b, qt, kBM)), qt, kBM, BN,
+            kt_begin, kt_end);
+  if (SPLIT && !take_part(p, part, kt_begin, kt_end, parts)) return;
 
   const T* kg = static_cast<const T*>(p.k) + b * p.skb + kvh * p.skh;
   const T* vg = static_cast<const T*>(p.v) + b * p.skb + kvh * p.skh;
@@ -473,6 +515,19 @@ void prefill_kernel(PrefillParams p) {
 
   l_run += __shfl_xor(l_run, 32, kWave);
   if (!valid_q) return;
+  if (SPLIT && parts > 1) {  // the row's partial of this part
+    const int64_t rows = (int64_t)p.B * p.H * p.T;
+    const int64_t slot = part * rows + ((int64_t)b * p.H + h) * p.T + i_q;
+    float* po = p.ws_o + slot * D + 4 * hi;
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(po + d * 32 + 8 * i) =
+            make_float4(oacc[d][4 * i], oacc[d][4 * i + 1], oacc[d][4 * i + 2], oacc[d][4 * i + 3]);
+    if (hi == 0) p.ws_ml[slot] = make_float2(m_run, l_run);
+    return;
+  }
   const float inv_l = 1.0f / l_run;
   T* dst = static_cast<T*>(p.out) + b * p.sob + (int64_t)i_q * p.sot + h * p.soh;
 #pragma unroll
@@ -486,21 +541,85 @@ void prefill_kernel(PrefillParams p) {
     }
 }
 
+// Merges the parts of a split launch: D / 4 lanes per (b, h, t) row, four channels each, the
+// parts in order. Rows of query tiles that were not split were written by their block.
 template <typename T, int D>
-static int launch_prefill_d(PrefillParams p, hipStream_t s) {
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p, int BM, int BN) {
+  constexpr int LPR = D / 4;
+  const int64_t rows = (int64_t)p.B * p.H * p.T;
+  const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  const int x = 4 * (threadIdx.x % LPR);
+  if (row >= rows) return;
+  const int i_q = (int)(row % p.T);
+  const int64_t bh = row / p.T;
+  const int h = (int)(bh % p.H), b = (int)(bh / p.H);
+  int begin, end;
+  tile_span(p.offset, p.T, p.window, 0, i_q / BM, BM, BN, begin, end);
+  const int parts = split_count(p, end - begin + 1);
+  if (parts < 2) return;
+  float M = kNegInf;
+  for (int i = 0; i < parts; ++i) M = fmaxf(M, p.ws_ml[i * rows + row].x);
+  float L = 0.0f;
+  float4 O = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  constexpr int U = 4;  // parts whose loads go out together
+  for (int i0 = 0; i0 < parts; i0 += U) {
+    float2 ml[U];
+    float4 o[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u < parts ? i0 + u : parts - 1;
+      ml[u] = p.ws_ml[i * rows + row];
+      o[u] = *reinterpret_cast<const float4*>(p.ws_o + (i * rows + row) * D + x);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float a = i0 + u < parts ? rescale(ml[u].x, M) : 0.0f;
+      L += a * ml[u].y;
+      O.x += a * o[u].x;
+      O.y += a * o[u].y;
+      O.z += a * o[u].z;
+      O.w += a * o[u].w;
+    }
+  }
+  const float inv_l = 1.0f / L;
+  T v[4] = {from_f32<T>(O.x * inv_l), from_f32<T>(O.y * inv_l), from_f32<T>(O.z * inv_l), from_f32<T>(O.w * inv_l)};
+  T* dst = static_cast<T*>(p.out) + b * p.sob + (int64_t)i_q * p.sot + h * p.soh + x;
+  *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<uint2*>(v);
+}
+
+template <typename T, int D>
+static int launch_prefill_combine(const PrefillParams& p, int BM, int BN, hipStream_t s) {
+  constexpr int RPB = 256 / (D / 4);
+  const int64_t rows = (int64_t)p.B * p.H * p.T;
+  const int64_t blocks = (rows + RPB - 1) / RPB;
+  if (blocks > 0x7fffffff) return set_error("grid too large");
+  hipLaunchKernelGGL((prefill_combine_kernel<T, D>), dim3((unsigned)blocks), dim3(256), 0, s, p, BM, BN);
+  return check_launch();
+}
+
+template <typename T, int D, bool SPLIT>
+static int launch_prefill_s(PrefillParams p, hipStream_t s) {
   using TL = Tile<D>;
   static bool attr_set = false;  // raise the dynamic LDS limit once per kernel
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_kernel<T, D>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_kernel<T, D, SPLIT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES) != hipSuccess)
       return set_error("forge_attn_prefill: cannot reserve the LDS the kernel needs");
     attr_set = true;
   }
   p.nqt = (p.T + TL::BM - 1) / TL::BM;
-  if ((int64_t)p.nqt * p.H * p.B > 0x7fffffff) return set_error("grid too large");
-  const dim3 grid((unsigned)((int64_t)p.nqt * p.H * p.B));
-  hipLaunchKernelGGL((prefill_kernel<T, D>), grid, dim3(TL::WAVES * 64), TL::LDS_BYTES, s, p);
+  p.xcd_map = ((int64_t)p.B * p.K * p.nsplit) % 8 == 0 ? 1 : 0;
+  const int64_t blocks = (int64_t)p.nqt * p.H * p.B * p.nsplit;
+  if (blocks > 0x7fffffff) return set_error("grid too large");
+  hipLaunchKernelGGL((prefill_kernel<T, D, SPLIT>), dim3((unsigned)blocks), dim3(TL::WAVES * 64), TL::LDS_BYTES, s, p);
   return check_launch();
+}
+
+template <typename T, int D>
+static int launch_prefill_d(const PrefillParams& p, hipStream_t s) {
+  if (p.nsplit < 2) return launch_prefill_s<T, D, false>(p, s);
+  const int st = launch_prefill_s<T, D, true>(p, s);
+  return st ? st : launch_prefill_combine<T, D>(p, Tile<D>::BM, Tile<D>::BN, s);
 }
 
 // ---------------------------------------------------------------- head dim 512
@@ -532,7 +651,7 @@ struct WideTile {
   static constexpr int LDS_BYTES = STAGES * 2 * TILEB + PART_BYTES + SS_BYTES;
 };
 
-template <typename T, int SPLIT>
+template <typename T, int SPLIT, bool KSPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
 void prefill_wide_kernel(PrefillParams p) {
   using V8 = typename Mfma<T>::vec;
@@ -561,8 +680,11 @@ void prefill_wide_kernel(PrefillParams p) {
 
   // block -> (query tile, head group, batch), heavy (late) causal tiles first; wave w takes
   // slice w % SPLIT of head HPB * hg + w / SPLIT
+  // (KSPLIT: the parts of a key-split launch between the query tile and the head group)
+  const int NS = KSPLIT ? p.nsplit : 1;
   const int HB = (p.H / HPB) * p.B;
-  const int qt = p.nqt - 1 - (int)blockIdx.x / HB;
+  const int qt = p.nqt - 1 - (int)blockIdx.x / (HB * NS);
+  const int kpart = (int)blockIdx.x % (HB * NS) / HB;
   const int hb = (int)blockIdx.x % HB;
   const int b = hb % p.B;
   const int slice = wave % SPLIT;
@@ -573,21 +695,17 @@ void prefill_wide_kernel(PrefillParams p) {
   const int i_q = qt * TL::BM + n;
   const bool valid_q = i_q < p.T;
   const int64_t S = p.offset + p.T;
-  const int64_t q_first = p.offset + (int64_t)qt * TL::BM;
   const int q_last_idx = qt * TL::BM + TL::BM - 1 < p.T - 1 ? qt * TL::BM + TL::BM - 1 : p.T - 1;
-  const int64_t blk_kmax = p.offset + q_last_idx;
-  int64_t blk_kmin = p.window > 0 ? q_first - p.window + 1 : 0;
-  if (blk_kmin < 0) blk_kmin = 0;
   const int32_t* dl = p.doc_lo ? p.doc_lo + b * p.sdb : nullptr;
-  int d_lane = 0, d_first = 0, d_last = 0;
+  int d_lane = 0, d_last = 0;
   if (dl) {
     d_lane = dl[i_q < p.T ? i_q : p.T - 1];
-    d_first = __builtin_amdgcn_readfirstlane(d_lane);
     d_last = __builtin_amdgcn_readlane(d_lane, q_last_idx - qt * TL::BM);
-    if (d_first > blk_kmin) blk_kmin = d_first;
   }
-  const int kt_begin = (int)(blk_kmin / BN);
-  const int kt_end = (int)(blk_kmax / BN);
+  int kt_begin, kt_end, parts = 1;
+  tile_span(p.offset, p.T, p.window, __builtin_amdgcn_readfirstlane(first_doc(p, b, qt, TL::BM)), qt, TL::BM, BN,
+            kt_begin, kt_end);
+  if (KSPLIT && !take_part(p, kpart, kt_begin, kt_end, parts)) return;
 
   const char* kgb = reinterpret_cast<const char*>(static_cast<const T*>(p.k) + b * p.skb + kvh * p.skh);
   const char* vgb = reinterpret_cast<const char*>(static_cast<const T*>(p.v) + b * p.skb + kvh * p.skh);
@@ -806,6 +924,19 @@ void prefill_wide_kernel(PrefillParams p) {
 
   l_run += __shfl_xor(l_run, 32, kWave);
   if (!valid_q) return;
+  if (KSPLIT && parts > 1) {
+    const int64_t rows = (int64_t)p.B * p.H * p.T;
+    const int64_t slot = kpart * rows + ((int64_t)b * p.H + h) * p.T + i_q;
+    float* po = p.ws_o + slot * D + CW * slice + 4 * hi;
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(po + d * 32 + 8 * i) =
+            make_float4(oacc[d][4 * i], oacc[d][4 * i + 1], oacc[d][4 * i + 2], oacc[d][4 * i + 3]);
+    if (hi == 0 && slice == 0) p.ws_ml[slot] = make_float2(m_run, l_run);
+    return;
+  }
   const float inv_l = 1.0f / l_run;
   T* dst = static_cast<T*>(p.out) + b * p.sob + (int64_t)i_q * p.sot + h * p.soh + CW * slice;
 #pragma unroll
@@ -819,29 +950,100 @@ void prefill_wide_kernel(PrefillParams p) {
     }
 }
 
-template <typename T, int SPLIT>
+template <typename T, int SPLIT, bool KSPLIT>
 static int launch_prefill_wide_s(PrefillParams p, hipStream_t s) {
   using TL = WideTile;
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_wide_kernel<T, SPLIT>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_wide_kernel<T, SPLIT, KSPLIT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES) != hipSuccess)
       return set_error("forge_attn_prefill: cannot reserve the LDS the kernel needs");
     attr_set = true;
   }
   constexpr int HPB = TL::WAVES / SPLIT;
   p.nqt = (p.T + TL::BM - 1) / TL::BM;
-  if ((int64_t)p.nqt * (p.H / HPB) * p.B > 0x7fffffff) return set_error("grid too large");
-  const dim3 grid((unsigned)((int64_t)p.nqt * (p.H / HPB) * p.B));
-  hipLaunchKernelGGL((prefill_wide_kernel<T, SPLIT>), grid, dim3(TL::WAVES * 64), TL::LDS_BYTES, s, p);
+  const int64_t blocks = (int64_t)p.nqt * (p.H / HPB) * p.B * p.nsplit;
+  if (blocks > 0x7fffffff) return set_error("grid too large");
+  hipLaunchKernelGGL((prefill_wide_kernel<T, SPLIT, KSPLIT>), dim3((unsigned)blocks), dim3(TL::WAVES * 64),
+                     TL::LDS_BYTES, s, p);
   return check_launch();
 }
 
 // Two heads of one KV head per block (head dim in halves) where the group is even: each K/V
 // tile is loaded once for both; else one head per block in quarter slices.
 template <typename T>
-static int launch_prefill_wide(PrefillParams p, hipStream_t s) {
-  return p.G % 2 == 0 ? launch_prefill_wide_s<T, 2>(p, s) : launch_prefill_wide_s<T, 4>(p, s);
+static int launch_prefill_wide(const PrefillParams& p, hipStream_t s) {
+  if (p.nsplit < 2)
+    return p.G % 2 == 0 ? launch_prefill_wide_s<T, 2, false>(p, s) : launch_prefill_wide_s<T, 4, false>(p, s);
+  const int st = p.G % 2 == 0 ? launch_prefill_wide_s<T, 2, true>(p, s) : launch_prefill_wide_s<T, 4, true>(p, s);
+  return st ? st : launch_prefill_combine<T, 512>(p, WideTile::BM, WideTile::BN, s);
+}
+
+// How a launch splits its query tiles' keys: parts of at most `tiles` key tiles, nsplit of them
+// for the longest query tile. A launch with fewer query tiles than the CUs take (a chunk of a
+// long prompt, a short batch) otherwise leaves CUs idle behind its longest blocks: one 512-token
+// chunk at position 15,360 (16 q / 8 KV heads, head dim 128) is 64 blocks of 248 tiles.
+struct PrefillPlan {
+  int nsplit, tiles;
+};
+constexpr int kMaxParts = 32;
+
+// Picks the split with the least modelled time. Measured on calls of 1 to 32 parts (graph
+// replays, one box; the model is within 15% of each): a tile takes kTileAlone us in a block
+// that has its CU to itself and kTileShared us of a CU that holds two (head dims 64 and 128), a
+// block's q prologue and epilogue cost about 2.5 tiles, its partial crosses memory twice at
+// about 4 TB/s, and the combine launch takes 3 us. So parts pay while CUs are idle and stop
+// paying once the partials' traffic grows: 16 q / 8 KV heads, head dim 128, 1 / 2 / 4 / 8 / 16
+// parts: T 512 at 15,360: 279 / 149 / 87 / 83 / 96 us; T 128 there: 267 / 143 / 79 / 49 / 39;
+// T 64 at 1,000: 25 / 20 / 16 / 15 / 17; T 1024 at 15,360: 288 / 170 / 143 / 162 / 191; a whole
+// prompt of 2,048: 44 / 49 / 53 / 71 / 115 (not split). Head dim 256 (8 q / 4 KV), T 512 at
+// 8,000: 352 / 186 / 105 / 69 / 86.
+static PrefillPlan prefill_plan(int B, int T, int H, int K, int D, int64_t offset, int window) {
+  const bool wide = D == 512;
+  const int BM = wide ? WideTile::BM : Tile<64>::BM;
+  const int BN = wide ? WideTile::BN : D == 256 ? Tile<256>::BN : Tile<128>::BN;
+  const int hpb = wide && (H / K) % 2 == 0 ? 2 : 1;  // heads per block
+  const double alone = wide ? 2.1 : D == 256 ? 1.3 : 1.2;
+  const double shared = wide ? 2.1 : D == 256 ? 1.3 : D == 128 ? 0.95 : 0.7;
+  const int64_t cus = device_cus();
+  const int64_t heads = (int64_t)(H / hpb) * B;
+  const int nqt = (T + BM - 1) / BM;
+  if (nqt * heads >= 4 * cus) return PrefillPlan{1, 0};  // several rounds of blocks already
+  int longest = 0;
+  for (int qt = 0; qt < nqt; ++qt) {
+    int begin, end;
+    tile_span(offset, T, window, 0, qt, BM, BN, begin, end);
+    longest = end - begin + 1 > longest ? end - begin + 1 : longest;
+  }
+  PrefillPlan best{1, longest};
+  double best_us = 0.0;
+  for (int c = 1, last = 0; c <= kMaxParts; ++c) {
+    const int tiles = (longest + c - 1) / c;
+    if (tiles == last) continue;
+    last = tiles;
+    int64_t blocks = 0, split = 0, work = 0;  // blocks, those that write a partial, key tiles
+    for (int qt = 0; qt < nqt; ++qt) {
+      int begin, end;
+      tile_span(offset, T, window, 0, qt, BM, BN, begin, end);
+      const int n = end - begin + 1, parts = (n + tiles - 1) / tiles;
+      blocks += parts;
+      if (parts > 1) split += parts;
+      work += n;
+    }
+    blocks *= heads;
+    const double per_block = (double)work * heads / blocks + 2.5;
+    const int64_t rounds = (blocks + cus - 1) / cus;
+    double us = (tiles + 2.5) * alone;                       // the longest block
+    if (rounds > 1 && rounds * per_block * shared > us) us = rounds * per_block * shared;
+    if (split) us += 3.0 + 2.0 * split * heads * hpb * BM * D * sizeof(float) / 4e6;
+    // (leaving the unsplit launch has to be worth more than the model's error)
+    if (c == 1 || us < (best.nsplit == 1 ? 0.85 : 0.95) * best_us) {
+      best = PrefillPlan{c, tiles};
+      best_us = us;
+    }
+  }
+  best.nsplit = best.nsplit > 1 ? (longest + best.tiles - 1) / best.tiles : 1;
+  return best;
 }
 
 template <typename T>
@@ -859,12 +1061,19 @@ static int launch_prefill(const PrefillParams& p, int D, hipStream_t s) {
 
 using namespace forge;
 
+// fp32 (m, l) pairs and partial outputs of every part of every row
+static size_t prefill_workspace(const PrefillPlan& plan, int B, int T, int H, int D) {
+  const size_t slots = (size_t)plan.nsplit * B * H * T;
+  return (slots * sizeof(float2) + 255) / 256 * 256 + slots * D * sizeof(float);
+}
+
 static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void* q, int64_t sqb,
                         int64_t sqh, int64_t sqt, const float* q_weight, float eps, int flags,
                         const float* cos, const float* sin, int64_t s_cos_t, const void* k,
                         const void* v, int64_t skb, int64_t skh, int64_t sks, int64_t offset,
                         int window, float scale, void* out, int64_t sob, int64_t sot, int64_t soh,
-                        const int32_t* doc_lo, int64_t sdb, void* stream) {
+                        const int32_t* doc_lo, int64_t sdb, void* workspace, size_t workspace_bytes,
+                        void* stream) {
   if (dtype != FORGE_BF16 && dtype != FORGE_F16)
     return set_error("forge_attn_prefill: dtype must be bf16 or fp16 (use forge_attn_decode)");
   if (D != 64 && D != 128 && D != 256 && D != 512)
@@ -906,7 +1115,6 @@ static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void
   p.H = H;
   p.K = K;
   p.G = H / K;
-  p.xcd_map = (B * K) % 8 == 0 ? 1 : 0;
   p.window = window;
   p.scale_log2 = scale * kLog2e;
   p.out = out;
@@ -915,6 +1123,18 @@ static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void
   p.soh = soh;
   p.doc_lo = doc_lo;
   p.sdb = sdb;
+  p.nsplit = 1;
+  if (workspace && !doc_lo) {
+    const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window);
+    if (plan.nsplit > 1) {
+      if (workspace_bytes < prefill_workspace(plan, B, T, H, D)) return set_error("workspace too small");
+      p.nsplit = plan.nsplit;
+      p.split_tiles = plan.tiles;
+      const int64_t slots = (int64_t)plan.nsplit * B * H * T;
+      p.ws_ml = static_cast<float2*>(workspace);
+      p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + ((size_t)slots * sizeof(float2) + 255) / 256 * 256);
+    }
+  }
   hipStream_t s = (hipStream_t)stream;
   return dtype == FORGE_BF16 ? launch_prefill<bf16>(p, D, s) : launch_prefill<f16>(p, D, s);
 }
@@ -929,7 +1149,7 @@ extern "C" int forge_attn_prefill(int dtype, int B, int T, int H, int K, int D, 
   clear_error();
   return prefill_call(dtype, B, T, H, K, D, q, sqb, sqh, sqt, q_weight, eps, flags, cos, sin,
                       s_cos_t, k, v, skb, skh, sks, offset, window, scale, out, sob, sot, soh,
-                      nullptr, 0, stream);
+                      nullptr, 0, nullptr, 0, stream);
 }
 
 extern "C" int forge_attn_prefill_docs(int dtype, int B, int T, int H, int K, int D,
@@ -945,5 +1165,29 @@ extern "C" int forge_attn_prefill_docs(int dtype, int B, int T, int H, int K, in
   if ((uintptr_t)doc_start % 4) return set_error("forge_attn_prefill_docs: doc_start must be 4-byte aligned");
   return prefill_call(dtype, B, T, H, K, D, q, sqb, sqh, sqt, q_weight, eps, flags, cos, sin,
                       s_cos_t, k, v, skb, skh, sks, offset, window, scale, out, sob, sot, soh,
-                      doc_start, s_doc_b, stream);
+                      doc_start, s_doc_b, nullptr, 0, stream);
+}
+
+extern "C" size_t forge_attn_prefill_workspace_bytes(int dtype, int B, int T, int H, int K, int D,
+                                                     int64_t offset, int window) {
+  if ((dtype != FORGE_BF16 && dtype != FORGE_F16) || (D != 64 && D != 128 && D != 256 && D != 512) || B <= 0 ||
+      T <= 0 || H <= 0 || K <= 0 || H % K || offset < 0 || window < 0 || offset + (int64_t)T + 256 >= (1LL << 31))
+    return 0;
+  const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window);
+  return plan.nsplit > 1 ? prefill_workspace(plan, B, T, H, D) : 0;
+}
+
+extern "C" int forge_attn_prefill_ws(int dtype, int B, int T, int H, int K, int D, const void* q, int64_t sqb,
+                                     int64_t sqh, int64_t sqt, const float* q_weight, float eps, int flags,
+                                     const float* cos, const float* sin, int64_t s_cos_t, const void* k,
+                                     const void* v, int64_t skb, int64_t skh, int64_t sks, int64_t offset,
+                                     int window, float scale, const int32_t* doc_start, int64_t s_doc_b,
+                                     void* out, int64_t sob, int64_t sot, int64_t soh, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+  clear_error();
+  if ((uintptr_t)doc_start % 4) return set_error("forge_attn_prefill_ws: doc_start must be 4-byte aligned");
+  if ((uintptr_t)workspace % 16) return set_error("forge_attn_prefill_ws: the workspace must be 16-byte aligned");
+  return prefill_call(dtype, B, T, H, K, D, q, sqb, sqh, sqt, q_weight, eps, flags, cos, sin,
+                      s_cos_t, k, v, skb, skh, sks, offset, window, scale, out, sob, sot, soh,
+                      doc_start, s_doc_b, workspace, workspace_bytes, stream);
 }

@@ -386,30 +386,28 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: fl
         out = torch.empty(B, T, H, D, dtype=q.dtype, device=dev)
     elif out.shape != (B, T, H, D) or out.dtype != q.dtype:
         raise ValueError(f"out must be [B,T,H,D] = {(B, T, H, D)} {q.dtype}")
-    if doc_start is None:
-        st = lib().forge_attn_prefill(dtype_code(q), B, T, H, K, D, _ptr(q), q.stride(0), q.stride(1),
-                                      q.stride(2), _ptr(w), float(eps), flags, _ptr(c), _ptr(s), s_t,
-                                      _ptr(k), _ptr(v), k.stride(0), k.stride(1), k.stride(2),
-                                      int(offset), int(window), float(scale),
-                                      _ptr(out), out.stride(0), out.stride(1), out.stride(2), _stream(dev))
-        check(st, "forge_attn_prefill")
-        return out
-    if doc_start.dtype != torch.int32 or doc_start.shape != (B, T) or doc_start.device != dev:
-        raise ValueError(f"doc_start must be int32 [B, T] = {(B, T)} on {dev}")
-    if doc_start.stride(1) != 1:
-        raise ValueError("doc_start: the last dimension must be contiguous")
-    if check_doc_start and not torch.cuda.is_current_stream_capturing():
-        pos = offset + torch.arange(T, device=dev, dtype=torch.int32)
-        if bool(((doc_start < 0) | (doc_start > pos)).any()) or \
-                bool((doc_start[:, 1:] < doc_start[:, :-1]).any()):
-            raise ValueError("doc_start must be non-decreasing and in [0, the query's position]")
-    st = lib().forge_attn_prefill_docs(dtype_code(q), B, T, H, K, D, _ptr(q), q.stride(0), q.stride(1),
-                                       q.stride(2), _ptr(w), float(eps), flags, _ptr(c), _ptr(s), s_t,
-                                       _ptr(k), _ptr(v), k.stride(0), k.stride(1), k.stride(2),
-                                       int(offset), int(window), float(scale), _ptr(doc_start),
-                                       doc_start.stride(0), _ptr(out), out.stride(0), out.stride(1),
-                                       out.stride(2), _stream(dev))
-    check(st, "forge_attn_prefill_docs")
+    doc_ptr, doc_stride = None, 0
+    if doc_start is not None:
+        if doc_start.dtype != torch.int32 or doc_start.shape != (B, T) or doc_start.device != dev:
+            raise ValueError(f"doc_start must be int32 [B, T] = {(B, T)} on {dev}")
+        if doc_start.stride(1) != 1:
+            raise ValueError("doc_start: the last dimension must be contiguous")
+        if check_doc_start and not torch.cuda.is_current_stream_capturing():
+            pos = offset + torch.arange(T, device=dev, dtype=torch.int32)
+            if bool(((doc_start < 0) | (doc_start > pos)).any()) or \
+                    bool((doc_start[:, 1:] < doc_start[:, :-1]).any()):
+                raise ValueError("doc_start must be non-decreasing and in [0, the query's position]")
+        doc_ptr, doc_stride = _ptr(doc_start), doc_start.stride(0)
+    # partials of a key-split launch (0: the shape is not split)
+    need = 0 if doc_ptr else lib().forge_attn_prefill_workspace_bytes(dtype_code(q), B, T, H, K, D, int(offset), int(window))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    st = lib().forge_attn_prefill_ws(dtype_code(q), B, T, H, K, D, _ptr(q), q.stride(0), q.stride(1),
+                                     q.stride(2), _ptr(w), float(eps), flags, _ptr(c), _ptr(s), s_t,
+                                     _ptr(k), _ptr(v), k.stride(0), k.stride(1), k.stride(2),
+                                     int(offset), int(window), float(scale), doc_ptr, doc_stride,
+                                     _ptr(out), out.stride(0), out.stride(1), out.stride(2), _ptr(ws), need,
+                                     _stream(dev))
+    check(st, "forge_attn_prefill")
     return out
 
 

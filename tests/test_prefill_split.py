@@ -1,0 +1,116 @@
+"""The key-split prefill launch (forge_attn_prefill_ws): when it splits, and its results at the
+edges of its parts, tiles and windows against the oracle and the unsplit launch."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import oracle
+from conftest import gpu_available
+from helpers import gen, max_abs, randn, scale_of, tables, tol
+from sleuth_amd import _lib
+
+DEV = "cuda"
+
+
+def _bytes(B, T, H, K, D, offset, window=0, dtype=_lib.BF16):
+    return _lib.lib().forge_attn_prefill_workspace_bytes(dtype, B, T, H, K, D, offset, window)
+
+
+def test_split_rule():
+    """Chunks of long prompts split (each partial: D + 2 floats per row and part); launches that
+    fill the CUs do not, nor short prompts, and refused shapes need nothing."""
+    row = 512 * 16
+    need = _bytes(1, 512, 16, 8, 128, 15360)
+    parts = need // (row * (128 + 2) * 4)
+    assert 2 <= parts <= 32 and need == parts * row * 4 * (128 + 2)
+    assert _bytes(1, 64, 16, 8, 128, 1000) > 0 and _bytes(1, 600, 16, 1, 512, 8000) > 0
+    assert _bytes(4, 4096, 16, 8, 128, 0) == 0      # 2,048 query tiles
+    assert _bytes(1, 2048, 16, 8, 128, 0) == 0      # the partials would cost what the split saves
+    assert _bytes(1, 333, 16, 8, 128, 0) == 0
+    assert _bytes(1, 512, 16, 8, 128, 15360, window=64) == 0   # few keys per query
+    assert _bytes(1, 512, 16, 8, 128, 15360, dtype=_lib.F32) == 0
+    assert _bytes(1, 512, 16, 8, 32, 15360) == 0 and _bytes(1, 512, 16, 3, 128, 15360) == 0
+
+
+def test_workspace_too_small_is_rejected():
+    lib = _lib.lib()
+    need = _bytes(1, 512, 16, 8, 128, 15360)
+    args = [_lib.BF16, 1, 512, 16, 8, 128, 4096, 0, 128, 2048, None, 1e-6, 0, None, None, 0, 4096, 4096, 0, 128, 1024,
+            15360, 0, 1.0, None, 0, 4096, 0, 128, 2048]
+    assert lib.forge_attn_prefill_ws(*args, 4096, need - 1, None) < 0
+    assert b"workspace" in lib.forge_last_error()
+    assert lib.forge_attn_prefill_ws(*args, 4104, need, None) < 0
+
+
+CASES = [
+    # dtype, B, T, H, K, D, offset, window: one query; one tile and a query; odd group; windows
+    # whose first part starts inside a tile and whose parts hold no key of some queries; hd 512 with
+    # two heads per block and (odd group) one
+    (torch.bfloat16, 1, 1, 4, 2, 128, 4095, 0),
+    (torch.bfloat16, 1, 17, 16, 8, 128, 3001, 0),
+    (torch.float16, 1, 129, 6, 2, 64, 2500, 0),
+    (torch.bfloat16, 2, 200, 3, 3, 128, 1900, 0),
+    (torch.float16, 1, 257, 4, 1, 256, 1500, 0),
+    (torch.bfloat16, 1, 1800, 8, 4, 256, 0, 0),
+    (torch.bfloat16, 1, 130, 4, 2, 128, 5000, 1500),
+    (torch.float16, 1, 640, 4, 4, 64, 1000, 700),
+    (torch.bfloat16, 1, 65, 4, 1, 512, 1777, 0),
+    (torch.float16, 1, 33, 3, 1, 512, 2000, 900),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_split_prefill_against_oracle(case):
+    from sleuth_amd import ops
+
+    dtype, B, T, H, K, D, offset, window = CASES[case]
+    S = offset + T
+    g = gen(900 + case)
+    q = randn(g, B, T, H, D, dtype=dtype).transpose(1, 2)
+    w = (1 + 0.1 * randn(g, D)).to(dtype)
+    kc, vc = randn(g, B, K, S + 3, D, dtype=dtype), randn(g, B, K, S + 3, D, dtype=dtype)
+    vc[:, :, S:] = 1e4                     # positions past the call's last key are never read
+    cos, sin = (t[offset:S] for t in tables(D, S, 1e4))
+    qn = oracle.head_norm_rope(q, w, 1e-6, cos, sin)
+    ref = oracle.sdpa(qn.float(), kc[:, :, :S].float(), vc[:, :, :S].float(), offset, window, scale_of(D))
+    dev = [t.to(DEV) for t in (q, kc, vc, w, cos, sin)]
+    kw = dict(q_weight=dev[3], eps=1e-6, norm_q=True, cos=dev[4], sin=dev[5], scale=scale_of(D), offset=offset,
+              window=window)
+    assert _bytes(B, T, H, K, D, offset, window, _lib.BF16) > 0
+    got = ops.attn_prefill(*dev[:3], **kw)
+    assert max_abs(got.cpu().transpose(1, 2), ref) <= tol(dtype)
+    # the unsplit launch (documents are never split; starts of 0 hide nothing): both round the
+    # weights and the outputs once to the dtype, so each is within 2 * 2^-p of exact in 2-norm
+    # (p = 9 in bf16, 12 in fp16)
+    whole = ops.attn_prefill(*dev[:3], doc_start=torch.zeros(B, T, dtype=torch.int32, device=DEV), **kw).float()
+    eps = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+    assert ((got.float() - whole).norm() / whole.norm()).item() <= 4 * eps
+    assert torch.equal(ops.attn_prefill(*dev[:3], **kw), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+def test_split_prefill_under_graph_capture():
+    """The partials' workspace belongs to the graph: replays on new inputs equal the eager calls."""
+    from sleuth_amd import ops
+
+    B, T, H, K, D, offset = 1, 96, 8, 4, 128, 3000
+    g = gen(950)
+    q = randn(g, B, H, T, D, dtype=torch.bfloat16).to(DEV)
+    kc, vc = (randn(g, B, K, offset + T, D, dtype=torch.bfloat16).to(DEV) for _ in range(2))
+    call = lambda: ops.attn_prefill(q, kc, vc, scale=scale_of(D), offset=offset)  # noqa: E731
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for seed in range(3):
+        q.copy_(randn(gen(960 + seed), B, H, T, D, dtype=torch.bfloat16))
+        want = call()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
