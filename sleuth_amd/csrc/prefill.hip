@@ -82,6 +82,7 @@ struct PrefillParams {
   // ceil(tiles / split_tiles) blocks, at most nsplit of them, each writing an fp32 partial
   // (m, l, o) that prefill_combine_kernel merges. nsplit 1: no split.
   int nsplit, split_tiles;
+  int heads_per_block;  // prefill_wide_kernel only
   float2* ws_ml;  // [nsplit][B*H*T]
   float* ws_o;    // [nsplit][B*H*T][D]
 };
@@ -625,20 +626,26 @@ static int launch_prefill_d(const PrefillParams& p, hipStream_t s) {
 // ---------------------------------------------------------------- head dim 512
 // Head dim 512 (Gemma 4's full-attention layers: 1 KV head of 512, reference
 // kv_cache.py:12-13). A wave's 32 queries would need 128 registers of Q^T and 256 of output
-// accumulators, so here the head dim is split over the block instead: a block of 4 waves
-// owns 32 queries of one (b, head), and wave w holds channels 128w .. 128w + 127 of Q^T and
-// of the output. Per key tile (32 keys, two LDS stages of 32 KB K + 32 KB V):
-//   * each wave computes the partial scores of its channels, S_w^T = K[:, slice] . Q^T[slice]
-//     (8 MFMAs), and stores them in LDS; after a barrier every wave adds the four partials
-//     in the same order (waves 0..3), so all waves hold identical scores;
-//   * every wave runs the same online softmax (the running max and sum are identical in
-//     all waves) and accumulates its own 128 output channels, O^T += V^T[slice] . P^T
-//     (8 MFMAs).
-// The q RMSNorm sums the squares of the four slices through LDS in the same order; RoPE
-// pairs channel c with c ^ 256, so each lane also loads its channels' partners.
-struct WideTile {
+// accumulators, so here the head dim is split over SPLIT waves, each with its D / SPLIT channels
+// of a head's 32 queries; a block of NW waves holds NW / SPLIT heads of one KV head, so each K/V
+// tile is loaded once for all of them. Per key tile (32 keys, two LDS stages of 32 KB K + 32 KB
+// V):
+//   * each wave computes the partial scores of its channels, S_w^T = K[:, slice] . Q^T[slice],
+//     and stores them in LDS; after a barrier every wave adds its head's partials in slice
+//     order, so the waves of a head hold identical scores;
+//   * every wave runs the same online softmax (the running max and sum are identical in the
+//     waves of a head) and accumulates its own output channels, O^T += V^T[slice] . P^T.
+// The q RMSNorm sums the squares of the slices through LDS in the same order; RoPE pairs
+// channel c with c ^ 256, so each lane also loads its channels' partners.
+// Eight waves (four heads, two waves per SIMD) against four (two heads, one per SIMD): half the
+// tile loads per FLOP, and one wave's softmax runs beside the other's MFMAs: 16 q / 1 KV head,
+// 4,096 causal: 384 us against 631 us (716 against 435 TFLOP/s). It needs the whole 256-register
+// budget of two waves per SIMD, hence the load and LDS addresses made from one register each and
+// the K operands held two steps ahead only: every spill reload in the tile loop would wait for
+// the tile loads in flight.
+template <int NW> struct WideTile {
   static constexpr int D = 512;
-  static constexpr int WAVES = 4;
+  static constexpr int WAVES = NW;
   static constexpr int BM = 32;                          // queries per block
   static constexpr int BN = 32;                          // keys per tile
   static constexpr int NCH = D / 8;
@@ -647,15 +654,14 @@ struct WideTile {
   static constexpr int LOADS = TILEB / (WAVES * 1024);   // 8
   static constexpr int STAGES = 2;
   static constexpr int PART_BYTES = WAVES * 64 * 16 * 4; // the waves' partial scores
-  static constexpr int SS_BYTES = WAVES * 32 * 4;        // the q slices' sums of squares
-  static constexpr int LDS_BYTES = STAGES * 2 * TILEB + PART_BYTES + SS_BYTES;
+  static constexpr int LDS_BYTES = STAGES * 2 * TILEB + PART_BYTES;
 };
 
-template <typename T, int SPLIT, bool KSPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
+template <typename T, int NW, int SPLIT, bool KSPLIT>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4)))
 void prefill_wide_kernel(PrefillParams p) {
   using V8 = typename Mfma<T>::vec;
-  using TL = WideTile;
+  using TL = WideTile<NW>;
   constexpr int D = TL::D;
   constexpr int BN = TL::BN;
   // SPLIT waves share a head, each with D / SPLIT channels; the block takes WAVES / SPLIT heads
@@ -670,7 +676,7 @@ void prefill_wide_kernel(PrefillParams p) {
 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   float* part = reinterpret_cast<float*>(smem + TL::STAGES * 2 * TL::TILEB);   // [wave][lane][16]
-  float* sh_ss = part + TL::WAVES * 64 * 16;                                     // [wave][32]
+  float* sh_ss = part;  // the q slices' sums of squares [wave][32], before any partial score
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -709,19 +715,20 @@ void prefill_wide_kernel(PrefillParams p) {
 
   const char* kgb = reinterpret_cast<const char*>(static_cast<const T*>(p.k) + b * p.skb + kvh * p.skh);
   const char* vgb = reinterpret_cast<const char*>(static_cast<const T*>(p.v) + b * p.skb + kvh * p.skh);
+  // A wave's 1 KB load is one key row (64 lanes x 16 bytes), so the row is wave-uniform: its
+  // address stays in scalar registers and a lane's offset is its swizzled chunk.
+  static_assert(TL::NCH == kWave, "one key row per wave load");
   auto issue = [&](int kt, int stage) {
-    const int64_t key0 = (int64_t)kt * BN;
-    const char* kt_base = kgb + key0 * p.sks * 2;
-    const char* vt_base = vgb + key0 * p.sks * 2;
     const unsigned kdst = lds_offset(smem + (2 * stage) * TL::TILEB + wave * TL::LOADS * 1024);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // the offsets are made here, one xor each, and not kept in registers
 #pragma unroll
     for (int i = 0; i < TL::LOADS; ++i) {
-      const int slot = (wave * TL::LOADS + i) * 64 + lane;
-      const int row = slot / TL::NCH, pch = slot % TL::NCH;
-      const int64_t key = key0 + row < S ? key0 + row : S - 1;   // rows past the end are masked
-      const unsigned rb = (unsigned)((key - key0) * p.sks * 2);
-      lds_dma16(kt_base, rb + (pch ^ swz_k<D>(row)) * 16, kdst + i * 1024);
-      lds_dma16(vt_base, rb + (pch ^ swz_v<D>(row)) * 16, kdst + TL::TILEB + i * 1024);
+      const int row = wave * TL::LOADS + i;
+      const int64_t key = (int64_t)kt * BN + row;
+      const int64_t off = (key < S ? key : S - 1) * p.sks * 2;   // rows past the end are masked
+      lds_dma16(kgb + off, (unsigned)((ln ^ swz_k<D>(row)) << 4), kdst + i * 1024);
+      lds_dma16(vgb + off, (unsigned)((ln ^ swz_v<D>(row)) << 4), kdst + TL::TILEB + i * 1024);
     }
   };
   issue(kt_begin, 0);
@@ -732,15 +739,9 @@ void prefill_wide_kernel(PrefillParams p) {
   {
     const int c0 = CW * slice + 8 * hi;
     const int pc0 = (CW * slice + 8 * hi) ^ 256;   // partner channels
-    // raw slices stay packed (16 bf16/fp16 values per k-step in 8 registers); each k-step is
-    // unpacked, normalised, rotated and rounded in turn
-    uint4 rx[KSTEPS], rz[KSTEPS];
+    // the raw slice is read once for the sum of squares and again per k-step, which is unpacked,
+    // normalised, rotated and rounded in turn: held in between, it and the partners' slice spill
     const T* src = static_cast<const T*>(p.q) + b * p.sqb + h * p.sqh + (int64_t)(valid_q ? i_q : 0) * p.sqt;
-#pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) {
-      rx[s] = load16(src + c0 + 16 * s);
-      rz[s] = load16(src + pc0 + 16 * s);
-    }
     const bool norm = (p.flags & FORGE_NORM_QK) != 0;
     float rs = 1.0f;
     if (norm) {
@@ -748,7 +749,7 @@ void prefill_wide_kernel(PrefillParams p) {
 #pragma unroll
       for (int s = 0; s < KSTEPS; ++s) {
         float x[8];
-        unpack16<T>(rx[s], x);
+        unpack16<T>(load16(src + c0 + 16 * s), x);
 #pragma unroll
         for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
       }
@@ -767,8 +768,8 @@ void prefill_wide_kernel(PrefillParams p) {
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
       float x[8], z[8];
-      unpack16<T>(rx[s], x);
-      unpack16<T>(rz[s], z);
+      unpack16<T>(load16(src + c0 + 16 * s), x);
+      unpack16<T>(load16(src + pc0 + 16 * s), z);
       if (norm) {
         float wx[8], wz[8];
         if (p.qw) {
@@ -801,13 +802,16 @@ void prefill_wide_kernel(PrefillParams p) {
   const int S32 = (int)S;
   const int qpos32 = (int)(p.offset + i_q);
   const int wq_lo = off + qt * TL::BM, wq_hi = off + q_last_idx;
-  const int k_rd = n * TL::ROWB;
-  const int k_sw = swz_k<D>(n);
+  // LDS read offsets of a lane within a stage's K and V tiles (the layouts of prefill_kernel).
+  // The swizzles only touch the low four chunk bits, so k-step st's operand lies at
+  // k_rd ^ 32 (st % 8) plus 256 bytes per 8 steps, and channel block d's at v_rd ^ 64 (d % 4)
+  // plus 256 bytes per 4 blocks: one xor from one register each.
   const int g = lane >> 4, kq = (lane >> 2) & 3, qq = lane & 3;
   const int v_row = 4 * (g >> 1) + kq;
-  const int v_sw = swz_v<D>(v_row);
-  const int v_chlo = 2 * (g & 1) + (qq >> 1);
-  const int v_byte = 8 * (qq & 1);
+  const unsigned k_rd = n * TL::ROWB + CCH * 16 * slice + ((hi ^ swz_k<D>(n)) << 4);
+  const unsigned v_rd = v_row * TL::ROWB + CCH * 16 * slice +
+                        (((2 * (g & 1) + (qq >> 1)) ^ swz_v<D>(v_row)) << 4) + 8 * (qq & 1);
+  const unsigned lds0 = lds_offset(smem);
 
   floatx16 oacc[DB];
 #pragma unroll
@@ -822,17 +826,32 @@ void prefill_wide_kernel(PrefillParams p) {
     wait_vm<0>();
     __syncthreads();   // tile kt in LDS; every wave is done with tile kt - 1 and its partials
     if (kt + 1 <= kt_end) issue(kt + 1, stage ^ 1);
-    const char* kl = smem + (2 * stage) * TL::TILEB + k_rd;
-    const char* vl = smem + (2 * stage + 1) * TL::TILEB;
+    const unsigned kl = lds0 + (2 * stage) * TL::TILEB + k_rd;
+    const unsigned vl = lds0 + (2 * stage + 1) * TL::TILEB + v_rd;
 
     // partial scores of this wave's channels
     floatx16 sp;
 #pragma unroll
     for (int x = 0; x < 16; ++x) sp[x] = 0.0f;
+    {
+      // K operands two k-steps ahead of their MFMA, pinned as in prefill_kernel (left alone the
+      // compiler reads them all first, and with eight waves spills)
+      auto kread = [&](int st) {
+        return *(__attribute__((address_space(3))) const V8*)((kl ^ (32 * (st & 7))) + 256 * (st >> 3));
+      };
+      V8 a0 = kread(0), a1 = kread(1), a2 = a1;
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
 #pragma unroll
-    for (int st = 0; st < KSTEPS; ++st) {
-      const V8 a = *reinterpret_cast<const V8*>(kl + ((CCH * slice + ((2 * st + hi) ^ k_sw)) << 4));
-      sp = Mfma<T>::run(a, qreg[st], sp);
+      for (int st = 0; st < KSTEPS; ++st) {
+        if (st + 2 < KSTEPS) {
+          a2 = kread(st + 2);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        sp = Mfma<T>::run(a0, qreg[st], sp);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        a0 = a1;
+        a1 = a2;
+      }
     }
     {
       float4* dst = reinterpret_cast<float4*>(part + (wave * 64 + lane) * 16);
@@ -907,14 +926,12 @@ void prefill_wide_kernel(PrefillParams p) {
       V8 pb;
 #pragma unroll
       for (int e = 0; e < 8; ++e) pb[e] = from_f32<T>(sacc[8 * hf + e]);
-      const char* vrow0 = vl + (16 * hf + v_row) * TL::ROWB + v_byte;
 #pragma unroll
       for (int d = 0; d < DB; ++d) {
-        const int ch = (CCH * slice + ((4 * d + v_chlo) ^ v_sw)) << 4;
-        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) i16x4*)(vrow0 + ch));
+        const unsigned va = (vl ^ (64 * (d & 3))) + 256 * (d >> 2) + 16 * hf * TL::ROWB;
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)va);
         const i16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) i16x4*)(vrow0 + 8 * TL::ROWB + ch));
+            (__attribute__((address_space(3))) i16x4*)(va + 8 * TL::ROWB));
         typedef short i16x8 __attribute__((ext_vector_type(8)));
         const i16x8 av = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
         oacc[d] = Mfma<T>::run(__builtin_bit_cast(V8, av), pb, oacc[d]);
@@ -950,12 +967,12 @@ void prefill_wide_kernel(PrefillParams p) {
     }
 }
 
-template <typename T, int SPLIT, bool KSPLIT>
+template <typename T, int NW, int SPLIT, bool KSPLIT>
 static int launch_prefill_wide_s(PrefillParams p, hipStream_t s) {
-  using TL = WideTile;
+  using TL = WideTile<NW>;
   static bool attr_set = false;
   if (!attr_set) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_wide_kernel<T, SPLIT, KSPLIT>),
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_wide_kernel<T, NW, SPLIT, KSPLIT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES) != hipSuccess)
       return set_error("forge_attn_prefill: cannot reserve the LDS the kernel needs");
     attr_set = true;
@@ -964,19 +981,25 @@ static int launch_prefill_wide_s(PrefillParams p, hipStream_t s) {
   p.nqt = (p.T + TL::BM - 1) / TL::BM;
   const int64_t blocks = (int64_t)p.nqt * (p.H / HPB) * p.B * p.nsplit;
   if (blocks > 0x7fffffff) return set_error("grid too large");
-  hipLaunchKernelGGL((prefill_wide_kernel<T, SPLIT, KSPLIT>), dim3((unsigned)blocks), dim3(TL::WAVES * 64),
+  hipLaunchKernelGGL((prefill_wide_kernel<T, NW, SPLIT, KSPLIT>), dim3((unsigned)blocks), dim3(TL::WAVES * 64),
                      TL::LDS_BYTES, s, p);
   return check_launch();
 }
 
-// Two heads of one KV head per block (head dim in halves) where the group is even: each K/V
-// tile is loaded once for both; else one head per block in quarter slices.
+template <typename T, int NW, int SPLIT>
+static int launch_prefill_wide_w(const PrefillParams& p, hipStream_t s) {
+  if (p.nsplit < 2) return launch_prefill_wide_s<T, NW, SPLIT, false>(p, s);
+  const int st = launch_prefill_wide_s<T, NW, SPLIT, true>(p, s);
+  return st ? st : launch_prefill_combine<T, 512>(p, WideTile<NW>::BM, WideTile<NW>::BN, s);
+}
+
 template <typename T>
 static int launch_prefill_wide(const PrefillParams& p, hipStream_t s) {
-  if (p.nsplit < 2)
-    return p.G % 2 == 0 ? launch_prefill_wide_s<T, 2, false>(p, s) : launch_prefill_wide_s<T, 4, false>(p, s);
-  const int st = p.G % 2 == 0 ? launch_prefill_wide_s<T, 2, true>(p, s) : launch_prefill_wide_s<T, 4, true>(p, s);
-  return st ? st : launch_prefill_combine<T, 512>(p, WideTile::BM, WideTile::BN, s);
+  switch (p.heads_per_block) {
+    case 4: return launch_prefill_wide_w<T, 8, 2>(p, s);
+    case 2: return launch_prefill_wide_w<T, 4, 2>(p, s);
+    default: return launch_prefill_wide_w<T, 4, 4>(p, s);
+  }
 }
 
 // How a launch splits its query tiles' keys: parts of at most `tiles` key tiles, nsplit of them
@@ -985,64 +1008,73 @@ static int launch_prefill_wide(const PrefillParams& p, hipStream_t s) {
 // chunk at position 15,360 (16 q / 8 KV heads, head dim 128) is 64 blocks of 248 tiles.
 struct PrefillPlan {
   int nsplit, tiles;
+  int heads_per_block;
 };
 constexpr int kMaxParts = 32;
 
 // Picks the split with the least modelled time. Measured on calls of 1 to 32 parts (graph
-// replays, one box; the model is within 15% of each): a tile takes kTileAlone us in a block
-// that has its CU to itself and kTileShared us of a CU that holds two (head dims 64 and 128), a
-// block's q prologue and epilogue cost about 2.5 tiles, its partial crosses memory twice at
-// about 4 TB/s, and the combine launch takes 3 us. So parts pay while CUs are idle and stop
-// paying once the partials' traffic grows: 16 q / 8 KV heads, head dim 128, 1 / 2 / 4 / 8 / 16
-// parts: T 512 at 15,360: 279 / 149 / 87 / 83 / 96 us; T 128 there: 267 / 143 / 79 / 49 / 39;
-// T 64 at 1,000: 25 / 20 / 16 / 15 / 17; T 1024 at 15,360: 288 / 170 / 143 / 162 / 191; a whole
-// prompt of 2,048: 44 / 49 / 53 / 71 / 115 (not split). Head dim 256 (8 q / 4 KV), T 512 at
-// 8,000: 352 / 186 / 105 / 69 / 86.
-static PrefillPlan prefill_plan(int B, int T, int H, int K, int D, int64_t offset, int window) {
+// replays, one box; the model is within 15% of each): a tile takes `alone` us in a block that has
+// its CU to itself and `shared` us of a CU that holds two (head dims 64 and 128), a block's q
+// prologue and epilogue cost about 2.5 tiles, its partial crosses memory twice at about 4 TB/s,
+// and the combine launch takes 3 us. So parts pay while CUs are idle and stop paying once the
+// partials' traffic grows: 16 q / 8 KV heads, head dim 128, 1 / 2 / 4 / 8 / 16 parts: T 512 at
+// 15,360: 279 / 149 / 87 / 83 / 96 us; T 128 there: 267 / 143 / 79 / 49 / 39; T 64 at 1,000:
+// 25 / 20 / 16 / 15 / 17; T 1024 at 15,360: 288 / 170 / 143 / 162 / 191; a whole prompt of
+// 2,048: 44 / 49 / 53 / 71 / 115 (not split). Head dim 256 (8 q / 4 KV), T 512 at 8,000: 352 /
+// 186 / 105 / 69 / 86.
+// At head dim 512 the same model picks the heads that share a block and its K/V tiles: four
+// take 2.55 us a tile where two take 2.1 us, so four win once the blocks fill the CUs (16 q / 1 KV
+// head, a prompt of 4,096: 384 us against 631; T 512 at 8,000, split: 211 against 301), two on
+// short calls (a prompt of 1,024: 80 us against 100).
+static PrefillPlan prefill_plan(int B, int T, int H, int K, int D, int64_t offset, int window, int max_parts) {
   const bool wide = D == 512;
-  const int BM = wide ? WideTile::BM : Tile<64>::BM;
-  const int BN = wide ? WideTile::BN : D == 256 ? Tile<256>::BN : Tile<128>::BN;
-  const int hpb = wide && (H / K) % 2 == 0 ? 2 : 1;  // heads per block
-  const double alone = wide ? 2.1 : D == 256 ? 1.3 : 1.2;
-  const double shared = wide ? 2.1 : D == 256 ? 1.3 : D == 128 ? 0.95 : 0.7;
+  const int BM = wide ? WideTile<4>::BM : Tile<64>::BM;
+  const int BN = wide ? WideTile<4>::BN : D == 256 ? Tile<256>::BN : Tile<128>::BN;
+  const int G = H / K;
+  const int most_heads = !wide ? 1 : G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
   const int64_t cus = device_cus();
-  const int64_t heads = (int64_t)(H / hpb) * B;
   const int nqt = (T + BM - 1) / BM;
-  if (nqt * heads >= 4 * cus) return PrefillPlan{1, 0};  // several rounds of blocks already
+  if ((int64_t)nqt * (H / most_heads) * B >= 4 * cus)  // several rounds of blocks already
+    return PrefillPlan{1, 0, most_heads};
   int longest = 0;
   for (int qt = 0; qt < nqt; ++qt) {
     int begin, end;
     tile_span(offset, T, window, 0, qt, BM, BN, begin, end);
     longest = end - begin + 1 > longest ? end - begin + 1 : longest;
   }
-  PrefillPlan best{1, longest};
+  PrefillPlan best{1, longest, most_heads};
   double best_us = 0.0;
-  for (int c = 1, last = 0; c <= kMaxParts; ++c) {
+  for (int c = 1, last = 0; c <= max_parts; ++c) {
     const int tiles = (longest + c - 1) / c;
     if (tiles == last) continue;
     last = tiles;
-    int64_t blocks = 0, split = 0, work = 0;  // blocks, those that write a partial, key tiles
+    int64_t blocks1 = 0, split1 = 0, work1 = 0;  // per head group: blocks, partials, key tiles
     for (int qt = 0; qt < nqt; ++qt) {
       int begin, end;
       tile_span(offset, T, window, 0, qt, BM, BN, begin, end);
       const int n = end - begin + 1, parts = (n + tiles - 1) / tiles;
-      blocks += parts;
-      if (parts > 1) split += parts;
-      work += n;
+      blocks1 += parts;
+      if (parts > 1) split1 += parts;
+      work1 += n;
     }
-    blocks *= heads;
-    const double per_block = (double)work * heads / blocks + 2.5;
-    const int64_t rounds = (blocks + cus - 1) / cus;
-    double us = (tiles + 2.5) * alone;                       // the longest block
-    if (rounds > 1 && rounds * per_block * shared > us) us = rounds * per_block * shared;
-    if (split) us += 3.0 + 2.0 * split * heads * hpb * BM * D * sizeof(float) / 4e6;
-    // (leaving the unsplit launch has to be worth more than the model's error)
-    if (c == 1 || us < (best.nsplit == 1 ? 0.85 : 0.95) * best_us) {
-      best = PrefillPlan{c, tiles};
-      best_us = us;
+    for (int hpb = most_heads; hpb >= (most_heads == 4 ? 2 : most_heads); hpb /= 2) {
+      const double alone = hpb == 4 ? 2.55 : wide ? 2.1 : D == 256 ? 1.3 : 1.2;
+      const double shared = wide || D == 256 ? alone : D == 128 ? 0.95 : 0.7;
+      const int64_t blocks = blocks1 * (H / hpb) * B;
+      const double per_block = (double)work1 / blocks1 + 2.5;
+      const int64_t rounds = (blocks + cus - 1) / cus;
+      double us = (tiles + 2.5) * alone;  // the longest block
+      if (rounds > 1 && rounds * per_block * shared > us) us = rounds * per_block * shared;
+      if (split1) us += 3.0 + 2.0 * split1 * H * B * BM * D * sizeof(float) / 4e6;
+      // (splitting has to be worth more than the model's error)
+      const bool first = c == 1 && hpb == most_heads;
+      if (first || us < (c > 1 && best.nsplit == 1 ? 0.85 : 0.95) * best_us) {
+        best = PrefillPlan{c, tiles, hpb};
+        best_us = us;
+      }
     }
   }
-  best.nsplit = best.nsplit > 1 ? (longest + best.tiles - 1) / best.tiles : 1;
+  if (best.nsplit > 1) best.nsplit = (longest + best.tiles - 1) / best.tiles;
   return best;
 }
 
@@ -1123,17 +1155,15 @@ static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void
   p.soh = soh;
   p.doc_lo = doc_lo;
   p.sdb = sdb;
-  p.nsplit = 1;
-  if (workspace && !doc_lo) {
-    const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window);
-    if (plan.nsplit > 1) {
-      if (workspace_bytes < prefill_workspace(plan, B, T, H, D)) return set_error("workspace too small");
-      p.nsplit = plan.nsplit;
-      p.split_tiles = plan.tiles;
-      const int64_t slots = (int64_t)plan.nsplit * B * H * T;
-      p.ws_ml = static_cast<float2*>(workspace);
-      p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + ((size_t)slots * sizeof(float2) + 255) / 256 * 256);
-    }
+  const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window, workspace && !doc_lo ? kMaxParts : 1);
+  p.nsplit = plan.nsplit;
+  p.split_tiles = plan.tiles;
+  p.heads_per_block = plan.heads_per_block;
+  if (plan.nsplit > 1) {
+    if (workspace_bytes < prefill_workspace(plan, B, T, H, D)) return set_error("workspace too small");
+    const size_t slots = (size_t)plan.nsplit * B * H * T;
+    p.ws_ml = static_cast<float2*>(workspace);
+    p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + (slots * sizeof(float2) + 255) / 256 * 256);
   }
   hipStream_t s = (hipStream_t)stream;
   return dtype == FORGE_BF16 ? launch_prefill<bf16>(p, D, s) : launch_prefill<f16>(p, D, s);
@@ -1173,7 +1203,7 @@ extern "C" size_t forge_attn_prefill_workspace_bytes(int dtype, int B, int T, in
   if ((dtype != FORGE_BF16 && dtype != FORGE_F16) || (D != 64 && D != 128 && D != 256 && D != 512) || B <= 0 ||
       T <= 0 || H <= 0 || K <= 0 || H % K || offset < 0 || window < 0 || offset + (int64_t)T + 256 >= (1LL << 31))
     return 0;
-  const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window);
+  const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window, kMaxParts);
   return plan.nsplit > 1 ? prefill_workspace(plan, B, T, H, D) : 0;
 }
 

@@ -114,3 +114,28 @@ def test_split_prefill_under_graph_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("dtype,window,docs", [(torch.bfloat16, 0, False), (torch.float16, 300, False),
+                                               (torch.bfloat16, 0, True)])
+def test_wide_prefill_with_four_heads_per_block(dtype, window, docs):
+    """Head dim 512 with enough query tiles for four heads per block (eight waves): 701 queries (a
+    last tile of 29), raw q with norm and RoPE, two KV heads of eight query heads each."""
+    from sleuth_amd import ops
+
+    B, T, H, K, D = 3, 701, 16, 2, 512
+    g = gen(980)
+    q = randn(g, B, T, H, D, dtype=dtype).transpose(1, 2)
+    w = (1 + 0.1 * randn(g, D)).to(dtype)
+    k, v = randn(g, B, K, T, D, dtype=dtype), randn(g, B, K, T, D, dtype=dtype)
+    cos, sin = tables(D, T, 1e4)
+    starts = torch.tensor([0] * 100 + [100] * 301 + [401] * 300, dtype=torch.int32)[None].expand(B, T).contiguous()
+    qn = oracle.head_norm_rope(q, w, 1e-6, cos, sin)
+    same = (starts[:, :, None] == starts[:, None, :])[:, None] if docs else None
+    ref = oracle.sdpa(qn.float(), k.float(), v.float(), 0, window, scale_of(D), same_doc=same)
+    got = ops.attn_prefill(q.to(DEV), k.to(DEV), v.to(DEV), scale=scale_of(D), window=window, q_weight=w.to(DEV),
+                           eps=1e-6, norm_q=True, cos=cos.to(DEV), sin=sin.to(DEV),
+                           doc_start=starts.to(DEV) if docs else None)
+    assert max_abs(got.cpu().transpose(1, 2), ref) <= tol(dtype)
