@@ -11,7 +11,9 @@
 //     below free of bank conflicts. LDS stages (two for every head dim today): the loads
 //     of tile j+1 are issued before tile j is computed, one barrier per tile separates
 //     the stages, and two blocks share a CU so that its SIMDs interleave two independent
-//     waves.
+//     waves. At head dim 256 (128 accumulator and 64 Q^T registers of the 256 a wave may use)
+//     that needs the load and LDS addresses to come from one register each: two waves per SIMD
+//     take 284 us where one took 378 us (4 x 4096 causal, 8 q / 4 KV heads; 386 -> 514 TFLOP/s).
 //   * Scores are computed transposed, S^T = K . Q^T: K is the MFMA A operand (128-bit
 //     LDS reads), Q^T the B operand held in registers for the whole block. In the 32x32
 //     accumulator layout each lane then owns ONE query (column l % 32) and 16 keys of a
@@ -223,7 +225,7 @@ __device__ __forceinline__ void load_q(const PrefillParams& p, int b, int h, int
 
 // SPLIT: the key-split launch (PrefillParams::nsplit > 1); otherwise one block per query tile.
 template <typename T, int D, bool SPLIT>
-__global__ __launch_bounds__(Tile<D>::WAVES * 64) __attribute__((amdgpu_waves_per_eu(D >= 256 ? 1 : 2)))
+__global__ __launch_bounds__(Tile<D>::WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_kernel(PrefillParams p) {
   using V8 = typename Mfma<T>::vec;
   using TL = Tile<D>;
@@ -295,44 +297,46 @@ void prefill_kernel(PrefillParams p) {
   const T* kg = static_cast<const T*>(p.k) + b * p.skb + kvh * p.skh;
   const T* vg = static_cast<const T*>(p.v) + b * p.skb + kvh * p.skh;
 
-  // Per-lane source byte offsets of the direct loads within a tile: load i of this wave
-  // fills LDS slots (wave*LOADS + i)*64 + lane, i.e. key row slot / NCH and swizzled
-  // chunk slot % NCH. The tile base is wave-uniform (scalar registers).
-  int ld_koff[TL::LOADS], ld_voff[TL::LOADS];
-#pragma unroll
-  for (int i = 0; i < TL::LOADS; ++i) {
-    const int slot = (wave * TL::LOADS + i) * 64 + lane;
-    const int row = slot / TL::NCH, pch = slot % TL::NCH;
-    ld_koff[i] = (int)(row * p.sks * 2) + (pch ^ swz_k<D>(row)) * 16;
-    ld_voff[i] = (int)(row * p.sks * 2) + (pch ^ swz_v<D>(row)) * 16;
-  }
   const char* kgb = reinterpret_cast<const char*>(kg);
   const char* vgb = reinterpret_cast<const char*>(vg);
+  // Load i of this wave fills LDS slots (wave*LOADS + i)*64 + lane with RL = 64 / NCH key rows, r0 +
+  // lane / NCH, in swizzled chunk order. r0 is wave-uniform (its address stays in scalar
+  // registers) and the swizzles split over r0 and the lane's part, so a lane's offsets take one
+  // xor each from registers shared by all the loads.
+  constexpr int RL = kWave / TL::NCH;
+  const int ld_row = lane / TL::NCH;
+  const int ld_k = ((lane % TL::NCH) ^ swz_k<D>(ld_row)) << 4, ld_v = ((lane % TL::NCH) ^ swz_v<D>(ld_row)) << 4;
+  const int ld_off = (int)(ld_row * p.sks * 2);
   // The loads are issued from inline asm (lds_dma16), so the compiler does not hold the
   // LDS reads of the current stage back until the next stage's loads have landed; the
   // loop waits for them itself (wait_vm before the barrier).
   auto issue = [&](int kt, int stage) {
     const int64_t key0 = (int64_t)kt * BN;
-    const char* kt_base = kgb + key0 * p.sks * 2;
-    const char* vt_base = vgb + key0 * p.sks * 2;
     const unsigned kdst = lds_offset(smem + (2 * stage) * TL::TILEB + wave * TL::LOADS * 1024);
     const unsigned vdst = kdst + TL::TILEB;
+    int lk = ld_k, lv = ld_v, lo = ld_off;
+    if constexpr (D >= 256) asm volatile("" : "+v"(lk), "+v"(lv));  // (registers short: not kept over the loop)
     if (key0 + BN <= S) {
+      const char* kt_base = kgb + key0 * p.sks * 2;
+      const char* vt_base = vgb + key0 * p.sks * 2;
 #pragma unroll
       for (int i = 0; i < TL::LOADS; ++i) {
-        lds_dma16(kt_base, (unsigned)ld_koff[i], kdst + i * 1024);
-        lds_dma16(vt_base, (unsigned)ld_voff[i], vdst + i * 1024);
+        const int r0 = RL * (wave * TL::LOADS + i);
+        const int64_t off = r0 * p.sks * 2;
+        lds_dma16(kt_base + off, (unsigned)(lo + (lk ^ (swz_k<D>(r0) << 4))), kdst + i * 1024);
+        lds_dma16(vt_base + off, (unsigned)(lo + (lv ^ (swz_v<D>(r0) << 4))), vdst + i * 1024);
       }
     } else {
-      // last, partial tile: rows past the end are masked; they read row S - 1 instead
+      // last, partial tile: rows past the end are masked; they read row S - 1 instead (the
+      // wave's row is clamped first, so a lane's offset, which is unsigned, stays at least 0)
 #pragma unroll
       for (int i = 0; i < TL::LOADS; ++i) {
-        const int slot = (wave * TL::LOADS + i) * 64 + lane;
-        const int row = slot / TL::NCH, pch = slot % TL::NCH;
-        const int64_t key = key0 + row < S ? key0 + row : S - 1;
-        const unsigned rb = (unsigned)((key - key0) * p.sks * 2);
-        lds_dma16(kt_base, rb + (pch ^ swz_k<D>(row)) * 16, kdst + i * 1024);
-        lds_dma16(vt_base, rb + (pch ^ swz_v<D>(row)) * 16, vdst + i * 1024);
+        const int r0 = RL * (wave * TL::LOADS + i);
+        const int64_t key = key0 + r0 < S ? key0 + r0 : S - 1;
+        const int64_t off = key * p.sks * 2;
+        const int o = ld_row <= S - 1 - key ? lo : (int)((S - 1 - key) * p.sks * 2);
+        lds_dma16(kgb + off, (unsigned)(o + (lk ^ (swz_k<D>(r0) << 4))), kdst + i * 1024);
+        lds_dma16(vgb + off, (unsigned)(o + (lv ^ (swz_v<D>(r0) << 4))), vdst + i * 1024);
       }
     }
   };
@@ -363,17 +367,17 @@ void prefill_kernel(PrefillParams p) {
     d_wlast = __builtin_amdgcn_readlane(d_lane, w_last - w_first > 0 ? w_last - w_first : 0);
   }
 
-  // LDS read offsets (bytes within a stage buffer).
-  // K operand: row 32kb + n, chunk 2s + hi, swizzled by row & 15 == n & 15.
-  const int k_rd = n * TL::ROWB;
-  const int k_sw = swz_k<D>(n);
-  // V^T operand (tr reads): source lane role g = lane/16, kq = (lane/4)%4, qq = lane%4
-  // addresses key row 16*half + 8i' + 4(g/2) + kq, channel 32db + 16(g%2) + 4qq.
+  // LDS read offsets of a lane within a stage's K and V tiles. K operand: row 32kb + n, chunk
+  // 2st + hi, swizzled by the row; V^T operand (tr reads): source lane role g = lane/16,
+  // kq = (lane/4)%4, qq = lane%4 addresses key row 16*half + 8i' + 4(g/2) + kq, channel
+  // 32db + 16(g%2) + 4qq (rows that differ by multiples of 8 share a swizzle). The swizzles only
+  // touch the low four chunk bits, so k-step st lies at k_rd ^ 32 (st % 8) plus 256 bytes per 8
+  // steps and channel block d at v_rd ^ 64 (d % 4) plus 256 bytes per 4: one xor from one register.
   const int g = lane >> 4, kq = (lane >> 2) & 3, qq = lane & 3;
   const int v_row = 4 * (g >> 1) + kq;
-  const int v_sw = swz_v<D>(v_row);  // rows differ from v_row by multiples of 8: same swizzle
-  const int v_chlo = 2 * (g & 1) + (qq >> 1);  // chunk within the 32-channel block (0..3)
-  const int v_byte = 8 * (qq & 1);
+  const unsigned k_rd = n * TL::ROWB + ((hi ^ swz_k<D>(n)) << 4);
+  const unsigned v_rd = v_row * TL::ROWB + (((2 * (g & 1) + (qq >> 1)) ^ swz_v<D>(v_row)) << 4) + 8 * (qq & 1);
+  const unsigned lds0 = lds_offset(smem);
 
   floatx16 oacc[DB];
 #pragma unroll
@@ -401,8 +405,8 @@ void prefill_kernel(PrefillParams p) {
                       (p.window <= 0 || wq_hi - key0 < p.window) && w_last - w_first == 31 &&
                       key0 >= d_wlast;
 
-    const char* kl = smem + (2 * stage) * TL::TILEB + k_rd;
-    const char* vl = smem + (2 * stage + 1) * TL::TILEB;
+    const unsigned kl = lds0 + (2 * stage) * TL::TILEB + k_rd;
+    const unsigned vl = lds0 + (2 * stage + 1) * TL::TILEB + v_rd;
 
     // ---- S^T = K . Q^T: KB independent accumulation chains. The K operands of step
     // st + 2 are read before the MFMAs of step st are issued (three register sets), so
@@ -415,7 +419,8 @@ void prefill_kernel(PrefillParams p) {
       for (int x = 0; x < 16; ++x) sacc[kb][x] = 0.0f;
     {
       auto kread = [&](int kb, int st) {
-        return *reinterpret_cast<const V8*>(kl + kb * 32 * TL::ROWB + (((2 * st + hi) ^ k_sw) << 4));
+        return *(__attribute__((address_space(3))) const V8*)((kl ^ (32 * (st & 7))) + 256 * (st >> 3) +
+                                                              kb * 32 * TL::ROWB);
       };
       V8 a0[KB], a1[KB], a2[KB];
 #pragma unroll
@@ -499,14 +504,12 @@ void prefill_kernel(PrefillParams p) {
       V8 pb;
 #pragma unroll
       for (int e = 0; e < 8; ++e) pb[e] = from_f32<T>(sacc[kb][8 * half + e]);
-      const char* vrow0 = vl + (16 * hf + v_row) * TL::ROWB + v_byte;
 #pragma unroll
       for (int d = 0; d < DB; ++d) {
-        const int ch = ((4 * d + v_chlo) ^ v_sw) << 4;
-        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) i16x4*)(vrow0 + ch));
+        const unsigned va = (vl ^ (64 * (d & 3))) + 256 * (d >> 2) + 16 * hf * TL::ROWB;
+        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4*)va);
         const i16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) i16x4*)(vrow0 + 8 * TL::ROWB + ch));
+            (__attribute__((address_space(3))) i16x4*)(va + 8 * TL::ROWB));
         typedef short i16x8 __attribute__((ext_vector_type(8)));
         const i16x8 av = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
         oacc[d] = Mfma<T>::run(__builtin_bit_cast(V8, av), pb, oacc[d]);
@@ -1014,7 +1017,7 @@ constexpr int kMaxParts = 32;
 
 // Picks the split with the least modelled time. Measured on calls of 1 to 32 parts (graph
 // replays, one box; the model is within 15% of each): a tile takes `alone` us in a block that has
-// its CU to itself and `shared` us of a CU that holds two (head dims 64 and 128), a block's q
+// its CU to itself and `shared` us of a CU that holds several (head dims 64 to 256), a block's q
 // prologue and epilogue cost about 2.5 tiles, its partial crosses memory twice at about 4 TB/s,
 // and the combine launch takes 3 us. So parts pay while CUs are idle and stop paying once the
 // partials' traffic grows: 16 q / 8 KV heads, head dim 128, 1 / 2 / 4 / 8 / 16 parts: T 512 at
@@ -1058,8 +1061,8 @@ static PrefillPlan prefill_plan(int B, int T, int H, int K, int D, int64_t offse
       work1 += n;
     }
     for (int hpb = most_heads; hpb >= (most_heads == 4 ? 2 : most_heads); hpb /= 2) {
-      const double alone = hpb == 4 ? 2.55 : wide ? 2.1 : D == 256 ? 1.3 : 1.2;
-      const double shared = wide || D == 256 ? alone : D == 128 ? 0.95 : 0.7;
+      const double alone = hpb == 4 ? 2.55 : wide ? 2.1 : D == 256 ? 1.25 : 1.2;
+      const double shared = wide ? alone : D == 256 ? 1.05 : D == 128 ? 0.95 : 0.65;
       const int64_t blocks = blocks1 * (H / hpb) * B;
       const double per_block = (double)work1 / blocks1 + 2.5;
       const int64_t rounds = (blocks + cus - 1) / cus;
@@ -1068,7 +1071,7 @@ static PrefillPlan prefill_plan(int B, int T, int H, int K, int D, int64_t offse
       if (split1) us += 3.0 + 2.0 * split1 * H * B * BM * D * sizeof(float) / 4e6;
       // (splitting has to be worth more than the model's error)
       const bool first = c == 1 && hpb == most_heads;
-      if (first || us < (c > 1 && best.nsplit == 1 ? 0.85 : 0.95) * best_us) {
+      if (first || us < (c > 1 && best.nsplit == 1 ? 0.8 : 0.95) * best_us) {
         best = PrefillPlan{c, tiles, hpb};
         best_us = us;
       }
