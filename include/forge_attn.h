@@ -239,6 +239,21 @@ int forge_attn_prefill_ws(int dtype, int B, int T, int H, int K, int D, const vo
                           int64_t sot, int64_t soh, void* workspace, size_t workspace_bytes,
                           void* stream);
 
+/*
+ * forge_attn_prefill in fp32 (fp32 matrix products and sums) for head dims 32, 64 and 128: the
+ * queries of a whole prompt or chunk, T > 16 in the module (SDPA is_causal and the chunked mask,
+ * attention.py:187-193). forge_attn_decode covers the other fp32 shapes. Arguments as
+ * forge_attn_prefill, the workspace as forge_attn_prefill_ws.
+ */
+size_t forge_attn_prefill_f32_workspace_bytes(int B, int T, int H, int K, int D, int64_t offset,
+                                              int window);
+int forge_attn_prefill_f32(int B, int T, int H, int K, int D, const void* q, int64_t sqb,
+                           int64_t sqh, int64_t sqt, const float* q_weight, float eps, int flags,
+                           const float* cos, const float* sin, int64_t s_cos_t, const void* k,
+                           const void* v, int64_t skb, int64_t skh, int64_t sks, int64_t offset,
+                           int window, float scale, void* out, int64_t sob, int64_t sot,
+                           int64_t soh, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

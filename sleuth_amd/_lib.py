@@ -112,6 +112,17 @@ SIGNATURES: dict[str, tuple] = {
         _p, _i64, _i64, _i64,                # out + strides (b, t, h)
         _p, C.c_size_t,                      # workspace, bytes
         _p]),
+    "forge_attn_prefill_f32_workspace_bytes": (C.c_size_t, [_i, _i, _i, _i, _i, _i64, _i]),
+    "forge_attn_prefill_f32": (_i, [
+        _i, _i, _i, _i, _i,                  # B, T, H, K, D
+        _p, _i64, _i64, _i64,                # q + strides
+        _p, _f, _i,                          # q_weight, eps, flags
+        _p, _p, _i64,                        # cos, sin, s_cos_t
+        _p, _p, _i64, _i64, _i64,            # k, v, skb, skh, sks
+        _i64, _i, _f,                        # offset, window, scale
+        _p, _i64, _i64, _i64,                # out + strides (b, t, h)
+        _p, C.c_size_t,                      # workspace, bytes
+        _p]),
 }
 
 _lock = threading.Lock()

@@ -14,8 +14,10 @@ of head_norm_rope + cache.update + SDPA):
       code does, and the kernels take q and k as they are), then attention:
       T > 16, bf16/fp16, head dim 64-512:     forge_kv_append, then forge_attn_prefill
                         (MFMA flash) with the q norm + RoPE in its q load;
+      T > 16, fp32, head dim 32-128:          forge_kv_append, then forge_attn_prefill_f32
+                        (the same on fp32 MFMA);
       otherwise         forge_attn_decode_append: the cache write and the split-K
-                        attention (decode, verify, static steps, fp32, other head sizes)
+                        attention (decode, verify, static steps, other head sizes)
                         in one launch, the q norm + RoPE fused into the q load.
       A boolean document mask (transformer.py:271-275) over a whole window (no cache,
       T > 16, the prefill dtypes and head dims) whose documents are contiguous runs goes
@@ -354,6 +356,12 @@ class Attention(nn.Module):
             self.last_path = "hip-prefill" if docs is None else "hip-prefill-docs"
             return ops.attn_prefill(q, kc, vc, scale=self.scale, offset=offset, window=self.window,
                                     doc_start=docs, check_doc_start=False, **q_args)
+        if T > DECODE_MAX_T and offset is not None and docs is None and \
+                (q_args["cos"] is None or q_args["cos"].dim() == 2) and \
+                ops.prefill_f32_supported(q, q_args["cos"], q_args["sin"]):
+            ops.kv_append(k, v, kc, vc, norm_v=norm_v, **pos_kw, **k_args)
+            self.last_path = "hip-decode"   # (what fp32 prompts have always reported)
+            return ops.attn_prefill_f32(q, kc, vc, scale=self.scale, offset=offset, window=self.window, **q_args)
         if docs is not None:
             raise RuntimeError("a document mask needs the prefill path (no cache, T > 16)")
         # the cache write and the attention in one call (one launch where the shape allows);

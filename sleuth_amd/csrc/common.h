@@ -153,6 +153,15 @@ __device__ __forceinline__ float max_xor32(float x) {
   return fmaxf(__uint_as_float(c0), __uint_as_float(c1));
 }
 
+// Buffer resource of one (batch row, KV head) slab of the cache (gfx9 raw buffer: stride
+// 0, range `bytes`). A load at a byte offset >= the range returns zeros without touching
+// memory, which is how the split-K loop skips keys outside a unit's range while still
+// issuing every load (kSkipOffset), and the fp32 prefill the keys past its last one.
+constexpr unsigned kBufferConfig = 0x00020000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t slab_rsrc(const void* base, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, (int)kBufferConfig);
+}
+
 // Base position of batch row b (see include/forge_attn.h).
 __device__ __forceinline__ int64_t row_base(const int32_t* row_pos, const int64_t* pos_dev,
                                             int64_t pos0, int b) {

@@ -338,12 +338,6 @@ __device__ __forceinline__ uint4 new_row_slice(uint4 raw, bool norm, const float
   return pack16<T>(x);
 }
 
-// Buffer resource of one (batch row, KV head) slab of the cache (gfx9 raw buffer: stride
-// 0, range `bytes`). A load at a byte offset >= the range returns zeros without touching
-// memory, which is how the split-K loop skips keys outside a unit's range while still
-// issuing every load (kSkipOffset).
-constexpr unsigned kBufferConfig = 0x00020000u;
-
 // s_waitcnt immediate (gfx9 layout) that waits until at most the K and V loads of `ITERS`
 // prefetched iterations (2 * NK each) are in flight; exp and lgkm counts left at maximum.
 template <int ITERS, int NK> constexpr int kWaitPrefetch() {
@@ -353,10 +347,6 @@ template <int ITERS, int NK> constexpr int kWaitPrefetch() {
 }
 constexpr unsigned kSkipOffset = 0x80000000u;  // beyond every slab (host check: < 2^31 bytes)
 constexpr int kNonTemporal = 2;                // cache policy of the streaming loads (nt)
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t slab_rsrc(const void* base, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, (int)kBufferConfig);
-}
 
 __device__ __forceinline__ uint4 load_slab(__amdgpu_buffer_rsrc_t rs, unsigned off) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));

@@ -41,6 +41,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 template <typename T> struct Mfma;
 template <> struct Mfma<bf16> {
@@ -586,9 +587,13 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p, i
     }
   }
   const float inv_l = 1.0f / L;
-  T v[4] = {from_f32<T>(O.x * inv_l), from_f32<T>(O.y * inv_l), from_f32<T>(O.z * inv_l), from_f32<T>(O.w * inv_l)};
   T* dst = static_cast<T*>(p.out) + b * p.sob + (int64_t)i_q * p.sot + h * p.soh + x;
-  *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<uint2*>(v);
+  if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<float4*>(dst) = make_float4(O.x / L, O.y / L, O.z / L, O.w / L);
+  } else {
+    T v[4] = {from_f32<T>(O.x * inv_l), from_f32<T>(O.y * inv_l), from_f32<T>(O.z * inv_l), from_f32<T>(O.w * inv_l)};
+    *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<uint2*>(v);
+  }
 }
 
 template <typename T, int D>
@@ -1005,6 +1010,327 @@ static int launch_prefill_wide(const PrefillParams& p, hipStream_t s) {
   }
 }
 
+// ---------------------------------------------------------------- fp32
+// fp32 prefill on v_mfma_f32_32x32x2_f32 (fp32 products and sums, as the split-K kernel's FMAs).
+// That instruction takes 64 clocks for 4,096 FLOP, so a wave needs little bandwidth and the
+// operands go from L2 straight into registers, with no LDS and no barrier in the loop: a block is
+// 32 queries of one (b, head), and its four waves take the 32-key tiles in turn (wave w tiles w,
+// w + 4, ...), each with its own running (m, l, o), merged through LDS at the end in a fixed
+// order. Splitting a query tile's keys over the waves keeps the chain of dependent tiles short
+// (1,025 causal queries: 9 tiles instead of 33), and small blocks fill the CUs on short calls.
+//   * S^T = K . Q^T: lane (n, hi) holds channels 8j + 4hi + e of key n (16-byte loads) and of query
+//     n; MFMA step (j, e) contracts channels 8j + e and 8j + 4 + e.
+//   * O^T = V^T . P^T straight from the score registers: step x pairs keys 8(x/4) + x%4 and + 4. Row
+//     m of output block d stands for channel DB m + d (DB = D / 32 blocks), so one load of DB
+//     consecutive channels feeds all the blocks.
+// V is requested before the tile's score MFMAs, the next tile's K after them.
+// Sums run in short chains added as trees (16 channels of a score, 16 keys of an output, per
+// chain): the 2-norm error against 64 bits stays that of the split-K path (1.4e-7 for 1,025 causal
+// queries at head dim 32, either way), where one chain each gave 2.2e-7 to 5e-7.
+// Against the split-K path, whose blocks of 8 rows each take every key through the VALU: 2 x
+// 1,025 causal, 8 q / 4 KV heads, head dim 32: 168 -> 23 us (46 TFLOP/s); 4 x 2,048 at head dim
+// 64: 3.0 -> 0.21 ms; 2,000 at 16 q / 8 KV heads, head dim 128: 3.1 -> 0.25 ms; 17 queries 11 -> 6 us.
+template <int D> struct F32Tile {
+  static constexpr int WAVES = 4;
+  static constexpr int BM = 32;            // queries per block
+  static constexpr int BN = 32 * WAVES;    // keys per step of the block
+  static constexpr int DB = D / 32;
+  static constexpr int LDS_BYTES = 2 * (32 * D + 64) * 4;  // two waves' partials
+};
+
+template <int DB> struct F32Vec;
+template <> struct F32Vec<1> { typedef float type __attribute__((ext_vector_type(1))); };
+template <> struct F32Vec<2> { typedef float type __attribute__((ext_vector_type(2))); };
+template <> struct F32Vec<4> { typedef float type __attribute__((ext_vector_type(4))); };
+
+template <int D, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D >= 128 ? 1 : 2))))
+void prefill_f32_kernel(PrefillParams p) {
+  using TL = F32Tile<D>;
+  constexpr int DB = TL::DB;
+  constexpr int NJ = D / 8;  // 16-byte pieces of a lane's half row
+  typedef typename F32Vec<DB>::type VecV;
+  extern __shared__ __attribute__((aligned(16))) float sh[];
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lane = tid % kWave;
+  const int n = lane & 31;
+  const int hi = lane >> 5;
+
+  // block -> (query tile, part, head, batch), heavy (late) causal tiles first
+  const int NS = SPLIT ? p.nsplit : 1;
+  const int HB = p.H * p.B;
+  const int qt = p.nqt - 1 - (int)blockIdx.x / (HB * NS);
+  const int part = (int)blockIdx.x % (HB * NS) / HB;
+  const int hb = (int)blockIdx.x % HB;
+  const int b = hb / p.H, h = hb % p.H;
+  const int kvh = h / p.G;
+  int kt_begin, kt_end, parts = 1;  // in steps of BN keys
+  tile_span(p.offset, p.T, p.window, 0, qt, TL::BM, TL::BN, kt_begin, kt_end);
+  if (SPLIT && !take_part(p, part, kt_begin, kt_end, parts)) return;
+
+  const int i0 = qt * TL::BM;
+  const int i_q = i0 + n;
+  const bool valid_q = i_q < p.T;
+  const int S = (int)p.offset + p.T;
+  const int qpos = (int)p.offset + i_q;
+  const int i_last = i0 + 31 < p.T - 1 ? i0 + 31 : p.T - 1;
+  const int q_lo = (int)p.offset + i0, q_hi = (int)p.offset + i_last;
+
+  // K and V through buffer resources that end with key S - 1 (host check: under 2^31 bytes): keys
+  // past it, which are masked, read zeros, and an address is one 32-bit offset
+  const unsigned row_bytes = (unsigned)p.sks * 4u;
+  const unsigned slab_bytes = (unsigned)(S - 1) * row_bytes + D * 4u;
+  const __amdgpu_buffer_rsrc_t krs = slab_rsrc(static_cast<const float*>(p.k) + b * p.skb + kvh * p.skh, slab_bytes);
+  const __amdgpu_buffer_rsrc_t vrs = slab_rsrc(static_cast<const float*>(p.v) + b * p.skb + kvh * p.skh, slab_bytes);
+  const unsigned k_lane = (unsigned)n * row_bytes + 16u * hi, v_lane = 4u * hi * row_bytes + 4u * DB * n;
+
+  // ---- Q^T: RMSNorm + RoPE in fp32 (pairs c, c + D/2 are pieces j, j + NJ/2 of one lane)
+  float q[NJ][4];
+  {
+    const float* src = static_cast<const float*>(p.q) + b * p.sqb + h * p.sqh +
+                       (int64_t)(valid_q ? i_q : p.T - 1) * p.sqt + 4 * hi;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const float4 x = *reinterpret_cast<const float4*>(src + 8 * j);
+      q[j][0] = x.x; q[j][1] = x.y; q[j][2] = x.z; q[j][3] = x.w;
+    }
+    if (p.flags & FORGE_NORM_QK) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += q[j][e] * q[j][e];
+      ss += __shfl_xor(ss, 32, kWave);
+      const float rs = rsqrtf(ss / (float)D + p.eps);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        float4 w = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        if (p.qw) w = *reinterpret_cast<const float4*>(p.qw + 8 * j + 4 * hi);
+        q[j][0] = q[j][0] * rs * w.x;
+        q[j][1] = q[j][1] * rs * w.y;
+        q[j][2] = q[j][2] * rs * w.z;
+        q[j][3] = q[j][3] * rs * w.w;
+      }
+    }
+    if (p.flags & FORGE_ROPE) {
+      const int64_t row = (int64_t)(valid_q ? i_q : p.T - 1) * p.cst + 4 * hi;
+#pragma unroll
+      for (int j = 0; j < NJ / 2; ++j) {
+        const float4 c1 = *reinterpret_cast<const float4*>(p.cos + row + 8 * j);
+        const float4 s1 = *reinterpret_cast<const float4*>(p.sin + row + 8 * j);
+        const float4 c2 = *reinterpret_cast<const float4*>(p.cos + row + 8 * j + D / 2);
+        const float4 s2 = *reinterpret_cast<const float4*>(p.sin + row + 8 * j + D / 2);
+        const float c1v[4] = {c1.x, c1.y, c1.z, c1.w}, s1v[4] = {s1.x, s1.y, s1.z, s1.w};
+        const float c2v[4] = {c2.x, c2.y, c2.z, c2.w}, s2v[4] = {s2.x, s2.y, s2.z, s2.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float a = q[j][e], z = q[j + NJ / 2][e];
+          q[j][e] = a * c1v[e] - z * s1v[e];
+          q[j + NJ / 2][e] = z * c2v[e] + a * s2v[e];
+        }
+      }
+    }
+  }
+
+  floatx16 oacc[DB];
+#pragma unroll
+  for (int d = 0; d < DB; ++d)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) oacc[d][x] = 0.0f;
+  float m_run = kNegInf, l_run = 0.0f;
+  const float c = p.scale_log2;
+
+  // first key of this wave's tile of step kt
+  auto tile_key = [&](int kt) { return kt * TL::BN + 32 * wave; };
+  floatx4 kr[NJ];
+  auto load_k = [&](int key0) {
+    const unsigned off = (unsigned)key0 * row_bytes + k_lane;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      kr[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(krs, (int)(off + 32 * j), 0, 0));
+  };
+  // a wave's tile lies outside every query's keys in the first and last steps only
+  auto needed = [&](int key0) {
+    return key0 <= q_hi && (p.window <= 0 || key0 + 31 > q_lo - p.window);
+  };
+  load_k(tile_key(kt_begin));
+  for (int kt = kt_begin; kt <= kt_end; ++kt) {
+    const int key0 = tile_key(kt);
+    if (!needed(key0)) {  // wave-uniform
+      if (kt < kt_end) load_k(tile_key(kt + 1));
+      continue;
+    }
+    VecV vr[16];
+    unsigned v_off = v_lane;
+    asm volatile("" : "+v"(v_off));  // (the 16 rows' offsets are made here, not kept over the loop)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      const int off = (int)((unsigned)(key0 + 8 * (x >> 2) + (x & 3)) * row_bytes + v_off);
+      if constexpr (DB == 1) vr[x] = __builtin_bit_cast(VecV, __builtin_amdgcn_raw_buffer_load_b32(vrs, off, 0, 0));
+      else if constexpr (DB == 2) vr[x] = __builtin_bit_cast(VecV, __builtin_amdgcn_raw_buffer_load_b64(vrs, off, 0, 0));
+      else vr[x] = __builtin_bit_cast(VecV, __builtin_amdgcn_raw_buffer_load_b128(vrs, off, 0, 0));
+    }
+    // 16 channels at a time in two chains of four steps: one chain over all the channels would
+    // round more often than the split-K path's lanes do
+    floatx16 sacc, sodd;  // (at head dim 128 the groups in two running sums)
+#pragma unroll
+    for (int j0 = 0; j0 < NJ; j0 += 2) {
+      floatx16 sc[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) sc[i][x] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) sc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[j0 + i][e], q[j0 + i][e], sc[i], 0, 0, 0);
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        const float u = sc[0][x] + sc[1][x];
+        if (D >= 128 && (j0 & 2)) sodd[x] = j0 == 2 ? u : sodd[x] + u;
+        else sacc[x] = j0 == 0 ? u : sacc[x] + u;
+      }
+      // (summed here: two partial tiles live at a time, not all of them)
+      if (D >= 128 && (j0 & 2)) asm volatile("" : "+v"(sodd));
+      else asm volatile("" : "+v"(sacc));
+    }
+    if constexpr (D >= 128) {
+#pragma unroll
+      for (int x = 0; x < 16; ++x) sacc[x] += sodd[x];
+    }
+    if (kt < kt_end) load_k(tile_key(kt + 1));
+
+#pragma unroll
+    for (int x = 0; x < 16; ++x) sacc[x] *= c;
+    const bool full = key0 + 31 <= q_lo && (p.window <= 0 || q_hi - key0 < p.window);
+    if (!full) {
+      const int base = key0 + 4 * hi;
+      const int top = qpos < S - 1 ? qpos : S - 1;  // (rows past T mask as their own position)
+      const int lo = p.window > 0 ? qpos - p.window + 1 : 0;
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        const int key = base + 8 * (x >> 2) + (x & 3);
+        sacc[x] = key <= top && key >= lo ? sacc[x] : kNegInf;
+      }
+    }
+    float mx = sacc[0];
+#pragma unroll
+    for (int x = 1; x < 16; ++x) mx = fmaxf(mx, sacc[x]);
+    mx = max_xor32(mx);
+    if (mx > m_run + kLazyLog2) {
+      const float alpha = m_run == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m_run - mx);
+      l_run *= alpha;
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) oacc[d][x] *= alpha;
+      m_run = mx;
+    }
+    const float ref = m_run == kNegInf ? 0.0f : m_run;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) sacc[x] = __builtin_amdgcn_exp2f(sacc[x] - ref);
+    {
+      float rs[8];  // summed as a tree
+#pragma unroll
+      for (int x = 0; x < 8; ++x) rs[x] = sacc[x] + sacc[x + 8];
+      l_run += ((rs[0] + rs[4]) + (rs[1] + rs[5])) + ((rs[2] + rs[6]) + (rs[3] + rs[7]));
+    }
+    // the tile's sum on its own in four chains, then into the running one: the error grows with the
+    // tiles and the keys of a chain, not with their product
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+      floatx16 sum;
+#pragma unroll
+      for (int x0 = 0; x0 < 16; x0 += 8) {
+        floatx16 ot[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int x = 0; x < 16; ++x) ot[i][x] = 0.0f;
+#pragma unroll
+        for (int x = x0; x < x0 + 8; ++x)
+          ot[x & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[x][d], sacc[x], ot[x & 1], 0, 0, 0);
+#pragma unroll
+        for (int x = 0; x < 16; ++x) sum[x] = x0 ? sum[x] + (ot[0][x] + ot[1][x]) : ot[0][x] + ot[1][x];
+        asm volatile("" : "+v"(sum));
+      }
+#pragma unroll
+      for (int x = 0; x < 16; ++x) oacc[d][x] += sum[x];
+      asm volatile("" : "+v"(oacc[d]));
+    }
+  }
+  l_run += __shfl_xor(l_run, 32, kWave);
+
+  // ---- merge the waves: (0, 2) and (1, 3), then (0, 1)
+  auto put = [&](int slot) {
+    float* dst = sh + slot * (32 * D + 64);
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) dst[(d * 16 + x) * kWave + lane] = oacc[d][x];
+    if (hi == 0) {
+      dst[32 * D + n] = m_run;
+      dst[32 * D + 32 + n] = l_run;
+    }
+  };
+  auto merge = [&](int slot) {
+    const float* src = sh + slot * (32 * D + 64);
+    const float m_o = src[32 * D + n], l_o = src[32 * D + 32 + n];
+    const float m_n = fmaxf(m_run, m_o);
+    const float a = rescale(m_run, m_n), z = rescale(m_o, m_n);
+    l_run = l_run * a + l_o * z;
+    m_run = m_n;
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int x = 0; x < 16; ++x) oacc[d][x] = oacc[d][x] * a + src[(d * 16 + x) * kWave + lane] * z;
+  };
+  if (wave >= 2) put(wave - 2);
+  __syncthreads();
+  if (wave < 2) merge(wave);
+  __syncthreads();
+  if (wave == 1) put(0);
+  __syncthreads();
+  if (wave != 0) return;
+  merge(0);
+  if (!valid_q) return;
+  // channel DB m + d, m = 8(x/4) + 4hi + x%4
+  if (SPLIT && parts > 1) {
+    const int64_t slot = part * ((int64_t)p.B * p.H * p.T) + ((int64_t)b * p.H + h) * p.T + i_q;
+    float* dst = p.ws_o + slot * D;
+#pragma unroll
+    for (int x = 0; x < 16; ++x)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) dst[DB * (8 * (x >> 2) + 4 * hi + (x & 3)) + d] = oacc[d][x];
+    if (hi == 0) p.ws_ml[slot] = make_float2(m_run, l_run);
+    return;
+  }
+  float* dst = static_cast<float*>(p.out) + b * p.sob + (int64_t)i_q * p.sot + h * p.soh;
+#pragma unroll
+  for (int x = 0; x < 16; ++x)
+#pragma unroll
+    for (int d = 0; d < DB; ++d) dst[DB * (8 * (x >> 2) + 4 * hi + (x & 3)) + d] = oacc[d][x] / l_run;
+}
+
+template <int D, bool SPLIT>
+static int launch_prefill_f32_s(PrefillParams p, hipStream_t s) {
+  using TL = F32Tile<D>;
+  p.nqt = (p.T + TL::BM - 1) / TL::BM;
+  const int64_t blocks = (int64_t)p.nqt * p.H * p.B * p.nsplit;
+  if (blocks > 0x7fffffff) return set_error("grid too large");
+  hipLaunchKernelGGL((prefill_f32_kernel<D, SPLIT>), dim3((unsigned)blocks), dim3(256), TL::LDS_BYTES, s, p);
+  return check_launch();
+}
+
+template <int D>
+static int launch_prefill_f32(const PrefillParams& p, hipStream_t s) {
+  if (p.nsplit < 2) return launch_prefill_f32_s<D, false>(p, s);
+  const int st = launch_prefill_f32_s<D, true>(p, s);
+  return st ? st : launch_prefill_combine<float, D>(p, F32Tile<D>::BM, F32Tile<D>::BN, s);
+}
+
 // How a launch splits its query tiles' keys: parts of at most `tiles` key tiles, nsplit of them
 // for the longest query tile. A launch with fewer query tiles than the CUs take (a chunk of a
 // long prompt, a short batch) otherwise leaves CUs idle behind its longest blocks: one 512-token
@@ -1029,12 +1355,13 @@ constexpr int kMaxParts = 32;
 // take 2.55 us a tile where two take 2.1 us, so four win once the blocks fill the CUs (16 q / 1 KV
 // head, a prompt of 4,096: 384 us against 631; T 512 at 8,000, split: 211 against 301), two on
 // short calls (a prompt of 1,024: 80 us against 100).
-static PrefillPlan prefill_plan(int B, int T, int H, int K, int D, int64_t offset, int window, int max_parts) {
+static PrefillPlan prefill_plan(bool f32, int B, int T, int H, int K, int D, int64_t offset, int window,
+                                int max_parts) {
   const bool wide = D == 512;
-  const int BM = wide ? WideTile<4>::BM : Tile<64>::BM;
-  const int BN = wide ? WideTile<4>::BN : D == 256 ? Tile<256>::BN : Tile<128>::BN;
+  const int BM = f32 ? F32Tile<32>::BM : wide ? WideTile<4>::BM : Tile<64>::BM;
+  const int BN = f32 ? F32Tile<32>::BN : wide ? WideTile<4>::BN : D == 256 ? Tile<256>::BN : Tile<128>::BN;
   const int G = H / K;
-  const int most_heads = !wide ? 1 : G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
+  const int most_heads = f32 || !wide ? 1 : G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1;
   const int64_t cus = device_cus();
   const int nqt = (T + BM - 1) / BM;
   if ((int64_t)nqt * (H / most_heads) * B >= 4 * cus)  // several rounds of blocks already
@@ -1061,8 +1388,12 @@ static PrefillPlan prefill_plan(int B, int T, int H, int K, int D, int64_t offse
       work1 += n;
     }
     for (int hpb = most_heads; hpb >= (most_heads == 4 ? 2 : most_heads); hpb /= 2) {
-      const double alone = hpb == 4 ? 2.55 : wide ? 2.1 : D == 256 ? 1.25 : 1.2;
-      const double shared = wide ? alone : D == 256 ? 1.05 : D == 128 ? 0.95 : 0.65;
+      double alone = hpb == 4 ? 2.55 : wide ? 2.1 : D == 256 ? 1.25 : 1.2;
+      double shared = wide ? alone : D == 256 ? 1.05 : D == 128 ? 0.95 : 0.65;
+      if (f32) {  // four waves' tiles: 128 D / 32 MFMAs of 64 clocks on each SIMD
+        alone = 0.6 + 1.0 * D / 32;
+        shared = 1.0 * D / 32;
+      }
       const int64_t blocks = blocks1 * (H / hpb) * B;
       const double per_block = (double)work1 / blocks1 + 2.5;
       const int64_t rounds = (blocks + cus - 1) / cus;
@@ -1102,17 +1433,13 @@ static size_t prefill_workspace(const PrefillPlan& plan, int B, int T, int H, in
   return (slots * sizeof(float2) + 255) / 256 * 256 + slots * D * sizeof(float);
 }
 
-static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void* q, int64_t sqb,
-                        int64_t sqh, int64_t sqt, const float* q_weight, float eps, int flags,
-                        const float* cos, const float* sin, int64_t s_cos_t, const void* k,
-                        const void* v, int64_t skb, int64_t skh, int64_t sks, int64_t offset,
-                        int window, float scale, void* out, int64_t sob, int64_t sot, int64_t soh,
-                        const int32_t* doc_lo, int64_t sdb, void* workspace, size_t workspace_bytes,
-                        void* stream) {
-  if (dtype != FORGE_BF16 && dtype != FORGE_F16)
-    return set_error("forge_attn_prefill: dtype must be bf16 or fp16 (use forge_attn_decode)");
-  if (D != 64 && D != 128 && D != 256 && D != 512)
-    return set_error("forge_attn_prefill: head dim must be 64, 128, 256 or 512");
+// Checks what every prefill entry point takes (`esize` bytes per element) and fills everything
+// of p but the documents and the plan. Returns 0, or the status of set_error.
+static int prefill_setup(PrefillParams& p, int esize, int B, int T, int H, int K, const void* q, int64_t sqb,
+                         int64_t sqh, int64_t sqt, const float* q_weight, float eps, int flags,
+                         const float* cos, const float* sin, int64_t s_cos_t, const void* k, const void* v,
+                         int64_t skb, int64_t skh, int64_t sks, int64_t offset, int window, float scale,
+                         void* out, int64_t sob, int64_t sot, int64_t soh) {
   if (B <= 0 || T <= 0 || H <= 0 || K <= 0) return set_error("sizes must be positive");
   if (H % K) return set_error("n_heads must be a multiple of the KV heads");
   if (offset < 0) return set_error("offset must be >= 0");
@@ -1121,14 +1448,14 @@ static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void
   if ((flags & FORGE_ROPE) && (!cos || !sin)) return set_error("FORGE_ROPE needs cos and sin");
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16)
     return set_error("forge_attn_prefill: tensors must be 16-byte aligned");
-  if ((sqb | sqh | sqt | skb | skh | sks) % 8)
-    return set_error("forge_attn_prefill: q/k/v strides must be multiples of 8 elements");
+  if ((sqb | sqh | sqt | skb | skh | sks) % (16 / esize))
+    return set_error("forge_attn_prefill: q/k/v strides must be multiples of 16 bytes");
   if ((sob | sot | soh) % 4) return set_error("forge_attn_prefill: out strides must be multiples of 4");
   if (offset + (int64_t)T + 256 >= (1LL << 31)) return set_error("forge_attn_prefill: positions must fit in 31 bits");
-  if (sks * 2 * 256 >= (1LL << 31)) return set_error("forge_attn_prefill: k/v row stride too large");
+  if (sks * esize * 256 >= (1LL << 31)) return set_error("forge_attn_prefill: k/v row stride too large");
   if (((uintptr_t)q_weight | (uintptr_t)cos | (uintptr_t)sin) % 16 || (cos && s_cos_t % 4))
     return set_error("forge_attn_prefill: gain and RoPE rows must be 16-byte aligned");
-  PrefillParams p{};
+  p = PrefillParams{};
   p.q = q;
   p.sqb = sqb;
   p.sqh = sqh;
@@ -1156,18 +1483,42 @@ static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void
   p.sob = sob;
   p.sot = sot;
   p.soh = soh;
-  p.doc_lo = doc_lo;
-  p.sdb = sdb;
-  const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window, workspace && !doc_lo ? kMaxParts : 1);
+  return 0;
+}
+
+// Puts a plan and its partials' workspace into p.
+static int prefill_bind(PrefillParams& p, const PrefillPlan& plan, int D, void* workspace, size_t workspace_bytes) {
   p.nsplit = plan.nsplit;
   p.split_tiles = plan.tiles;
   p.heads_per_block = plan.heads_per_block;
-  if (plan.nsplit > 1) {
-    if (workspace_bytes < prefill_workspace(plan, B, T, H, D)) return set_error("workspace too small");
-    const size_t slots = (size_t)plan.nsplit * B * H * T;
-    p.ws_ml = static_cast<float2*>(workspace);
-    p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + (slots * sizeof(float2) + 255) / 256 * 256);
-  }
+  if (plan.nsplit < 2) return 0;
+  if (workspace_bytes < prefill_workspace(plan, p.B, p.T, p.H, D)) return set_error("workspace too small");
+  const size_t slots = (size_t)plan.nsplit * p.B * p.H * p.T;
+  p.ws_ml = static_cast<float2*>(workspace);
+  p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + (slots * sizeof(float2) + 255) / 256 * 256);
+  return 0;
+}
+
+static int prefill_call(int dtype, int B, int T, int H, int K, int D, const void* q, int64_t sqb,
+                        int64_t sqh, int64_t sqt, const float* q_weight, float eps, int flags,
+                        const float* cos, const float* sin, int64_t s_cos_t, const void* k,
+                        const void* v, int64_t skb, int64_t skh, int64_t sks, int64_t offset,
+                        int window, float scale, void* out, int64_t sob, int64_t sot, int64_t soh,
+                        const int32_t* doc_lo, int64_t sdb, void* workspace, size_t workspace_bytes,
+                        void* stream) {
+  if (dtype != FORGE_BF16 && dtype != FORGE_F16)
+    return set_error("forge_attn_prefill: dtype must be bf16 or fp16 (use forge_attn_decode)");
+  if (D != 64 && D != 128 && D != 256 && D != 512)
+    return set_error("forge_attn_prefill: head dim must be 64, 128, 256 or 512");
+  PrefillParams p;
+  int st = prefill_setup(p, 2, B, T, H, K, q, sqb, sqh, sqt, q_weight, eps, flags, cos, sin, s_cos_t, k, v, skb,
+                         skh, sks, offset, window, scale, out, sob, sot, soh);
+  if (st) return st;
+  p.doc_lo = doc_lo;
+  p.sdb = sdb;
+  st = prefill_bind(p, prefill_plan(false, B, T, H, K, D, offset, window, workspace && !doc_lo ? kMaxParts : 1), D,
+                    workspace, workspace_bytes);
+  if (st) return st;
   hipStream_t s = (hipStream_t)stream;
   return dtype == FORGE_BF16 ? launch_prefill<bf16>(p, D, s) : launch_prefill<f16>(p, D, s);
 }
@@ -1206,7 +1557,7 @@ extern "C" size_t forge_attn_prefill_workspace_bytes(int dtype, int B, int T, in
   if ((dtype != FORGE_BF16 && dtype != FORGE_F16) || (D != 64 && D != 128 && D != 256 && D != 512) || B <= 0 ||
       T <= 0 || H <= 0 || K <= 0 || H % K || offset < 0 || window < 0 || offset + (int64_t)T + 256 >= (1LL << 31))
     return 0;
-  const PrefillPlan plan = prefill_plan(B, T, H, K, D, offset, window, kMaxParts);
+  const PrefillPlan plan = prefill_plan(false, B, T, H, K, D, offset, window, kMaxParts);
   return plan.nsplit > 1 ? prefill_workspace(plan, B, T, H, D) : 0;
 }
 
@@ -1223,4 +1574,35 @@ extern "C" int forge_attn_prefill_ws(int dtype, int B, int T, int H, int K, int 
   return prefill_call(dtype, B, T, H, K, D, q, sqb, sqh, sqt, q_weight, eps, flags, cos, sin,
                       s_cos_t, k, v, skb, skh, sks, offset, window, scale, out, sob, sot, soh,
                       doc_start, s_doc_b, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t forge_attn_prefill_f32_workspace_bytes(int B, int T, int H, int K, int D, int64_t offset,
+                                                         int window) {
+  if ((D != 32 && D != 64 && D != 128) || B <= 0 || T <= 0 || H <= 0 || K <= 0 || H % K || offset < 0 ||
+      window < 0 || offset + (int64_t)T + 256 >= (1LL << 31))
+    return 0;
+  const PrefillPlan plan = prefill_plan(true, B, T, H, K, D, offset, window, kMaxParts);
+  return plan.nsplit > 1 ? prefill_workspace(plan, B, T, H, D) : 0;
+}
+
+extern "C" int forge_attn_prefill_f32(int B, int T, int H, int K, int D, const void* q, int64_t sqb, int64_t sqh,
+                                      int64_t sqt, const float* q_weight, float eps, int flags,
+                                      const float* cos, const float* sin, int64_t s_cos_t, const void* k,
+                                      const void* v, int64_t skb, int64_t skh, int64_t sks, int64_t offset,
+                                      int window, float scale, void* out, int64_t sob, int64_t sot,
+                                      int64_t soh, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  if (D != 32 && D != 64 && D != 128) return set_error("forge_attn_prefill_f32: head dim must be 32, 64 or 128");
+  if ((uintptr_t)workspace % 16) return set_error("forge_attn_prefill_f32: the workspace must be 16-byte aligned");
+  PrefillParams p;
+  int st = prefill_setup(p, 4, B, T, H, K, q, sqb, sqh, sqt, q_weight, eps, flags, cos, sin, s_cos_t, k, v, skb,
+                         skh, sks, offset, window, scale, out, sob, sot, soh);
+  if (st) return st;
+  if (sks < D || sks * 4 * (offset + T + 256) >= (1LL << 31))
+    return set_error("forge_attn_prefill_f32: one (batch, kv head) slab of keys must span < 2^31 bytes");
+  st = prefill_bind(p, prefill_plan(true, B, T, H, K, D, offset, window, workspace ? kMaxParts : 1), D, workspace,
+                    workspace_bytes);
+  if (st) return st;
+  hipStream_t s = (hipStream_t)stream;
+  return D == 32 ? launch_prefill_f32<32>(p, s) : D == 64 ? launch_prefill_f32<64>(p, s) : launch_prefill_f32<128>(p, s);
 }

@@ -411,5 +411,50 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: fl
     return out
 
 
-__all__ = ["head_norm_rope", "kv_append", "attn_decode", "attn_decode_append", "attn_decode_noalloc", "attn_prefill", "decode_chunk",
+PREFILL_F32_HEAD_DIMS = (32, 64, 128)
+
+
+def prefill_f32_supported(q: torch.Tensor, cos: torch.Tensor | None = None, sin: torch.Tensor | None = None) -> bool:
+    """attn_prefill_f32 takes this q and these tables (16-byte aligned rows; attn_decode takes any)."""
+    aligned = all(t is None or (t.data_ptr() % 16 == 0 and t.dtype == torch.float32 and t.stride(-1) == 1 and
+                                all(n % 4 == 0 for n in t.stride()[:-1])) for t in (cos, sin))
+    return q.dtype == torch.float32 and q.shape[-1] in PREFILL_F32_HEAD_DIMS and aligned
+
+
+def attn_prefill_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float, offset: int = 0,
+                     window: int = 0, q_weight: torch.Tensor | None = None, eps: float = 1e-6,
+                     norm_q: bool = False, cos: torch.Tensor | None = None,
+                     sin: torch.Tensor | None = None) -> torch.Tensor:
+    """attn_prefill in fp32 (forge_attn_prefill_f32): queries at positions offset..offset+T-1 over
+    keys 0..offset+T-1 of k/v [B,K,>=offset+T,D]. Returns [B,T,H,D]."""
+    B, H, T, D = q.shape
+    Bk, K, S, Dk = k.shape
+    if Bk != B or Dk != D or v.shape != k.shape or H % K:
+        raise ValueError(f"q {tuple(q.shape)} does not fit k/v {tuple(k.shape)}")
+    if S < offset + T:
+        raise ValueError(f"k/v hold {S} positions, need offset + T = {offset + T}")
+    if k.stride() != v.stride():
+        raise ValueError("k and v must have the same strides")
+    if not prefill_f32_supported(q) or k.dtype != q.dtype or v.dtype != q.dtype:
+        raise ValueError(f"fp32 prefill takes fp32 with head dim in {PREFILL_F32_HEAD_DIMS}")
+    dev = _need_device(q, k, v, cos, sin)
+    _last_dim_contiguous(q, "q")
+    _last_dim_contiguous(k, "k")
+    c, s, s_b, s_t = _rope_tables(cos, sin, B, T, D)
+    if s_b:
+        raise ValueError("prefill takes [T, D] cos/sin shared by the batch")
+    flags = (NORM_QK if norm_q else 0) | (ROPE if c is not None else 0)
+    w = _weight(q_weight, D) if norm_q else None
+    out = torch.empty(B, T, H, D, dtype=q.dtype, device=dev)
+    need = lib().forge_attn_prefill_f32_workspace_bytes(B, T, H, K, D, int(offset), int(window))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    st = lib().forge_attn_prefill_f32(B, T, H, K, D, _ptr(q), q.stride(0), q.stride(1), q.stride(2), _ptr(w),
+                                      float(eps), flags, _ptr(c), _ptr(s), s_t, _ptr(k), _ptr(v), k.stride(0),
+                                      k.stride(1), k.stride(2), int(offset), int(window), float(scale), _ptr(out),
+                                      out.stride(0), out.stride(1), out.stride(2), _ptr(ws), need, _stream(dev))
+    check(st, "forge_attn_prefill_f32")
+    return out
+
+
+__all__ = ["head_norm_rope", "kv_append", "attn_decode", "attn_decode_append", "attn_decode_noalloc", "attn_prefill", "attn_prefill_f32", "decode_chunk",
            "decode_workspace_bytes", "attn_drafter", "prefill_supported", "dtype_code", "_lib"]

@@ -1,0 +1,111 @@
+"""fp32 prefill on matrix cores (forge_attn_prefill_f32): results at the edges of its tiles, parts and
+windows, its error against 64 bits beside the split-K path's, and the module's route to it."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+import oracle
+from conftest import gpu_available
+from helpers import gen, max_abs, randn, scale_of, tables, tol
+from sleuth_amd import _lib
+
+DEV = "cuda"
+F32 = torch.float32
+
+
+def test_rejections():
+    lib = _lib.lib()
+    size = lib.forge_attn_prefill_f32_workspace_bytes
+    assert size(1, 20, 8, 4, 32, 4000, 0) > 0 and size(8, 2048, 8, 4, 32, 0, 0) == 0
+    assert size(1, 20, 8, 4, 256, 4000, 0) == 0 and size(1, 20, 8, 3, 32, 4000, 0) == 0
+    ok = dict(D=32, sks=32, q=4096, offset=0)
+
+    def call(**kw):
+        a = {**ok, **kw}
+        return lib.forge_attn_prefill_f32(1, 20, 8, 4, a["D"], a["q"], 0, 32, 256, None, 1e-6, 0, None, None, 0, 4096,
+                                          4096, 0, 32, a["sks"], a["offset"], 0, 1.0, None, 0, 256, 32, None, 0, None)
+
+    for kw in (dict(), dict(D=256), dict(q=4100), dict(sks=34), dict(offset=-1), dict(offset=2 ** 27)):
+        assert call(**kw) < 0     # (the first: no output)
+    lib.forge_attn_prefill_ws     # bound
+    assert lib.forge_head_norm_rope(_lib.F32, None, None, 0, 0, 0, 2, 0, 0, 0, 0, 0, 0, None, 0.0, 0, None, None, 0, 0,
+                                    None) < 0
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("B,T,H,K,D,offset,window", [
+    (1, 1, 4, 4, 32, 0, 0),          # one query, one key
+    (2, 17, 8, 4, 32, 0, 0), (1, 32, 8, 4, 32, 0, 0), (1, 33, 8, 4, 64, 95, 0), (2, 129, 4, 2, 32, 127, 0),
+    (1, 200, 6, 2, 64, 0, 50),       # windows shorter and longer than a wave's tile, starting inside one
+    (1, 300, 4, 1, 128, 77, 200), (1, 150, 4, 4, 32, 1000, 1),
+    (1, 20, 4, 2, 32, 4000, 0), (1, 40, 4, 2, 128, 2500, 0),   # key-split
+    (3, 257, 16, 8, 128, 0, 0),
+])
+def test_fp32_prefill(B, T, H, K, D, offset, window):
+    from sleuth_amd import ops
+
+    S = offset + T
+    g = gen(T + D + offset)
+    q = randn(g, B, T, H, D).transpose(1, 2)
+    w = 1 + 0.1 * randn(g, D)
+    kc, vc = randn(g, B, K, S + 40, D), randn(g, B, K, S + 40, D)
+    kc[:, :, S:] = float("nan")      # positions past the call's last key are never used
+    vc[:, :, S:] = float("nan")
+    cos, sin = (t[offset:S] for t in tables(D, S, 1e4))
+    qn = oracle.head_norm_rope(q, w, 1e-6, cos, sin)
+    ref = oracle.sdpa(qn.double(), kc[:, :, :S].double(), vc[:, :, :S].double(), offset, window, scale_of(D))
+    dev = [t.to(DEV) for t in (q, kc, vc, w, cos, sin)]
+    kw = dict(scale=scale_of(D), window=window, q_weight=dev[3], eps=1e-6, norm_q=True, cos=dev[4], sin=dev[5])
+    got = ops.attn_prefill_f32(*dev[:3], offset=offset, **kw)
+    assert max_abs(got.cpu().transpose(1, 2), ref.float()) <= tol(F32)
+    # no less exact than the split-K path: both are within a few units of 2^-24 of 64 bits (2-norm), so a
+    # factor of 1.3 covers what the draw of one case moves
+    old = ops.attn_decode(*dev[:3], pos=offset, **kw)
+    err = lambda y: ((y.cpu().transpose(1, 2).double() - ref).norm() / ref.norm()).item()  # noqa: E731
+    assert err(got) <= 1.3 * max(err(old), 2.0 ** -24)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("scale", [0.0, -0.3, 4.0])
+def test_fp32_prefill_scales(scale):
+    """Equal, reversed and very peaked weights (scores move the reference maximum often)."""
+    from sleuth_amd import ops
+
+    g = gen(7)
+    q, k, v = randn(g, 1, 4, 100, 32), randn(g, 1, 2, 100, 32), randn(g, 1, 2, 100, 32)
+    s = q.double() @ k.double().repeat_interleave(2, 1).transpose(-1, -2) * scale
+    s = s.masked_fill(~torch.ones(100, 100, dtype=torch.bool).tril(), -math.inf)
+    ref = (s.softmax(-1) @ v.double().repeat_interleave(2, 1)).transpose(1, 2)
+    got = ops.attn_prefill_f32(q.to(DEV), k.to(DEV), v.to(DEV), scale=scale)
+    assert max_abs(got.cpu(), ref.float()) <= tol(F32)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+def test_module_takes_fp32_prompts_to_it_and_unaligned_tables_elsewhere(monkeypatch):
+    from sleuth_amd import ops
+    from sleuth_amd.attention import Attention
+    from sleuth_amd.config import ModelConfig
+    from sleuth_amd.kv_cache import KVCache
+
+    torch.manual_seed(3)
+    cfg = ModelConfig(vocab_size=16, d_model=128, n_layers=1, n_heads=4, n_kv_heads=2, qk_norm=True, max_seq_len=256)
+    a = Attention(cfg, 0).to(DEV).eval()
+    x = torch.randn(2, 60, 128, device=DEV)
+    cos, sin = (t[:60].to(DEV) for t in tables(32, 64, 1e4))
+    odd = [torch.empty(60 * 32 + 1, device=DEV)[1:].view(60, 32).copy_(t) for t in (cos, sin)]
+    outs, calls, fn = [], [], ops.attn_prefill_f32
+    monkeypatch.setattr(ops, "attn_prefill_f32", lambda *a, **kw: calls.append(1) or fn(*a, **kw))
+    with torch.no_grad():
+        for c, s in ((cos, sin), odd):
+            cache = KVCache([(2, 32)], 2, 128, DEV, F32)
+            outs.append((a(x, c, s, cache), cache.k[0].clone(), len(calls)))
+    assert [o[2] for o in outs] == [1, 1]
+    assert torch.equal(outs[0][1], outs[1][1])
+    assert max_abs(outs[0][0], outs[1][0]) <= 1e-5   # fp32 sums in another order
