@@ -123,6 +123,14 @@ SIGNATURES: dict[str, tuple] = {
         _p, _i64, _i64, _i64,                # out + strides (b, t, h)
         _p, C.c_size_t,                      # workspace, bytes
         _p]),
+    "forge_linear_small": (_i, [
+        _i, _i, _i, _i,                      # dtype, M, N, K
+        _p, _i64,                            # x, row stride
+        _p, _p, _i64,                        # w, w2 or None, row stride
+        _p, _p, _i, _f,                      # bias, gain, norm, eps
+        _p, _i64,                            # residual, row stride
+        _p, _i64,                            # out, row stride
+        _p]),
 }
 
 _lock = threading.Lock()

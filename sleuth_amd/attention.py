@@ -158,6 +158,29 @@ def fused_qkv_entry(weight: torch.Tensor) -> "_FusedQKV | None":
     return e if e is not None and e.owner() is weight else None
 
 
+def plain_module(m: nn.Module, cls: type) -> bool:
+    """m is exactly a `cls` that runs its own forward: no subclass, no forward hooks, nothing put
+    in place of forward. Only such modules' work may be done inside a fused launch."""
+    return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+
+
+def no_global_hooks() -> bool:
+    g = nn.modules.module
+    return not g._global_forward_hooks and not g._global_forward_pre_hooks
+
+
+def _linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, norm: RMSNorm | None = None) -> torch.Tensor:
+    """F.linear(norm(x), w, b) without autograd: one launch of this package's kernel for the few
+    rows of a decode or verify step, the library's GEMM otherwise."""
+    from . import ops
+
+    if ops.linear_small_ok(x, w):
+        if norm is None:
+            return ops.linear_small(x, w, b)
+        return ops.linear_small(x, w, b, gain=norm.weight_f32(), eps=norm.eps, norm=True)
+    return F.linear(x if norm is None else norm(x), w, b)
+
+
 class Attention(nn.Module):
     def __init__(self, cfg: ModelConfig, layer_idx: int):
         super().__init__()
@@ -186,7 +209,7 @@ class Attention(nn.Module):
         self.last_path = ""   # "hip-decode" | "hip-prefill" | "torch" (for tests and stats)
 
     # ------------------------------------------------------------------ projections
-    def _qkv_fused(self, x: torch.Tensor) -> torch.Tensor | None:
+    def _qkv_fused(self, x: torch.Tensor, norm: RMSNorm | None = None) -> torch.Tensor | None:
         """q_proj, k_proj and v_proj (attention.py:106-108) as one GEMM during GPU inference.
 
         The weights are concatenated once into a [(H + 2K)·hd, d] buffer and the projections'
@@ -198,7 +221,9 @@ class Attention(nn.Module):
         a graph is being captured (the captured GEMM would read a buffer a later rebuild
         frees): then the separate projections run. Returns None where they run: on the
         CPU, with autograd, and whenever a projection is not a plain nn.Linear or has hooks
-        (adapters, quantised layers and forward hooks see the same calls as in the reference)."""
+        (adapters, quantised layers and forward hooks see the same calls as in the reference).
+        norm: the block's RMSNorm, applied to x first (in the same launch for the few rows of a
+        decode or verify step)."""
         if not x.is_cuda or torch.is_grad_enabled() or hip_disabled():
             return None
         mods = [self.q_proj, self.k_proj] + ([self.v_proj] if self.v_proj is not None else [])
@@ -211,7 +236,7 @@ class Attention(nn.Module):
         state = tuple((t.data_ptr(), t._version, t.dtype, t.device) for t in params)
         entry = fused_qkv_entry(mods[0].weight)
         if entry is not None and entry.ids == ids and entry.state == state:
-            return F.linear(x, entry.w, entry.b)
+            return _linear(x, entry.w, entry.b, norm)
         if entry is not None and entry.ids != ids:
             return None   # the q weight is tied to another module with different k/v: no fusion
         if torch.cuda.is_current_stream_capturing():
@@ -236,7 +261,7 @@ class Attention(nn.Module):
             weakref.finalize(mods[0].weight, _FUSED_QKV.pop, key, None)
         _FUSED_QKV[key] = _FusedQKV(mods[0].weight, ids, state, w, b)
         _FusedQKV.builds += 1
-        return F.linear(x, w, b)
+        return _linear(x, w, b, norm)
 
     # ------------------------------------------------------------------ dispatch
     def _use_hip(self, q: torch.Tensor, cache, same_doc) -> tuple[bool, torch.Tensor | None]:
@@ -266,9 +291,27 @@ class Attention(nn.Module):
 
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, cache=None,
                 same_doc=None) -> torch.Tensor:
+        return self._layer(x, cos, sin, cache, same_doc)
+
+    def _out(self, y: torch.Tensor, residual: torch.Tensor | None) -> torch.Tensor:
+        """o_proj(y), plus the residual stream where the block hands it in."""
+        o = self.o_proj
+        if y.is_cuda and not torch.is_grad_enabled() and not hip_disabled() and plain_module(o, nn.Linear) and \
+                no_global_hooks():
+            from . import ops
+
+            if ops.linear_small_ok(y, o.weight):
+                return ops.linear_small(y, o.weight, o.bias, residual=residual)
+        return o(y) if residual is None else residual + o(y)
+
+    def _layer(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, cache, same_doc,
+               norm: RMSNorm | None = None, residual: torch.Tensor | None = None) -> torch.Tensor:
+        """forward(norm(x), ...) + residual, either of them None in forward itself."""
         B, T, _ = x.shape
         H, K, hd = self.n_heads, self.n_kv, self.hd
-        y = self._qkv_fused(x)
+        y = self._qkv_fused(x, norm)
+        if y is None and norm is not None:
+            x = norm(x)
         if y is not None:  # one GEMM; q, k, v are strided views of its rows
             q = y[..., :H * hd].view(B, T, H, hd).transpose(1, 2)
             k = y[..., H * hd:(H + K) * hd].view(B, T, K, hd).transpose(1, 2)
@@ -284,7 +327,7 @@ class Attention(nn.Module):
             y = self._forward_torch(q, k, v, cos, sin, cache, same_doc).transpose(1, 2)
             self.last_path = "torch"
         y = self.tap_z(y)                # [B, T, H, hd] per-head outputs
-        return self.o_proj(y.reshape(B, T, self.n_heads * self.hd))
+        return self._out(y.reshape(B, T, self.n_heads * self.hd), residual)
 
     # ------------------------------------------------------------------ HIP path
     def _forward_hip(self, q, k, v, cos, sin, cache, docs=None) -> torch.Tensor:

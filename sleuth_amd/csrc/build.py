@@ -18,7 +18,7 @@ PKG = CSRC.parent
 ROOT = PKG.parent
 LIB_DIR = PKG / "_lib"
 LIB_NAME = "libforge_attn.so"
-SOURCES = ["abi.hip", "prep.hip", "decode.hip", "prefill.hip"]
+SOURCES = ["abi.hip", "prep.hip", "decode.hip", "prefill.hip", "linear.hip"]
 ARCH = "gfx950"
 
 # -packed-fp32-ops: keep hipcc from emitting packed fp32 VALU ops (v_pk_*_f32).

@@ -17,11 +17,12 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from .attention import Attention
+from . import ops
+from .attention import Attention, hip_disabled, no_global_hooks, plain_module
 from .config import ModelConfig
 from .norm import RMSNorm
 from .rope import rope_tables
-from .taps import make_tap, name_taps
+from .taps import make_tap, name_taps, tap_active
 
 
 class SwiGLU(nn.Module):
@@ -46,7 +47,30 @@ class Block(nn.Module):
         self.tap_attn_out = make_tap()
         self.tap_resid_post = make_tap()
 
+    def _small_step(self, x: torch.Tensor) -> bool:
+        """The few rows of a decode or verify step without autograd, and nothing that listens to or
+        stands in for the block's parts: the norms and residual sums ride in the projections'
+        launches (6 launches per block instead of about 20)."""
+        m = self.mlp
+        if not x.is_cuda or torch.is_grad_enabled() or hip_disabled() or not no_global_hooks():
+            return False
+        if not (plain_module(self.norm1, RMSNorm) and plain_module(self.norm2, RMSNorm) and
+                plain_module(self.attn, Attention) and plain_module(m, SwiGLU) and plain_module(m.gate, nn.Linear) and
+                plain_module(m.up, nn.Linear) and plain_module(m.down, nn.Linear)):
+            return False
+        if tap_active(self.tap_attn_out) or tap_active(self.tap_resid_post) or m.gate.bias is not None or \
+                m.up.bias is not None or m.gate.weight.shape != m.up.weight.shape:
+            return False
+        return ops.linear_small_ok(x, m.gate.weight) and ops.linear_small_ok(x, m.up.weight) and \
+            m.down.weight.is_contiguous() and m.down.weight.dtype == x.dtype and m.gate.weight.shape[0] % 32 == 0 and \
+            m.down.weight.data_ptr() % 16 == 0
+
     def forward(self, x, cos, sin, cache=None, same_doc=None):
+        if self._small_step(x):
+            x = self.attn._layer(x, cos, sin, cache, same_doc, norm=self.norm1, residual=x)
+            m, n = self.mlp, self.norm2
+            h = ops.linear_small(x, m.gate.weight, w_up=m.up.weight, gain=n.weight_f32(), eps=n.eps, norm=True)
+            return ops.linear_small(h, m.down.weight, m.down.bias, residual=x)
         x = x + self.tap_attn_out(self.attn(self.norm1(x), cos, sin, cache, same_doc))
         return self.tap_resid_post(x + self.mlp(self.norm2(x)))
 
@@ -135,11 +159,18 @@ class Transformer(nn.Module):
             raise ValueError(f"sequence length {offset + T} exceeds max_seq_len {self.cfg.max_seq_len}")
         if getattr(cache, "static", False):
             cache.new_step()
-        rope = self.rope_rows(offset, T, cache)
+        # (fp32 rows, made once per pass: a model cast to bf16 holds its tables in bf16, and every layer
+        # would convert the same rows)
+        rope = {k: (c.float(), s.float()) for k, (c, s) in self.rope_rows(offset, T, cache).items()}
         x = self.tok_emb(idx)
         for block in self.blocks:
             x = block(x, *rope[block.kind], cache)
         if cache is not None:
             cache.advance(T)
-        h = self.norm_f(x)
-        return ModelOutput(self.lm_head(h), h if return_hidden else None)
+        n, head = self.norm_f, self.lm_head
+        if x.is_cuda and not return_hidden and not torch.is_grad_enabled() and not hip_disabled() and \
+                no_global_hooks() and plain_module(n, RMSNorm) and plain_module(head, nn.Linear) and \
+                ops.linear_small_ok(x, head.weight):
+            return ModelOutput(ops.linear_small(x, head.weight, head.bias, gain=n.weight_f32(), eps=n.eps, norm=True))
+        h = n(x)
+        return ModelOutput(head(h), h if return_hidden else None)

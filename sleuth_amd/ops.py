@@ -456,5 +456,35 @@ def attn_prefill_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale
     return out
 
 
+LINEAR_SMALL_ROWS = 16   # rows of x that forge_linear_small takes
+
+
+def linear_small_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """linear_small takes x [..., K] and w [N, K]: at most 16 rows, bf16/fp16, K a multiple of 32,
+    contiguous and aligned, on a device whose HIP path is on and with nothing (autocast,
+    tracing, a tensor subclass) between the call and the memory."""
+    K = x.shape[-1]
+    return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and
+            w.device == x.device and 0 < x.numel() <= LINEAR_SMALL_ROWS * K and K % 32 == 0 and
+            w.shape[-1] == K and type(x) is torch.Tensor and x.is_contiguous() and w.is_contiguous() and
+            x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled() and
+            not torch.compiler.is_compiling())
+
+
+def linear_small(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
+                 w_up: torch.Tensor | None = None, gain: torch.Tensor | None = None, eps: float = 0.0,
+                 norm: bool = False, residual: torch.Tensor | None = None) -> torch.Tensor:
+    """F.linear(x, w, bias) of a decode or verify step (forge_linear_small), x [..., K] as
+    linear_small_ok takes it; norm: x gets RMSNorm (gain fp32 [K]) first; w_up: returns
+    silu(x . w^T) * (x . w_up^T); residual [..., N], contiguous: added to the result."""
+    K, N = x.shape[-1], w.shape[0]
+    M = x.numel() // K
+    out = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
+    st = lib().forge_linear_small(_DTYPES[x.dtype], M, N, K, x.data_ptr(), K, w.data_ptr(), _ptr(w_up), K, _ptr(bias),
+                                  _ptr(gain), int(norm), eps, _ptr(residual), N, out.data_ptr(), N, _stream(x.device))
+    check(st, "forge_linear_small")
+    return out
+
+
 __all__ = ["head_norm_rope", "kv_append", "attn_decode", "attn_decode_append", "attn_decode_noalloc", "attn_prefill", "attn_prefill_f32", "decode_chunk",
            "decode_workspace_bytes", "attn_drafter", "prefill_supported", "dtype_code", "_lib"]

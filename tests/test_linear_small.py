@@ -1,0 +1,125 @@
+"""forge_linear_small, the projections of a decode or verify step, against torch in 64 bits with the
+eager layers' roundings, and the block's use of it."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from conftest import gpu_available
+from helpers import gen, randn
+from sleuth_amd import _lib
+
+DEV = "cuda"
+needs_gpu = pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+
+
+def test_rejections():
+    lib = _lib.lib()
+
+    def call(dtype=_lib.BF16, M=1, N=16, K=64, x=4096, sx=64, w=4096, w2=None, sw=64, bias=None, out=None):
+        return lib.forge_linear_small(dtype, M, N, K, x, sx, w, w2, sw, bias, None, 0, 0.0, None, 0, out, N, None)
+
+    for kw in (dict(), dict(dtype=_lib.F32), dict(M=17), dict(M=0), dict(K=48), dict(x=4098), dict(sw=60), dict(M=2, sx=56),
+               dict(w2=4096, bias=4096)):
+        assert call(**{"out": 4096 if kw else None, **kw}) < 0
+
+
+@pytest.mark.gpu
+@needs_gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("N,K", [(1, 32), (17, 96), (100, 1024), (256, 3104)])
+@pytest.mark.parametrize("form", ["plain", "bias", "norm", "norm+residual", "swiglu", "norm+swiglu"])
+def test_linear_small(dtype, M, N, K, form):
+    from sleuth_amd import ops
+
+    g = gen(N + K + M)
+    x = randn(g, M, K, dtype=dtype)
+    w, u = (randn(g, N, K, dtype=dtype) * 0.05 for _ in range(2))
+    bias, res, gain = randn(g, N, dtype=dtype), randn(g, M, N, dtype=dtype), 1 + 0.1 * randn(g, K)
+    rnd = lambda t: t.to(dtype).double()  # noqa: E731
+    xn = x.double()
+    if "norm" in form:
+        xn = rnd(xn * torch.rsqrt(xn.square().mean(-1, keepdim=True) + 1e-6) * gain.double())
+    y = xn @ w.double().T
+    if form == "bias":
+        y = y + bias.double()
+    if "swiglu" in form:
+        y = rnd(F.silu(rnd(y))) * rnd(xn @ u.double().T)
+    if "residual" in form:
+        y = rnd(y) + res.double()
+    d = lambda t: t.to(DEV)  # noqa: E731
+    kw = dict(w_up=d(u) if "swiglu" in form else None, gain=d(gain) if "norm" in form else None, eps=1e-6,
+              norm="norm" in form, residual=d(res) if "residual" in form else None)
+    assert ops.linear_small_ok(d(x), d(w))
+    call = lambda rows, **o: ops.linear_small(d(x)[rows].contiguous(), d(w), d(bias) if form == "bias" else None,  # noqa: E731
+                                              **{**kw, **o})
+    got = call(slice(None))
+    # relative to the value, a rounding moves it by at most 2^-p (p = 8, 11: half a spacing), and by
+    # twice that against the reference's where fp32 and 64 bits fall on either side of an edge; a
+    # single value (M = N = 1) can meet that at each of its roundings: of x, gate, silu, up, the
+    # product before the sum, and the result (whose reference is not rounded: 2^-p)
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    inner = {"plain": 0, "bias": 0, "norm": 1, "norm+residual": 2, "swiglu": 3, "norm+swiglu": 4}[form]
+    err = (got.cpu().double() - y).norm() / y.norm()
+    assert err.item() <= ulp * (1 + 2 * inner)
+    one = call(slice(M - 1, M), residual=d(res)[M - 1:] if "residual" in form else None)
+    assert torch.equal(one, got[M - 1:])      # a row does not depend on the others
+
+
+def _model(**kw):
+    from sleuth_amd.config import ModelConfig
+    from sleuth_amd.model import Transformer
+
+    torch.manual_seed(5)
+    cfg = ModelConfig(vocab_size=128, d_model=128, n_layers=2, n_heads=4, n_kv_heads=2, qk_norm=True, max_seq_len=128,
+                      ffn_hidden=160, init_std=0.05, **kw)
+    return Transformer(cfg).to(DEV, torch.bfloat16).eval()
+
+
+@pytest.mark.gpu
+@needs_gpu
+@pytest.mark.parametrize("T", [1, 5])
+def test_block_step_and_what_turns_its_fusion_off(T, monkeypatch):
+    """A decode/verify step takes four fused launches per block (and one for the head); a hook, a
+    listener, a replaced forward, autograd or a prompt keep the modules' own calls, with equal
+    logits up to bf16 roundings."""
+    from sleuth_amd import ops
+    from sleuth_amd.kv_cache import KVCache
+    from sleuth_amd.taps import listen
+
+    m = _model()
+    prompt, ids = torch.randint(0, 128, (1, 40), device=DEV), torch.randint(0, 128, (1, T), device=DEV)
+    calls, fn = [], ops.linear_small
+    monkeypatch.setattr(ops, "linear_small", lambda *a, **kw: calls.append(1) or fn(*a, **kw))
+
+    @torch.no_grad()
+    def step():
+        cache = KVCache.for_model(m, 1)
+        m(prompt, cache=cache)
+        calls.clear()
+        return m(ids, cache=cache).logits.float(), len(calls)
+
+    step()
+    fused, n = step()
+    assert n == 2 * 4 + 1
+    blk = m.blocks[0]
+
+    def same(want):
+        y, k = step()
+        assert k == want and ((y - fused).norm() / fused.norm()).item() <= 0.03   # two layers of bf16 roundings
+    seen = []
+    h = blk.norm2.register_forward_hook(lambda mod, a, out: seen.append(out.shape))
+    same(5 + 2)                                  # the other block and the head; this one's q/k/v and o_proj
+    assert len(seen) == 2                        # the prompt and the step
+    h.remove()
+    with listen(m, {"blocks.0.resid_post": lambda name, x: seen.append(1)}):
+        same(5 + 2)
+    blk.mlp.forward = type(blk.mlp).forward.__get__(blk.mlp)
+    same(5 + 2)
+    del blk.mlp.forward
+    calls.clear()
+    m(ids).logits.sum().backward()               # autograd: none
+    assert not calls and m.blocks[0].mlp.down.weight.grad is not None
