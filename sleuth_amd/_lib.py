@@ -8,10 +8,12 @@ or its ABI version differs, `lib()` raises.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libforge_attn.so"
+HOST_PATH = LIB_PATH.with_name("_forge_host.so")
 ABI_VERSION = 3
 
 F32, BF16, F16 = 0, 1, 2
@@ -163,6 +165,27 @@ def lib() -> C.CDLL:
                 raise ForgeError(f"libforge_attn ABI version {v}, expected {ABI_VERSION}: rebuild it")
             _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host module (csrc/host.cpp; loaded once). Raises if it was not built."""
+    global _host
+    if _host is not None:
+        return _host
+    lib()   # torch and the library first: the module links to both
+    with _lock:
+        if _host is None:
+            if not HOST_PATH.exists():
+                raise ForgeError(f"{HOST_PATH} is missing: build it with `python -m sleuth_amd.csrc.build` "
+                                 "(or __graft_entry__.build())")
+            spec = importlib.util.spec_from_file_location("_forge_host", HOST_PATH)
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            _host = mod
+    return _host
 
 
 def check(status: int, what: str) -> None:

@@ -172,12 +172,13 @@ def no_global_hooks() -> bool:
 def _linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, norm: RMSNorm | None = None) -> torch.Tensor:
     """F.linear(norm(x), w, b) without autograd: one launch of this package's kernel for the few
     rows of a decode or verify step, the library's GEMM otherwise."""
-    from . import ops
+    if x.numel() <= 16 * x.shape[-1]:
+        from . import ops
 
-    if ops.linear_small_ok(x, w):
-        if norm is None:
-            return ops.linear_small(x, w, b)
-        return ops.linear_small(x, w, b, gain=norm.weight_f32(), eps=norm.eps, norm=True)
+        y = ops.linear_small(x, w, b) if norm is None else \
+            ops.linear_small(x, w, b, gain=norm.weight_f32(), eps=norm.eps, norm=True)
+        if y is not None:
+            return y
     return F.linear(x if norm is None else norm(x), w, b)
 
 
@@ -231,10 +232,15 @@ class Attention(nn.Module):
             return None
         if nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks:
             return None
-        params = tuple(t for m in mods for t in (m.weight, m.bias) if t is not None)
+        params = tuple([t for m in mods for t in (m.weight, m.bias) if t is not None])
+        entry = fused_qkv_entry(mods[0].weight)
+        if entry is not None:
+            from . import ops
+
+            if ops.host().tensors_are(params, entry.ids, entry.state, entry.w):
+                return _linear(x, entry.w, entry.b, norm)
         ids = tuple(id(t) for t in params)
         state = tuple((t.data_ptr(), t._version, t.dtype, t.device) for t in params)
-        entry = fused_qkv_entry(mods[0].weight)
         if entry is not None and entry.ids == ids and entry.state == state:
             return _linear(x, entry.w, entry.b, norm)
         if entry is not None and entry.ids != ids:
@@ -296,12 +302,13 @@ class Attention(nn.Module):
     def _out(self, y: torch.Tensor, residual: torch.Tensor | None) -> torch.Tensor:
         """o_proj(y), plus the residual stream where the block hands it in."""
         o = self.o_proj
-        if y.is_cuda and not torch.is_grad_enabled() and not hip_disabled() and plain_module(o, nn.Linear) and \
-                no_global_hooks():
+        if y.numel() <= 16 * y.shape[-1] and y.is_cuda and not torch.is_grad_enabled() and not hip_disabled() and \
+                plain_module(o, nn.Linear) and no_global_hooks():
             from . import ops
 
-            if ops.linear_small_ok(y, o.weight):
-                return ops.linear_small(y, o.weight, o.bias, residual=residual)
+            r = ops.linear_small(y, o.weight, o.bias, residual=residual)
+            if r is not None:
+                return r
         return o(y) if residual is None else residual + o(y)
 
     def _layer(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, cache, same_doc,

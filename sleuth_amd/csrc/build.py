@@ -1,4 +1,5 @@
-"""Builds libforge_attn.so (the HIP kernels + C ABI) in-tree for gfx950 with hipcc.
+"""Builds libforge_attn.so (the HIP kernels + C ABI) in-tree for gfx950 with hipcc, and the native
+host module (host.cpp) with g++.
 
 Usage: python -m sleuth_amd.csrc.build [-v]
 The library lands in sleuth_amd/_lib/ so that it travels with the source tree.
@@ -18,6 +19,7 @@ PKG = CSRC.parent
 ROOT = PKG.parent
 LIB_DIR = PKG / "_lib"
 LIB_NAME = "libforge_attn.so"
+HOST_NAME = "_forge_host.so"
 SOURCES = ["abi.hip", "prep.hip", "decode.hip", "prefill.hip", "linear.hip"]
 ARCH = "gfx950"
 
@@ -54,8 +56,35 @@ def _compile(src: Path, obj: Path, verbose: bool) -> None:
         print(r.stderr, file=sys.stderr)
 
 
+def build_host(verbose: bool = False) -> Path:
+    """Compile the native host module (host.cpp, plain C++ against torch's headers) beside the
+    library, which must be there; returns its path."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    torch_lib = Path(torch.__file__).resolve().parent / "lib"
+    out = LIB_DIR / HOST_NAME
+    tmp = out.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
+    for inc in include_paths("cuda") + [sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", inc]
+    cmd += [str(CSRC / "host.cpp"), "-o", str(tmp), f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch_python", f"-L{LIB_DIR}", "-lforge_attn", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, out)
+    return out
+
+
 def build(verbose: bool = False) -> Path:
-    """Compile every source and link the shared library; returns its path."""
+    """Compile every source, link the shared library and build the host module; returns the
+    library's path."""
     obj_dir = PKG / "_build"
     obj_dir.mkdir(exist_ok=True)
     LIB_DIR.mkdir(exist_ok=True)
@@ -72,6 +101,7 @@ def build(verbose: bool = False) -> Path:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, out)
+    build_host(verbose)
     return out
 
 

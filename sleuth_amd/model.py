@@ -52,25 +52,27 @@ class Block(nn.Module):
         stands in for the block's parts: the norms and residual sums ride in the projections'
         launches (6 launches per block instead of about 20)."""
         m = self.mlp
-        if not x.is_cuda or torch.is_grad_enabled() or hip_disabled() or not no_global_hooks():
+        if x.numel() > ops.LINEAR_SMALL_ROWS * x.shape[-1] or not x.is_cuda or torch.is_grad_enabled() or \
+                hip_disabled() or not no_global_hooks():
             return False
         if not (plain_module(self.norm1, RMSNorm) and plain_module(self.norm2, RMSNorm) and
                 plain_module(self.attn, Attention) and plain_module(m, SwiGLU) and plain_module(m.gate, nn.Linear) and
                 plain_module(m.up, nn.Linear) and plain_module(m.down, nn.Linear)):
             return False
         if tap_active(self.tap_attn_out) or tap_active(self.tap_resid_post) or m.gate.bias is not None or \
-                m.up.bias is not None or m.gate.weight.shape != m.up.weight.shape:
+                m.up.bias is not None:
             return False
-        return ops.linear_small_ok(x, m.gate.weight) and ops.linear_small_ok(x, m.up.weight) and \
-            m.down.weight.is_contiguous() and m.down.weight.dtype == x.dtype and m.gate.weight.shape[0] % 32 == 0 and \
-            m.down.weight.data_ptr() % 16 == 0
+        return True
 
     def forward(self, x, cos, sin, cache=None, same_doc=None):
         if self._small_step(x):
             x = self.attn._layer(x, cos, sin, cache, same_doc, norm=self.norm1, residual=x)
             m, n = self.mlp, self.norm2
             h = ops.linear_small(x, m.gate.weight, w_up=m.up.weight, gain=n.weight_f32(), eps=n.eps, norm=True)
-            return ops.linear_small(h, m.down.weight, m.down.bias, residual=x)
+            if h is None:
+                return x + m(n(x))
+            y = ops.linear_small(h, m.down.weight, m.down.bias, residual=x)
+            return y if y is not None else x + m.down(h)
         x = x + self.tap_attn_out(self.attn(self.norm1(x), cos, sin, cache, same_doc))
         return self.tap_resid_post(x + self.mlp(self.norm2(x)))
 
@@ -168,9 +170,11 @@ class Transformer(nn.Module):
         if cache is not None:
             cache.advance(T)
         n, head = self.norm_f, self.lm_head
-        if x.is_cuda and not return_hidden and not torch.is_grad_enabled() and not hip_disabled() and \
-                no_global_hooks() and plain_module(n, RMSNorm) and plain_module(head, nn.Linear) and \
-                ops.linear_small_ok(x, head.weight):
-            return ModelOutput(ops.linear_small(x, head.weight, head.bias, gain=n.weight_f32(), eps=n.eps, norm=True))
+        if x.numel() <= ops.LINEAR_SMALL_ROWS * x.shape[-1] and x.is_cuda and not return_hidden and \
+                not torch.is_grad_enabled() and not hip_disabled() and no_global_hooks() and \
+                plain_module(n, RMSNorm) and plain_module(head, nn.Linear):
+            y = ops.linear_small(x, head.weight, head.bias, gain=n.weight_f32(), eps=n.eps, norm=True)
+            if y is not None:
+                return ModelOutput(y)
         h = n(x)
         return ModelOutput(head(h), h if return_hidden else None)

@@ -1,7 +1,8 @@
 """Torch-tensor front ends of the HIP kernels (C ABI in include/forge_attn.h).
 
 These functions only check shapes on the host, pick pointers/strides and launch on
-torch's current stream. They never compute anything themselves: if the library is not
+torch's current stream; calls whose arguments need no conversion are checked and launched by the
+native host module (csrc/host.cpp), which returns None for the others. They never compute anything themselves: if the library is not
 built they raise (sleuth_amd._lib.ForgeError).
 
 Layouts (reference names): q [B,H,T,D] (any strides, last dim contiguous: the transposed
@@ -14,7 +15,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._lib import BF16, F16, F32, NORM_QK, NORM_V, ROPE, WS_ZEROED, check, lib
+from ._lib import BF16, F16, F32, NORM_QK, NORM_V, ROPE, WS_ZEROED, check, host, lib
 
 _DTYPES = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 
@@ -127,6 +128,11 @@ def kv_append(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor, v_cache: 
               cos: torch.Tensor | None = None, sin: torch.Tensor | None = None) -> None:
     """Normalise/rotate the new k (and v_norm v) and write them into the cache at
     base_b + t (KVCache.update, kv_cache.py:52-60; StaticKVCache.update 107-114)."""
+    if pos_dev is None and row_pos is None:
+        st = host().kv_append(k, v, k_cache, v_cache, int(pos or 0), k_weight, float(eps), bool(norm_k), bool(norm_v),
+                              cos, sin)
+        if st is not None:
+            return check(st, "forge_kv_append")
     B, K, T, D = k.shape
     if v.shape != k.shape:
         raise ValueError(f"k {tuple(k.shape)} and v {tuple(v.shape)} differ")
@@ -269,6 +275,12 @@ def attn_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
     Without a workspace (and outside graph capture) the call uses this module's zeroed
     workspace for the current stream (FORGE_WS_ZEROED: no ticket-reset kernel);
     workspace_zeroed=True makes the same promise for a workspace the caller cleared once."""
+    if out is None and workspace is None:
+        r = host().decode_append(_STREAM_WS, q, k, v, k_cache, v_cache, float(scale), pos, pos_dev, row_pos, max_kv_len,
+                                 window, q_weight, k_weight, float(eps), bool(norm_q), bool(norm_k), bool(norm_v), cos,
+                                 sin, chunk)
+        if r is not None:
+            return r if r.__class__ is not int else check(r, "forge_attn_decode_append")
     B, K, T, D = k.shape
     if v.shape != k.shape or q.shape[0] != B or q.shape[2] != T or q.shape[3] != D:
         raise ValueError(f"q {tuple(q.shape)}, k {tuple(k.shape)} and v {tuple(v.shape)} do not fit")
@@ -364,6 +376,10 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: fl
     It must be non-decreasing along T and at most the query's own position: checked here
     (two host synchronisations) unless check_doc_start is False, for a caller that built
     it so (the module's own starts, taken from the mask), or under graph capture."""
+    if out is None and doc_start is None and q.dtype != torch.float32:
+        r = host().prefill(q, k, v, float(scale), offset, window, q_weight, float(eps), bool(norm_q), cos, sin)
+        if r is not None:
+            return r if r.__class__ is not int else check(r, "forge_attn_prefill")
     B, H, T, D = q.shape
     Bk, K, S, Dk = k.shape
     if Bk != B or Dk != D or v.shape != k.shape or H % K:
@@ -427,6 +443,10 @@ def attn_prefill_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale
                      sin: torch.Tensor | None = None) -> torch.Tensor:
     """attn_prefill in fp32 (forge_attn_prefill_f32): queries at positions offset..offset+T-1 over
     keys 0..offset+T-1 of k/v [B,K,>=offset+T,D]. Returns [B,T,H,D]."""
+    if q.dtype == torch.float32:
+        r = host().prefill(q, k, v, float(scale), offset, window, q_weight, float(eps), bool(norm_q), cos, sin)
+        if r is not None:
+            return r if r.__class__ is not int else check(r, "forge_attn_prefill_f32")
     B, H, T, D = q.shape
     Bk, K, S, Dk = k.shape
     if Bk != B or Dk != D or v.shape != k.shape or H % K:
@@ -459,31 +479,19 @@ def attn_prefill_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale
 LINEAR_SMALL_ROWS = 16   # rows of x that forge_linear_small takes
 
 
-def linear_small_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """linear_small takes x [..., K] and w [N, K]: at most 16 rows, bf16/fp16, K a multiple of 32,
-    contiguous and aligned, on a device whose HIP path is on and with nothing (autocast,
-    tracing, a tensor subclass) between the call and the memory."""
-    K = x.shape[-1]
-    return (x.is_cuda and x.dtype in (torch.bfloat16, torch.float16) and w.dtype == x.dtype and
-            w.device == x.device and 0 < x.numel() <= LINEAR_SMALL_ROWS * K and K % 32 == 0 and
-            w.shape[-1] == K and type(x) is torch.Tensor and x.is_contiguous() and w.is_contiguous() and
-            x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled() and
-            not torch.compiler.is_compiling())
-
-
 def linear_small(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
                  w_up: torch.Tensor | None = None, gain: torch.Tensor | None = None, eps: float = 0.0,
-                 norm: bool = False, residual: torch.Tensor | None = None) -> torch.Tensor:
-    """F.linear(x, w, bias) of a decode or verify step (forge_linear_small), x [..., K] as
-    linear_small_ok takes it; norm: x gets RMSNorm (gain fp32 [K]) first; w_up: returns
-    silu(x . w^T) * (x . w_up^T); residual [..., N], contiguous: added to the result."""
-    K, N = x.shape[-1], w.shape[0]
-    M = x.numel() // K
-    out = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
-    st = lib().forge_linear_small(_DTYPES[x.dtype], M, N, K, x.data_ptr(), K, w.data_ptr(), _ptr(w_up), K, _ptr(bias),
-                                  _ptr(gain), int(norm), eps, _ptr(residual), N, out.data_ptr(), N, _stream(x.device))
-    check(st, "forge_linear_small")
-    return out
+                 norm: bool = False, residual: torch.Tensor | None = None) -> torch.Tensor | None:
+    """F.linear(x, w, bias) of a decode or verify step (forge_linear_small), without autograd;
+    norm: x gets RMSNorm (gain fp32 [K]) first; w_up: silu(x . w^T) * (x . w_up^T); residual [..., N]:
+    added to the result. None where the call is not of the kernel's form (the caller then makes
+    the torch calls): it takes bf16/fp16 on one GPU, x [..., K] of at most 16 rows, K a multiple of
+    32, everything contiguous and 16-byte aligned, and nothing (autocast, tracing, a tensor
+    subclass) between the call and the memory."""
+    if torch.is_autocast_enabled() or torch.compiler.is_compiling():
+        return None
+    r = host().linear_small(x, w, bias, w_up, gain, float(eps), bool(norm), residual)
+    return r if r.__class__ is not int else check(r, "forge_linear_small")
 
 
 __all__ = ["head_norm_rope", "kv_append", "attn_decode", "attn_decode_append", "attn_decode_noalloc", "attn_prefill", "attn_prefill_f32", "decode_chunk",

@@ -53,7 +53,6 @@ def test_linear_small(dtype, M, N, K, form):
     d = lambda t: t.to(DEV)  # noqa: E731
     kw = dict(w_up=d(u) if "swiglu" in form else None, gain=d(gain) if "norm" in form else None, eps=1e-6,
               norm="norm" in form, residual=d(res) if "residual" in form else None)
-    assert ops.linear_small_ok(d(x), d(w))
     call = lambda rows, **o: ops.linear_small(d(x)[rows].contiguous(), d(w), d(bias) if form == "bias" else None,  # noqa: E731
                                               **{**kw, **o})
     got = call(slice(None))
