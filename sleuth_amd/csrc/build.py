@@ -20,7 +20,9 @@ ROOT = PKG.parent
 LIB_DIR = PKG / "_lib"
 LIB_NAME = "libforge_attn.so"
 HOST_NAME = "_forge_host.so"
-SOURCES = ["abi.hip", "prep.hip", "decode.hip", "prefill.hip", "linear.hip"]
+# (source, defines, object name); decode.hip's kernels are built per dtype, side by side
+SOURCES = [("abi.hip", [], "abi"), ("prep.hip", [], "prep"), ("prefill.hip", [], "prefill"), ("linear.hip", [], "linear"),
+           *(("decode.hip", [f"-DFORGE_DECODE_PART={n}"], f"decode{n}") for n in range(4))]
 ARCH = "gfx950"
 
 # -packed-fp32-ops: keep hipcc from emitting packed fp32 VALU ops (v_pk_*_f32).
@@ -45,8 +47,8 @@ def hipcc() -> str:
     return exe
 
 
-def _compile(src: Path, obj: Path, verbose: bool) -> None:
-    cmd = [hipcc(), *HIPCC_FLAGS, "-I", str(ROOT / "include"), "-c", str(src), "-o", str(obj)]
+def _compile(src: Path, defines: list[str], obj: Path, verbose: bool) -> None:
+    cmd = [hipcc(), *HIPCC_FLAGS, *defines, "-I", str(ROOT / "include"), "-c", str(src), "-o", str(obj)]
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -88,10 +90,10 @@ def build(verbose: bool = False) -> Path:
     obj_dir = PKG / "_build"
     obj_dir.mkdir(exist_ok=True)
     LIB_DIR.mkdir(exist_ok=True)
-    objs = [obj_dir / (Path(s).stem + ".o") for s in SOURCES]
+    objs = [obj_dir / (name + ".o") for _, _, name in SOURCES]
     jobs = min(len(SOURCES), int(os.environ.get("MAX_JOBS", "8")))
     with cf.ThreadPoolExecutor(jobs) as ex:
-        list(ex.map(lambda so: _compile(CSRC / so[0], so[1], verbose), zip(SOURCES, objs)))
+        list(ex.map(lambda so: _compile(CSRC / so[0][0], so[0][1], so[1], verbose), zip(SOURCES, objs)))
     out = LIB_DIR / LIB_NAME
     tmp = out.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]

@@ -25,6 +25,12 @@
 // (score -inf -> weight 0, reference max unchanged), and merges run in a fixed order. So
 // a row's output does not depend on T or on the other rows in the call: a verify row
 // equals the decode of that token alone, bit for bit (same chunk).
+//
+// The file is built in four parts side by side (build.py): FORGE_DECODE_PART 0 holds the entry
+// points, 1, 2 and 3 the kernels of bf16, fp16 and fp32.
+#ifndef FORGE_DECODE_PART
+#define FORGE_DECODE_PART 0
+#endif
 #include <limits.h>
 #include <stdio.h>
 
@@ -2166,10 +2172,13 @@ static int vec_of(int dtype) { return dtype == FORGE_F32 ? 4 : 8; }
 template <int D> constexpr int split_max_rows() { return D >= 512 ? 4 : 8; }
 static int rows_per_block(int rows_total, int D) {
   const int cap = D >= 512 ? split_max_rows<512>() : split_max_rows<256>();
-  if (rows_total >= cap) return cap;
-  int r = 1;
-  while (r < rows_total) r <<= 1;
-  return r;
+  // as few blocks as the cap allows, of equal size: a block's VALU work goes with its rows, valid or
+  // not (a row's own arithmetic does not depend on ROWS, so neither do its bits). 10 rows (16 q /
+  // 8 KV heads, T = 5, head dim 128, 8 rows of 6,005 fp16 keys) as 5 + 5 against 8 + 2 of 8: 87
+  // against 122 us per step.
+  const int blocks = (rows_total + cap - 1) / cap;
+  const int r = (rows_total + blocks - 1) / blocks;
+  return r == 7 ? 8 : r;
 }
 
 static int keys_per_iter(int dtype, int D) { return (kSplitThreads / (D / vec_of(dtype))) * kSplitNK; }
@@ -2329,7 +2338,7 @@ constexpr int kPersistBlocksPerCU = 2;
 // graph-capturable.
 static int resident_blocks(const void* kernel) {
   struct Entry { int dev; const void* k; int n; };
-  static Entry cache[64];
+  static Entry cache[128];
   static int used = 0;
   static std::mutex mu;
   int dev = 0;
@@ -2342,7 +2351,7 @@ static int resident_blocks(const void* kernel) {
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kSplitThreads, 0) != hipSuccess) return 0;
   if (per_cu > kPersistBlocksPerCU) per_cu = kPersistBlocksPerCU;
   const int n = ncu * (per_cu > 0 ? per_cu : 1);
-  if (used < 64) cache[used++] = Entry{dev, kernel, n};
+  if (used < 128) cache[used++] = Entry{dev, kernel, n};
   return n;
 }
 
@@ -2363,17 +2372,16 @@ static int launch_split_d(SplitParams p, int rows, hipStream_t s) {
   const int n_rb = (p.rows_total + rows - 1) / rows;
   const void* kern = nullptr;
   switch (rows) {
-    case 1: kern = reinterpret_cast<const void*>(&splitk_kernel<T, D, 1>); break;
-    case 2: kern = reinterpret_cast<const void*>(&splitk_kernel<T, D, 2>); break;
-    case 4: kern = reinterpret_cast<const void*>(&splitk_kernel<T, D, 4>); break;
-    case 8:
-      if constexpr (split_max_rows<D>() >= 8) {
-        kern = reinterpret_cast<const void*>(&splitk_kernel<T, D, 8>);
-        break;
-      }
-      return set_error("internal: rows per block");
-    default: return set_error("internal: rows per block");
+#define FORGE_ROWS(R) \
+  case R: kern = reinterpret_cast<const void*>(&splitk_kernel<T, D, R>); break;
+    FORGE_ROWS(1) FORGE_ROWS(2) FORGE_ROWS(3) FORGE_ROWS(4)
+#undef FORGE_ROWS
+#define FORGE_ROWS(R) \
+  case R: if constexpr (split_max_rows<D>() >= R) kern = reinterpret_cast<const void*>(&splitk_kernel<T, D, R>); break;
+    FORGE_ROWS(5) FORGE_ROWS(6) FORGE_ROWS(8)
+#undef FORGE_ROWS
   }
+  if (!kern) return set_error("internal: rows per block");
   dim3 grid;
   // Persistent only for per-row lengths (ragged rows): there it saves the blocks a dense
   // grid would spend past each row's end. With one position for every row, host-known or on
@@ -2403,12 +2411,15 @@ static int launch_split_d(SplitParams p, int rows, hipStream_t s) {
   switch (rows) {
 #define FORGE_ROWS(R) \
   case R: hipLaunchKernelGGL((splitk_kernel<T, D, R>), grid, dim3(kSplitThreads), 0, s, p); break;
-    FORGE_ROWS(1) FORGE_ROWS(2) FORGE_ROWS(4)
+    FORGE_ROWS(1) FORGE_ROWS(2) FORGE_ROWS(3) FORGE_ROWS(4)
 #undef FORGE_ROWS
-    case 8:
-      if constexpr (split_max_rows<D>() >= 8)
-        hipLaunchKernelGGL((splitk_kernel<T, D, 8>), grid, dim3(kSplitThreads), 0, s, p);
-      break;
+#define FORGE_ROWS(R) \
+  case R: \
+    if constexpr (split_max_rows<D>() >= R) \
+      hipLaunchKernelGGL((splitk_kernel<T, D, R>), grid, dim3(kSplitThreads), 0, s, p); \
+    break;
+    FORGE_ROWS(5) FORGE_ROWS(6) FORGE_ROWS(8)
+#undef FORGE_ROWS
   }
   int st = check_launch();
   if (st || p.max_chunks < 2) return st;
@@ -2466,13 +2477,13 @@ static int launch_verify_d(SplitParams p, hipStream_t s) {
 }
 
 template <typename T>
-static int launch_verify(const SplitParams& p, int D, hipStream_t s) {
+int launch_verify(const SplitParams& p, int D, hipStream_t s) {
   return D == 128 ? launch_verify_d<T, 128>(p, s)
                   : D == 256 ? launch_verify_d<T, 256>(p, s) : launch_verify_d<T, 512>(p, s);
 }
 
 template <typename T>
-static int launch_split(const SplitParams& p, int D, int rows, hipStream_t s) {
+int launch_split(const SplitParams& p, int D, int rows, hipStream_t s) {
   switch (D) {
     case 32: return launch_split_d<T, 32>(p, rows, s);
     case 64: return launch_split_d<T, 64>(p, rows, s);
@@ -2485,8 +2496,25 @@ static int launch_split(const SplitParams& p, int D, int rows, hipStream_t s) {
   }
 }
 
+#if FORGE_DECODE_PART == 0
+extern template int launch_verify<bf16>(const SplitParams&, int, hipStream_t);
+extern template int launch_verify<f16>(const SplitParams&, int, hipStream_t);
+extern template int launch_split<bf16>(const SplitParams&, int, int, hipStream_t);
+extern template int launch_split<f16>(const SplitParams&, int, int, hipStream_t);
+extern template int launch_split<float>(const SplitParams&, int, int, hipStream_t);
+#elif FORGE_DECODE_PART == 1
+template int launch_verify<bf16>(const SplitParams&, int, hipStream_t);
+template int launch_split<bf16>(const SplitParams&, int, int, hipStream_t);
+#elif FORGE_DECODE_PART == 2
+template int launch_verify<f16>(const SplitParams&, int, hipStream_t);
+template int launch_split<f16>(const SplitParams&, int, int, hipStream_t);
+#else
+template int launch_split<float>(const SplitParams&, int, int, hipStream_t);
+#endif
+
 }  // namespace forge
 
+#if FORGE_DECODE_PART == 0
 using namespace forge;
 
 extern "C" int forge_attn_decode_chunk(int dtype, int B, int T, int H, int K, int D,
@@ -2773,3 +2801,4 @@ extern "C" int forge_attn_decode_noalloc(int dtype, int B, int T, int H, int K, 
   }
   return decode_launch(p, dtype, D, (hipStream_t)stream);
 }
+#endif  // FORGE_DECODE_PART == 0
