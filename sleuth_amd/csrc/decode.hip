@@ -853,7 +853,7 @@ void splitk_kernel(SplitParams p) {
 
 // Zeroes the work ticket of the next persistent launch on this stream (a kernel rather
 // than a memset, so that the call can be captured into a graph).
-__global__ void ticket_reset_kernel(int* ctr) {
+static __global__ void ticket_reset_kernel(int* ctr) {
   if (threadIdx.x == 0) ctr[0] = 0;
 }
 
