@@ -259,13 +259,13 @@ int forge_attn_prefill_f32(int B, int T, int H, int K, int D, const void* q, int
  * attention, attention.py:106-108,157, and the SwiGLU MLP and head of transformer.py:75-99), bf16/fp16,
  * fp32 sums. x [M, K] with row stride sx, W [N, K] with row stride sw (nn.Linear's layout), K a
  * multiple of 32, y [M, N] with row stride so. Optional, each rounding to the dtype where the
- * eager layers do: norm != 0: RMSNorm of x's rows first (gain fp32 [K] or NULL, eps); w2 != NULL:
+ * eager layers do: norm != 0: RMSNorm of x's rows first (gain [K] of gain_dtype: fp32 or x's type; eps); w2 != NULL:
  * y = silu(x . W^T) * (x . w2^T); bias [N]; residual [M, N] (row stride sr): added last.
  */
 int forge_linear_small(int dtype, int M, int N, int K, const void* x, int64_t sx, const void* w,
-                       const void* w2, int64_t sw, const void* bias, const float* gain, int norm,
-                       float eps, const void* residual, int64_t sr, void* out, int64_t so,
-                       void* stream);
+                       const void* w2, int64_t sw, const void* bias, const void* gain,
+                       int gain_dtype, int norm, float eps, const void* residual, int64_t sr,
+                       void* out, int64_t so, void* stream);
 
 #ifdef __cplusplus
 }

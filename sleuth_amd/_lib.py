@@ -129,7 +129,7 @@ SIGNATURES: dict[str, tuple] = {
         _i, _i, _i, _i,                      # dtype, M, N, K
         _p, _i64,                            # x, row stride
         _p, _p, _i64,                        # w, w2 or None, row stride
-        _p, _p, _i, _f,                      # bias, gain, norm, eps
+        _p, _p, _i, _i, _f,                  # bias, gain, gain dtype, norm, eps
         _p, _i64,                            # residual, row stride
         _p, _i64,                            # out, row stride
         _p]),

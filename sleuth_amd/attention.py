@@ -176,7 +176,7 @@ def _linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, norm: RMSN
         from . import ops
 
         y = ops.linear_small(x, w, b) if norm is None else \
-            ops.linear_small(x, w, b, gain=norm.weight_f32(), eps=norm.eps, norm=True)
+            ops.linear_small(x, w, b, gain=norm.weight, eps=norm.eps, norm=True)
         if y is not None:
             return y
     return F.linear(x if norm is None else norm(x), w, b)

@@ -18,16 +18,17 @@ namespace {
 
 using at::Tensor;
 
-// A tensor as plain memory on a GPU: no subclass, functorch wrapper or fake tensor.
+// A tensor as plain memory on a GPU: no subclass, functorch wrapper, fake tensor or forward-mode dual.
 bool plain(const Tensor& t) {
   return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.unsafeGetTensorImpl()->is_python_dispatch() &&
-         t.has_storage() && !t.is_conj() && !t.is_neg() &&
+         t.has_storage() && !t.is_conj() && !t.is_neg() && !t._fw_grad(0).defined() &&
          !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched,
                                                    c10::DispatchKey::FuncTorchGradWrapper,
                                                    c10::DispatchKey::Functionalize, c10::DispatchKey::Python}));
 }
 
-// The tensor behind a Python argument; false for anything that is no plain GPU tensor.
+// The tensor behind a Python argument (a Parameter counts as one); false for anything that is no
+// plain GPU tensor.
 bool take(PyObject* o, Tensor& t) {
   if (!THPVariable_CheckExact(o)) return false;
   t = THPVariable_Unpack(o);
@@ -271,21 +272,11 @@ PyObject* prefill_impl(PyObject* const* a) {
 // most 16 rows, w and w_up [N, K], residual [..., N]
 PyObject* linear_small_impl(PyObject* const* a) {
   Tensor x, w, b, up, gain, res;
-  PyObject* wo = a[1];  // a Parameter is as good as a tensor here
-  if (!take(a[0], x) || !THPVariable_Check(wo) || !take_opt(a[4], gain) || !take_opt(a[7], res)) return nullptr;
-  w = THPVariable_Unpack(wo);
-  if (a[2] != Py_None) {
-    if (!THPVariable_Check(a[2])) return nullptr;
-    b = THPVariable_Unpack(a[2]);
-    if (!plain(b)) return nullptr;
-  }
-  if (a[3] != Py_None) {
-    if (!THPVariable_Check(a[3])) return nullptr;
-    up = THPVariable_Unpack(a[3]);
-    if (!plain(up)) return nullptr;
-  }
+  if (!take(a[0], x) || !take(a[1], w) || !take_opt(a[2], b) || !take_opt(a[3], up) || !take_opt(a[4], gain) ||
+      !take_opt(a[7], res))
+    return nullptr;
   float eps;
-  if (!as_float(a[5], eps) || !plain(w) || x.dim() < 1 || w.dim() != 2) return nullptr;
+  if (!as_float(a[5], eps) || x.dim() < 1 || w.dim() != 2) return nullptr;
   const bool norm = a[6] == Py_True;
   const int64_t K = x.size(-1), N = w.size(0);
   const int dt = dtype_of(x);
@@ -295,7 +286,11 @@ PyObject* linear_small_impl(PyObject* const* a) {
     return nullptr;
   for (const Tensor* t : {&w, &b, &up, &res})
     if (t->defined() && (t->scalar_type() != x.scalar_type() || t->device() != dev || !t->is_contiguous())) return nullptr;
-  if ((b.defined() && b.numel() != N) || (up.defined() && up.sizes() != w.sizes()) || !gain_ok(gain, K, dev)) return nullptr;
+  if ((b.defined() && b.numel() != N) || (up.defined() && up.sizes() != w.sizes())) return nullptr;
+  if (norm && !gain.defined()) return nullptr;
+  if (gain.defined() && ((gain.scalar_type() != at::kFloat && gain.scalar_type() != x.scalar_type()) ||
+                         gain.device() != dev || !gain.is_contiguous() || gain.numel() != K))
+    return nullptr;
   const int64_t M = x.numel() / K;
   if (res.defined() && res.numel() != M * N) return nullptr;
   if (((uintptr_t)ptr(x) | (uintptr_t)ptr(w) | (uintptr_t)ptr(up) | (uintptr_t)ptr(gain)) % 16) return nullptr;
@@ -303,7 +298,7 @@ PyObject* linear_small_impl(PyObject* const* a) {
   shape.back() = N;
   Tensor out = at::empty(shape, x.options().requires_grad(false));
   const int st = forge_linear_small(dt, (int)M, (int)N, (int)K, ptr(x), K, ptr(w), ptr(up), K, ptr(b),
-                                    static_cast<const float*>(ptr(gain)), norm, eps, ptr(res), N, out.data_ptr(), N,
+                                    ptr(gain), gain.defined() ? dtype_of(gain) : FORGE_F32, norm, eps, ptr(res), N, out.data_ptr(), N,
                                     c10::hip::getCurrentHIPStream(dev.index()).stream());
   return result(st, out);
 }

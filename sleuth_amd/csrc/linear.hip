@@ -47,7 +47,8 @@ struct LinearParams {
   const void* w2;  // SwiGLU: w is the gate, w2 the up projection
   int64_t sw;
   const void* bias;
-  const float* gain;  // RMSNorm of x (norm != 0), or null
+  const void* gain;  // RMSNorm of x (norm != 0), or null; fp32 or of x's type, as the module holds it
+  int gain_f32;
   int norm;
   float eps;
   const void* res;
@@ -136,7 +137,8 @@ void linear_small_kernel(LinearParams p) {
           for (int e = 0; e < 8; ++e) v[e] *= rs;
           if (p.gain) {
             float w[8];
-            load_f32x8(p.gain + 32 * s + 8 * g, w);
+            if (p.gain_f32) load_f32x8(static_cast<const float*>(p.gain) + 32 * s + 8 * g, w);
+            else unpack16<T>(load16(static_cast<const T*>(p.gain) + 32 * s + 8 * g), w);
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] *= w[e];
           }
@@ -193,8 +195,8 @@ static int launch_linear(const LinearParams& p, hipStream_t s) {
 using namespace forge;
 
 extern "C" int forge_linear_small(int dtype, int M, int N, int K, const void* x, int64_t sx, const void* w,
-                                  const void* w2, int64_t sw, const void* bias, const float* gain, int norm,
-                                  float eps, const void* residual, int64_t sr, void* out, int64_t so,
+                                  const void* w2, int64_t sw, const void* bias, const void* gain,
+                                  int gain_dtype, int norm, float eps, const void* residual, int64_t sr, void* out, int64_t so,
                                   void* stream) {
   clear_error();
   if (dtype != FORGE_BF16 && dtype != FORGE_F16) return set_error("forge_linear_small: dtype must be bf16 or fp16");
@@ -203,10 +205,12 @@ extern "C" int forge_linear_small(int dtype, int M, int N, int K, const void* x,
   if (!x || !w || !out) return set_error("null tensor pointer");
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)w2 | (uintptr_t)gain) % 16)
     return set_error("forge_linear_small: x, the weights and the gain must be 16-byte aligned");
+  if (gain && gain_dtype != FORGE_F32 && gain_dtype != dtype)
+    return set_error("forge_linear_small: the gain must be fp32 or of x's type");
   if (sx % 8 || sw % 8 || sw < K || (M > 1 && sx < K))
     return set_error("forge_linear_small: row strides must be multiples of 8 elements and hold a row");
   if (w2 && (bias || residual)) return set_error("forge_linear_small: SwiGLU takes no bias or residual");
-  LinearParams p{x, sx, w, w2, sw, bias, gain, norm, eps, residual, sr, out, so, M, N, K};
+  LinearParams p{x, sx, w, w2, sw, bias, gain, gain_dtype == FORGE_F32, norm, eps, residual, sr, out, so, M, N, K};
   hipStream_t s = (hipStream_t)stream;
   return dtype == FORGE_BF16 ? launch_linear<bf16>(p, s) : launch_linear<f16>(p, s);
 }

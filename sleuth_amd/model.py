@@ -68,7 +68,7 @@ class Block(nn.Module):
         if self._small_step(x):
             x = self.attn._layer(x, cos, sin, cache, same_doc, norm=self.norm1, residual=x)
             m, n = self.mlp, self.norm2
-            h = ops.linear_small(x, m.gate.weight, w_up=m.up.weight, gain=n.weight_f32(), eps=n.eps, norm=True)
+            h = ops.linear_small(x, m.gate.weight, w_up=m.up.weight, gain=n.weight, eps=n.eps, norm=True)
             if h is None:
                 return x + m(n(x))
             y = ops.linear_small(h, m.down.weight, m.down.bias, residual=x)
@@ -173,7 +173,7 @@ class Transformer(nn.Module):
         if x.numel() <= ops.LINEAR_SMALL_ROWS * x.shape[-1] and x.is_cuda and not return_hidden and \
                 not torch.is_grad_enabled() and not hip_disabled() and no_global_hooks() and \
                 plain_module(n, RMSNorm) and plain_module(head, nn.Linear):
-            y = ops.linear_small(x, head.weight, head.bias, gain=n.weight_f32(), eps=n.eps, norm=True)
+            y = ops.linear_small(x, head.weight, head.bias, gain=n.weight, eps=n.eps, norm=True)
             if y is not None:
                 return ModelOutput(y)
         h = n(x)

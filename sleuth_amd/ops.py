@@ -483,12 +483,13 @@ def linear_small(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = N
                  w_up: torch.Tensor | None = None, gain: torch.Tensor | None = None, eps: float = 0.0,
                  norm: bool = False, residual: torch.Tensor | None = None) -> torch.Tensor | None:
     """F.linear(x, w, bias) of a decode or verify step (forge_linear_small), without autograd;
-    norm: x gets RMSNorm (gain fp32 [K]) first; w_up: silu(x . w^T) * (x . w_up^T); residual [..., N]:
+    norm: x gets RMSNorm (gain [K], fp32 or of x's type) first; w_up: silu(x . w^T) * (x . w_up^T); residual [..., N]:
     added to the result. None where the call is not of the kernel's form (the caller then makes
     the torch calls): it takes bf16/fp16 on one GPU, x [..., K] of at most 16 rows, K a multiple of
-    32, everything contiguous and 16-byte aligned, and nothing (autocast, tracing, a tensor
-    subclass) between the call and the memory."""
-    if torch.is_autocast_enabled() or torch.compiler.is_compiling():
+    32, everything contiguous and 16-byte aligned, and nothing (autocast, tracing, a dispatch or
+    function mode, a tensor subclass, a forward-mode tangent) between the call and the memory."""
+    if torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or \
+            torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack():
         return None
     r = host().linear_small(x, w, bias, w_up, gain, float(eps), bool(norm), residual)
     return r if r.__class__ is not int else check(r, "forge_linear_small")

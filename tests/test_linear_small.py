@@ -18,11 +18,12 @@ needs_gpu = pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
 def test_rejections():
     lib = _lib.lib()
 
-    def call(dtype=_lib.BF16, M=1, N=16, K=64, x=4096, sx=64, w=4096, w2=None, sw=64, bias=None, out=None):
-        return lib.forge_linear_small(dtype, M, N, K, x, sx, w, w2, sw, bias, None, 0, 0.0, None, 0, out, N, None)
+    def call(dtype=_lib.BF16, M=1, N=16, K=64, x=4096, sx=64, w=4096, w2=None, sw=64, bias=None, gain=None, gd=0, out=None):
+        return lib.forge_linear_small(dtype, M, N, K, x, sx, w, w2, sw, bias, gain, gd, 0, 0.0, None, 0, out, N, None)
 
     for kw in (dict(), dict(dtype=_lib.F32), dict(M=17), dict(M=0), dict(K=48), dict(x=4098), dict(sw=60), dict(M=2, sx=56),
-               dict(w2=4096, bias=4096)):
+               dict(w2=4096, bias=4096),
+               dict(gain=4096, gd=_lib.F16)):
         assert call(**{"out": 4096 if kw else None, **kw}) < 0
 
 
@@ -64,8 +65,41 @@ def test_linear_small(dtype, M, N, K, form):
     inner = {"plain": 0, "bias": 0, "norm": 1, "norm+residual": 2, "swiglu": 3, "norm+swiglu": 4}[form]
     err = (got.cpu().double() - y).norm() / y.norm()
     assert err.item() <= ulp * (1 + 2 * inner)
+    if "norm" in form:                        # a gain of x's type, read as it is
+        low = d(gain).to(dtype)
+        assert torch.equal(call(slice(None), gain=low), call(slice(None), gain=low.float()))
     one = call(slice(M - 1, M), residual=d(res)[M - 1:] if "residual" in form else None)
     assert torch.equal(one, got[M - 1:])      # a row does not depend on the others
+
+
+@pytest.mark.gpu
+@needs_gpu
+def test_declines_what_stands_between_the_call_and_the_memory():
+    """Forward-mode tangents, tensor subclasses, tracing, function and dispatch modes: torch's own call."""
+    import torch.autograd.forward_ad as fwd
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from sleuth_amd import ops
+
+    class Sub(torch.nn.Parameter):
+        pass
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x, w = torch.ones(1, 64, dtype=torch.bfloat16, device=DEV), torch.ones(16, 64, dtype=torch.bfloat16, device=DEV)
+    with torch.no_grad():
+        assert ops.linear_small(x, w) is not None and ops.linear_small(x, torch.nn.Parameter(w)) is not None
+        assert ops.linear_small(x, Sub(w)) is None
+        with fwd.dual_level():
+            assert ops.linear_small(fwd.make_dual(x, x), w) is None
+            assert ops.linear_small(x, fwd.make_dual(w, w)) is None
+        for mode in (Mode(), torch.overrides.BaseTorchFunctionMode()):
+            with mode:
+                assert ops.linear_small(x, w) is None
+        seen = []
+        torch.jit.trace(lambda t: seen.append(ops.linear_small(t, w)) or t + 1, x, check_trace=False)
+        assert seen == [None]
 
 
 def _model(**kw):
@@ -122,3 +156,34 @@ def test_block_step_and_what_turns_its_fusion_off(T, monkeypatch):
     calls.clear()
     m(ids).logits.sum().backward()               # autograd: none
     assert not calls and m.blocks[0].mlp.down.weight.grad is not None
+
+
+@pytest.mark.gpu
+@needs_gpu
+def test_recorded_step_reads_the_norm_gains_live():
+    """A recorded step multiplies by the norms' parameters themselves: gains changed in place between
+    replays count at once, and no copy of them is freed under the graph."""
+    from sleuth_amd.generate import GraphDecoder
+    from sleuth_amd.kv_cache import KVCache
+
+    m = _model()
+    prompt, ids = torch.randint(0, 128, (1, 40), device=DEV), torch.randint(0, 128, (1,), device=DEV)
+    dec = GraphDecoder(m, 64, torch.bfloat16)
+
+    @torch.no_grad()
+    def both():
+        dec.cache.reset()
+        m(prompt, cache=dec.cache)
+        got = dec.step(ids).clone()
+        cache = KVCache.for_model(m, 1)
+        m(prompt, cache=cache)
+        want = m(ids[None], cache=cache).logits[0]
+        return got.float(), want.float()
+
+    both()
+    for scale in (0.5, 3.0):
+        with torch.no_grad():
+            for n in (m.blocks[0].norm1, m.blocks[1].norm2, m.norm_f):
+                n.weight.copy_(torch.linspace(0.5, 1.5, n.weight.numel(), device=DEV) * scale)
+        got, want = both()
+        assert ((got - want).norm() / want.norm()).item() <= 0.03   # two layers of bf16 roundings
