@@ -7,16 +7,24 @@
 // A step of a layer is a chain of such calls, so launches and their gaps cost as much as the
 // streams, hence the fused neighbours.
 //
-// Split. A block of 8 waves takes 16 output columns; the waves take slices of K, all their W
-// loads (16 bytes per lane, up to kAhead k-steps) in flight before anything else, and add their
-// tiles through LDS in wave order. On v_mfma_f32_16x16x32 the 16 W rows are the A operand and the
-// (up to 16) x rows the B operand, both straight from memory in operand layout, so the same kernel
-// serves 1 to 16 rows at the cost of one. A row's result does not depend on the other rows.
-// Measured against hipBLASLt (bf16, graph replays of the call alone, one box), N x K at 1 / 5 / 16
-// rows: 4096 x 1024: 5.1 / 5.1 / 5.5 us against 6.3; 1024 x 2048: 5.0 / 5.1 / 5.9 against 8.2; 1024 x
-// 3072: 7.5 / 7.6 / 8.8 against 9.4; 8192 x 1024: 7.0 / 7.2 / 8.1 against 6.7; 32768 x 4096: 51 / 53 /
-// 74 against 62. A four-layer model's decode step (d 1024, hidden 3072; GraphDecoder) with the norms,
-// residual sums and SwiGLU product in these launches (and the RoPE rows converted once per pass): 416 -> 207 us.
+// Split. A block of 8 waves takes 16 output columns; the waves take slices of K and add their tiles
+// through LDS in wave order. On v_mfma_f32_16x16x32 the 16 W rows are the A operand and the (up to
+// 16) x rows the B operand, both straight from memory in operand layout, so the same kernel serves 1
+// to 16 rows. A row's result does not depend on the other rows. Every load of a slice (x, the gain,
+// W; A k-steps of them) goes out before anything is computed, and a slot's next load as soon as the
+// slot is used. The RMSNorm sums the squares of the slices that the products read, so x is read
+// once and the norm adds one barrier: a pass over x of its own, with W's loads only in flight, took
+// 1.3 us more at K 1,024 (5.2 us against 3.9 without the norm; now 3.7 against 2.7).
+//
+// Measured (bf16, graph replays of the call alone, 1 / 5 / 16 rows, us; in brackets the form before,
+// one box each): 4096 x 1024 with norm 3.7 / 3.9 / 4.4 (5.2 / 5.4 / 6.2), hipBLASLt's product alone
+// 6.3; 1024 x 2048 with residual 3.8 / 4.1 / 5.2 (4.3 / 4.4 / 5.2), hipBLASLt 8.2; 3072 x 1024 SwiGLU
+// with norm 4.7 / 4.9 / 5.4 (6.9 / 7.3 / 8.2); 1024 x 3072 with residual 4.9 / 5.4 / 6.9 (6.4 / 6.7 /
+// 7.8), hipBLASLt 9.4; 8192 x 1024 with norm 5.0 / 5.3 / 6.2 (7.1 / 7.4 / 8.8), hipBLASLt 6.7; 4096 x
+// 14336 with residual 19.6 / 20.9 / 26.7 (27.4 / 29.1 / 32.5; 6.0 TB/s at one row); 32768 x 4096 with norm
+// 55 / 55 / 68 (60 / 63 / 83), hipBLASLt 62; 6144 x 4096 with norm 16.1 / 18.3 / 25.1 (17.0 / 17.8 / 23.5).
+// A four-layer model's decode step (d 1024, hidden 3072; GraphDecoder), with the norms, residual sums
+// and SwiGLU product in these launches: 175 us (206 the form before, 411 with torch's calls).
 #include "common.h"
 #include "forge_internal.h"
 
@@ -47,7 +55,7 @@ struct LinearParams {
   const void* w2;  // SwiGLU: w is the gate, w2 the up projection
   int64_t sw;
   const void* bias;
-  const void* gain;  // RMSNorm of x (norm != 0), or null; fp32 or of x's type, as the module holds it
+  const void* gain;  // RMSNorm of x (norm != 0): fp32 or of x's type, as the module holds it
   int gain_f32;
   int norm;
   float eps;
@@ -60,15 +68,26 @@ struct LinearParams {
 
 constexpr int kLinWaves = 8;
 constexpr int kLinRows = 16;   // rows of x
-constexpr int kLinCols = 16;   // output columns per block
-constexpr int kAhead = 8;      // k-steps whose W loads are in flight
+constexpr int kLinCols = 16;   // output columns of a tile
+// Outputs from which a block takes two tiles: x's rows are then read half as often, and two blocks per
+// CU are left. 32768 x 4096 with norm at 5 rows 54 us against 63 with one tile, at 16 rows 66 against 83.
+constexpr int kLinWideN = 16384;
 
-template <typename T, bool GATED>
-__global__ __launch_bounds__(64 * kLinWaves)
+// What the kernel does to x's rows first.
+enum LinNorm { kLinPlain, kLinGain, kLinGainF32 };  // nothing; RMSNorm with a gain of x's type; with an fp32 gain
+
+// Unpack the register here, not earlier: the floats of all the k-steps in flight would cost a CU its
+// second block.
+__device__ __forceinline__ void keep_packed(uint4& u) { asm volatile("" : "+v"(u.x), "+v"(u.y), "+v"(u.z), "+v"(u.w)); }
+
+// TILES: tiles of 16 output columns per block; GATED: each of them twice (gate and up); A: k-steps
+// whose loads are in flight.
+template <typename T, bool GATED, int TILES, int NORM, int A>
+__global__ __launch_bounds__(64 * kLinWaves) __attribute__((amdgpu_waves_per_eu(4)))
 void linear_small_kernel(LinearParams p) {
   using V8 = typename LMfma<T>::vec;
-  constexpr int NT = GATED ? 2 : 1;  // tiles per wave
-  __shared__ float sh_rs[kLinRows];
+  constexpr int NT = GATED ? 2 * TILES : TILES;  // MFMA tiles per wave
+  __shared__ float sh_ss[kLinWaves][kLinRows];
   __shared__ float sh_acc[kLinWaves][NT][kLinCols * kLinRows];
 
   const int tid = threadIdx.x;
@@ -76,81 +95,104 @@ void linear_small_kernel(LinearParams p) {
   const int lane = tid % kWave;
   const int r = lane & 15;  // W row of the tile (A operand), x row (B operand)
   const int g = lane >> 4;  // channels 32 s + 8 g .. + 7 of k-step s
-  const int n0 = blockIdx.x * kLinCols;
-  const int n = n0 + r < p.N ? n0 + r : p.N - 1;  // columns past N repeat the last one, not written
+  const int n0 = blockIdx.x * (kLinCols * TILES);
 
   // this wave's k-steps
   const int steps = p.K / 32;
   const int s_lo = (int)((int64_t)steps * wave / kLinWaves), s_hi = (int)((int64_t)steps * (wave + 1) / kLinWaves);
   const T* wp[NT];
-  wp[0] = static_cast<const T*>(p.w) + n * p.sw + 8 * g;
-  if constexpr (GATED) wp[1] = static_cast<const T*>(p.w2) + n * p.sw + 8 * g;
-  uint4 wr[NT][kAhead];
-  auto load_w = [&](int s0) {
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      const int s = s0 + i < s_hi ? s0 + i : s_hi - 1;  // (a wave with no step skips the loop)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) wr[t][i] = load16(wp[t] + 32 * s);
-    }
+  for (int t = 0; t < NT; ++t) {
+    const int c = n0 + kLinCols * (t % TILES) + r;
+    const int n = c < p.N ? c : p.N - 1;  // columns past N repeat the last one, not written
+    wp[t] = static_cast<const T*>(t < TILES ? p.w : p.w2) + n * p.sw + 8 * g;
+  }
+  // x through a buffer resource: the lanes of rows past M read zeros without an access
+  const __amdgpu_buffer_rsrc_t xs = slab_rsrc(p.x, (unsigned)(((p.M - 1) * p.sx + p.K) * sizeof(T)));
+  const unsigned x_off = r < p.M ? (unsigned)((r * p.sx + 8 * g) * sizeof(T)) : 0x80000000u;
+  auto load_x = [&](int s) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(xs, (int)(x_off + 64 * s), 0, 0));
   };
-  if (s_lo < s_hi) load_w(s_lo);
+  const T* gp = static_cast<const T*>(p.gain) + 8 * g;
+  uint4 wr[NT][A], xr[A], gr[NORM == kLinGain ? A : 1];
+  auto load = [&](int i, int s) {  // k-step s (the last one's again where the wave has fewer) into slot i
+    const int last = s < s_hi ? s : s_hi - 1, at = 32 * last;
+    xr[i] = load_x(last);
+    if constexpr (NORM == kLinGain) gr[i] = load16(gp + at);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wr[t][i] = load16(wp[t] + at);
+  };
+  if (s_lo < s_hi) {  // wave-uniform; a wave with no step contributes zeros
+#pragma unroll
+    for (int i = 0; i < A; ++i) load(i, s_lo + i);
+  }
 
-  const bool row = r < p.M;
-  const T* xp = static_cast<const T*>(p.x) + (row ? r : 0) * p.sx + 8 * g;
   float rs = 1.0f;
-  if (p.norm) {  // RMSNorm factors of the rows: wave w takes rows w and w + 8
+  if constexpr (NORM != kLinPlain) {
+    // RMSNorm factors of the rows: each wave sums the squares of its slice, from the registers that
+    // the products read as far as those reach
+    float ss = 0.0f;
+    auto square = [&](uint4 raw) {
+      float v[8];
+      unpack16<T>(raw, v);
 #pragma unroll
-    for (int j = 0; j < kLinRows / kLinWaves; ++j) {
-      const int m = wave + kLinWaves * j;
-      if (m < p.M) {
-        const T* xr = static_cast<const T*>(p.x) + m * p.sx;
-        float ss = 0.0f;
-        for (int k = 8 * lane; k < p.K; k += 8 * kWave) {
-          float v[8];
-          unpack16<T>(load16(xr + k), v);
+      for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+    };
 #pragma unroll
-          for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
-        }
-        ss = group_sum<kWave>(ss);
-        if (lane == 0) sh_rs[m] = rsqrtf(ss / (float)p.K + p.eps);
+    for (int i = 0; i < A; ++i)
+      if (s_lo + i < s_hi) {  // wave-uniform
+        square(xr[i]);
+        keep_packed(xr[i]);
       }
+    for (int s = s_lo + A; s < s_hi; s += 4) {
+      uint4 more[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) more[i] = load_x(s + i < s_hi ? s + i : s_hi - 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (s + i < s_hi) square(more[i]);
     }
+    ss += __shfl_xor(ss, 16);
+    ss += __shfl_xor(ss, 32);
+    if (g == 0) sh_ss[wave][r] = ss;
     __syncthreads();
-    rs = row ? sh_rs[r] : 0.0f;
+    float all = sh_ss[0][r];
+#pragma unroll
+    for (int w = 1; w < kLinWaves; ++w) all += sh_ss[w][r];
+    rs = rsqrtf(all / (float)p.K + p.eps);
   }
 
   l_floatx4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = l_floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int s0 = s_lo; s0 < s_hi; s0 += kAhead) {
+  auto multiply = [&](int i, int s) {
+    uint4 xv = xr[i];
+    if constexpr (NORM != kLinPlain) {
+      float v[8], w[8];
+      unpack16<T>(xv, v);
+      if constexpr (NORM == kLinGain) {
+        keep_packed(gr[i]);
+        unpack16<T>(gr[i], w);
+      } else load_f32x8(static_cast<const float*>(p.gain) + 32 * s + 8 * g, w);
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) {
-      const int s = s0 + i;
-      if (s < s_hi) {  // wave-uniform
-        uint4 xr = make_uint4(0, 0, 0, 0);
-        if (row) xr = load16(xp + 32 * s);
-        if (p.norm) {
-          float v[8];
-          unpack16<T>(xr, v);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] *= rs;
-          if (p.gain) {
-            float w[8];
-            if (p.gain_f32) load_f32x8(static_cast<const float*>(p.gain) + 32 * s + 8 * g, w);
-            else unpack16<T>(load16(static_cast<const T*>(p.gain) + 32 * s + 8 * g), w);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] *= w[e];
-          }
-          xr = pack16<T>(v);
-        }
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          acc[t] = LMfma<T>::run(__builtin_bit_cast(V8, wr[t][i]), __builtin_bit_cast(V8, xr), acc[t]);
-      }
+      for (int e = 0; e < 8; ++e) v[e] = v[e] * rs * w[e];
+      xv = pack16<T>(v);
     }
-    if (s0 + kAhead < s_hi) load_w(s0 + kAhead);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      acc[t] = LMfma<T>::run(__builtin_bit_cast(V8, wr[t][i]), __builtin_bit_cast(V8, xv), acc[t]);
+  };
+  int s0 = s_lo;
+  for (; s0 + A < s_hi; s0 += A) {  // each slot's next loads go out as soon as it is used
+#pragma unroll
+    for (int i = 0; i < A; ++i) {
+      multiply(i, s0 + i);
+      load(i, s0 + A + i);
+    }
   }
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+    if (s0 + i < s_hi) multiply(i, s0 + i);  // wave-uniform
 
   // tile element (column 4 g + j of the block, x row r) of every wave, added in wave order
 #pragma unroll
@@ -158,15 +200,16 @@ void linear_small_kernel(LinearParams p) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) sh_acc[wave][t][r * kLinCols + 4 * g + j] = acc[t][j];
   __syncthreads();
-  if (tid >= kLinCols * kLinRows) return;
-  const int m = tid / kLinCols, c = n0 + tid % kLinCols;
+  if (tid >= TILES * kLinCols * kLinRows) return;
+  const int tile = tid / (kLinCols * kLinRows), in = tid % (kLinCols * kLinRows);
+  const int m = in / kLinCols, c = n0 + tile * kLinCols + in % kLinCols;
   if (m >= p.M || c >= p.N) return;
-  float v[NT];
+  float v[GATED ? 2 : 1];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    v[t] = sh_acc[0][t][tid];
+  for (int t = 0; t < (GATED ? 2 : 1); ++t) {
+    v[t] = sh_acc[0][t * TILES + tile][in];
 #pragma unroll
-    for (int w = 1; w < kLinWaves; ++w) v[t] += sh_acc[w][t][tid];
+    for (int w = 1; w < kLinWaves; ++w) v[t] += sh_acc[w][t * TILES + tile][in];
   }
   float y = v[0];
   if (p.bias) y += to_f32<T>(static_cast<const T*>(p.bias)[c]);
@@ -182,11 +225,34 @@ void linear_small_kernel(LinearParams p) {
   static_cast<T*>(p.out)[m * p.so + c] = from_f32<T>(y);
 }
 
+template <typename T, bool GATED, int TILES, int A>
+static void launch_plain(const LinearParams& p, dim3 grid, hipStream_t s) {
+  hipLaunchKernelGGL((linear_small_kernel<T, GATED, TILES, kLinPlain, A>), grid, dim3(64 * kLinWaves), 0, s, p);
+}
+
+template <typename T, bool GATED, int TILES>
+static void launch_tiles(const LinearParams& p, hipStream_t s) {
+  const dim3 grid((unsigned)((p.N + kLinCols * TILES - 1) / (kLinCols * TILES))), block(64 * kLinWaves);
+  if (p.norm) {
+    if (p.gain_f32) hipLaunchKernelGGL((linear_small_kernel<T, GATED, TILES, kLinGainF32, 4>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((linear_small_kernel<T, GATED, TILES, kLinGain, 4>), grid, block, 0, s, p);
+    return;
+  }
+  // k-steps in flight: all of a wave's where 12 or fewer. A slot without a step repeats the last one's
+  // loads, so slots fit the steps: 12 slots for 4 steps, and x's rows past M read as row 0, took 4.6 us
+  // at 4096 x 1024; 4 slots and no such reads 2.7 us. Kernels with a norm or two tiles have 4 slots:
+  // 8 need up to 229 registers, which leaves one block per CU.
+  const int steps = (p.K / 32 + kLinWaves - 1) / kLinWaves;  // of a wave
+  if (GATED || TILES > 1 || steps <= 4) launch_plain<T, GATED, TILES, 4>(p, grid, s);
+  else if (steps > 8 && steps <= 12) launch_plain<T, false, 1, 12>(p, grid, s);
+  else launch_plain<T, false, 1, 8>(p, grid, s);
+}
+
 template <typename T>
 static int launch_linear(const LinearParams& p, hipStream_t s) {
-  const dim3 grid((unsigned)((p.N + kLinCols - 1) / kLinCols));
-  if (p.w2) hipLaunchKernelGGL((linear_small_kernel<T, true>), grid, dim3(64 * kLinWaves), 0, s, p);
-  else hipLaunchKernelGGL((linear_small_kernel<T, false>), grid, dim3(64 * kLinWaves), 0, s, p);
+  if (p.w2) launch_tiles<T, true, 1>(p, s);
+  else if (p.N >= kLinWideN) launch_tiles<T, false, 2>(p, s);
+  else launch_tiles<T, false, 1>(p, s);
   return check_launch();
 }
 
@@ -205,10 +271,13 @@ extern "C" int forge_linear_small(int dtype, int M, int N, int K, const void* x,
   if (!x || !w || !out) return set_error("null tensor pointer");
   if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)w2 | (uintptr_t)gain) % 16)
     return set_error("forge_linear_small: x, the weights and the gain must be 16-byte aligned");
+  if (norm && !gain) return set_error("forge_linear_small: norm needs a gain");
   if (gain && gain_dtype != FORGE_F32 && gain_dtype != dtype)
     return set_error("forge_linear_small: the gain must be fp32 or of x's type");
   if (sx % 8 || sw % 8 || sw < K || (M > 1 && sx < K))
     return set_error("forge_linear_small: row strides must be multiples of 8 elements and hold a row");
+  if (M > 1 && sx > (1 << 25)) return set_error("forge_linear_small: rows of x more than 2^25 elements apart");
+  if (K > (1 << 25)) return set_error("forge_linear_small: K of more than 2^25");
   if (w2 && (bias || residual)) return set_error("forge_linear_small: SwiGLU takes no bias or residual");
   LinearParams p{x, sx, w, w2, sw, bias, gain, gain_dtype == FORGE_F32, norm, eps, residual, sr, out, so, M, N, K};
   hipStream_t s = (hipStream_t)stream;

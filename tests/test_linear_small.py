@@ -31,7 +31,7 @@ def test_rejections():
 @needs_gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 5, 16])
-@pytest.mark.parametrize("N,K", [(1, 32), (17, 96), (100, 1024), (256, 3104)])
+@pytest.mark.parametrize("N,K", [(1, 32), (17, 96), (100, 1024), (40, 2048), (40, 3072), (256, 3104), (16403, 64), (16384, 288)])
 @pytest.mark.parametrize("form", ["plain", "bias", "norm", "norm+residual", "swiglu", "norm+swiglu"])
 def test_linear_small(dtype, M, N, K, form):
     from sleuth_amd import ops
