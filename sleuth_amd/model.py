@@ -22,7 +22,7 @@ from .attention import Attention, hip_disabled, no_global_hooks, plain_module
 from .config import ModelConfig
 from .norm import RMSNorm
 from .rope import rope_tables
-from .taps import make_tap, name_taps, tap_active
+from .taps import make_tap, name_taps, tap_active, tap_class
 
 
 class SwiGLU(nn.Module):
@@ -59,10 +59,9 @@ class Block(nn.Module):
                 plain_module(self.attn, Attention) and plain_module(m, SwiGLU) and plain_module(m.gate, nn.Linear) and
                 plain_module(m.up, nn.Linear) and plain_module(m.down, nn.Linear)):
             return False
-        if tap_active(self.tap_attn_out) or tap_active(self.tap_resid_post) or m.gate.bias is not None or \
-                m.up.bias is not None:
+        if any(tap_active(t) or not plain_module(t, tap_class()) for t in (self.tap_attn_out, self.tap_resid_post)):
             return False
-        return True
+        return m.gate.bias is None and m.up.bias is None
 
     def forward(self, x, cos, sin, cache=None, same_doc=None):
         if self._small_step(x):

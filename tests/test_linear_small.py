@@ -3,6 +3,8 @@ eager layers' roundings, and the block's use of it."""
 
 from __future__ import annotations
 
+import types
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -112,6 +114,37 @@ def _model(**kw):
     return Transformer(cfg).to(DEV, torch.bfloat16).eval()
 
 
+def _block_and_step():
+    """A block on the CPU, and a stand-in for the one GPU row that its dispatch looks at."""
+    from sleuth_amd.config import ModelConfig
+    from sleuth_amd.model import Block
+
+    cfg = ModelConfig(vocab_size=16, d_model=64, n_layers=1, n_heads=2, n_kv_heads=1, max_seq_len=32, ffn_hidden=64)
+    return Block(cfg, 0), types.SimpleNamespace(numel=lambda: 64, shape=(1, 1, 64), is_cuda=True)
+
+
+@torch.no_grad()
+def test_what_stands_in_for_a_tap_turns_the_fused_step_off():
+    blk, x = _block_and_step()
+    assert blk._small_step(x)
+    for name in ("tap_attn_out", "tap_resid_post"):
+        tap = getattr(blk, name)
+        for register in (tap.register_forward_hook, tap.register_forward_pre_hook):
+            h = register(lambda *a: None)
+            assert not blk._small_step(x)
+            h.remove()
+        tap.listeners.append(lambda name, t: None)
+        assert not blk._small_step(x)
+        tap.listeners.clear()
+        tap.forward = lambda t: 2 * t
+        assert not blk._small_step(x)
+        del tap.forward
+        setattr(blk, name, torch.nn.Dropout(0.5))
+        assert not blk._small_step(x)
+        setattr(blk, name, tap)
+        assert blk._small_step(x)
+
+
 @pytest.mark.gpu
 @needs_gpu
 @pytest.mark.parametrize("T", [1, 5])
@@ -150,6 +183,15 @@ def test_block_step_and_what_turns_its_fusion_off(T, monkeypatch):
     h.remove()
     with listen(m, {"blocks.0.resid_post": lambda name, x: seen.append(1)}):
         same(5 + 2)
+    for name in ("tap_attn_out", "tap_resid_post"):
+        seen.clear()
+        h = getattr(blk, name).register_forward_hook(lambda mod, a, out: seen.append(out.shape))
+        same(5 + 2)
+        assert len(seen) == 2                    # the prompt and the step
+        h.remove()
+    tap, blk.tap_attn_out = blk.tap_attn_out, torch.nn.Identity()
+    same(5 + 2)
+    blk.tap_attn_out = tap
     blk.mlp.forward = type(blk.mlp).forward.__get__(blk.mlp)
     same(5 + 2)
     del blk.mlp.forward
