@@ -35,6 +35,7 @@ from __future__ import annotations
 
 import math
 import os
+import sys
 import weakref
 
 import torch
@@ -160,8 +161,16 @@ def fused_qkv_entry(weight: torch.Tensor) -> "_FusedQKV | None":
 
 def plain_module(m: nn.Module, cls: type) -> bool:
     """m is exactly a `cls` that runs its own forward: no subclass, no forward hooks, nothing put
-    in place of forward. Only such modules' work may be done inside a fused launch."""
-    return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__
+    in place of forward on the module or its class, no module.compile(), and nn.Module's own call.
+    Only such modules' work may be done inside a fused launch."""
+    return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__ and \
+        m._compiled_call_impl is None and _defined_in(cls.forward, cls.__module__) and \
+        _defined_in(cls.__call__, nn.Module.__module__) and _defined_in(cls._call_impl, nn.Module.__module__)
+
+
+def _defined_in(fn, module: str) -> bool:
+    """fn is a function written in that module (what a replacement, wrapped or not, is not)."""
+    return getattr(fn, "__globals__", None) is sys.modules[module].__dict__
 
 
 def no_global_hooks() -> bool:

@@ -145,6 +145,34 @@ def test_what_stands_in_for_a_tap_turns_the_fused_step_off():
         assert blk._small_step(x)
 
 
+@torch.no_grad()
+def test_what_stands_in_for_a_class_turns_the_fused_step_off(monkeypatch):
+    import functools
+
+    from sleuth_amd.attention import Attention
+    from sleuth_amd.model import SwiGLU
+    from sleuth_amd.norm import RMSNorm
+
+    blk, x = _block_and_step()
+    for cls in (Attention, SwiGLU, RMSNorm, torch.nn.Linear, type(blk.tap_attn_out)):
+        own = cls.forward
+        for other in (lambda self, *a, **kw: None, functools.wraps(own)(lambda self, *a, **kw: own(self, *a, **kw)),
+                      functools.partialmethod(own)):
+            with monkeypatch.context() as m:
+                m.setattr(cls, "forward", other)
+                assert not blk._small_step(x), cls
+    for name in ("__call__", "_call_impl"):
+        with monkeypatch.context() as m:
+            m.setattr(torch.nn.Module, name, lambda self, *a, **kw: None)
+            assert not blk._small_step(x)
+    assert blk._small_step(x)
+    for part in (blk.attn, blk.mlp, blk.norm1, blk.mlp.down):
+        part.compile()
+        assert not blk._small_step(x)
+        part._compiled_call_impl = None
+    assert blk._small_step(x)
+
+
 @pytest.mark.gpu
 @needs_gpu
 @pytest.mark.parametrize("T", [1, 5])
