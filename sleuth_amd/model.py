@@ -160,9 +160,10 @@ class Transformer(nn.Module):
             raise ValueError(f"sequence length {offset + T} exceeds max_seq_len {self.cfg.max_seq_len}")
         if getattr(cache, "static", False):
             cache.new_step()
-        # (fp32 rows, made once per pass: a model cast to bf16 holds its tables in bf16, and every layer
-        # would convert the same rows)
-        rope = {k: (c.float(), s.float()) for k, (c, s) in self.rope_rows(offset, T, cache).items()}
+        # (fp32 rows of 16-bit tables, made once per pass: a model cast to bf16 holds its tables in bf16,
+        # and every layer would convert the same rows)
+        rope = {k: (c.float(), s.float()) if c.element_size() < 4 else (c, s)
+                for k, (c, s) in self.rope_rows(offset, T, cache).items()}
         x = self.tok_emb(idx)
         for block in self.blocks:
             x = block(x, *rope[block.kind], cache)

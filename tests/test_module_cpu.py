@@ -429,3 +429,20 @@ def test_gated_attention_torch_path_matches_oracle():
             vp = vn if vp is None else torch.cat([vp, vn], 2)
             torch.testing.assert_close(got, m.o_proj(y), atol=1e-5, rtol=1e-4)
     assert m.last_path == "torch"
+
+
+@pytest.mark.parametrize("model,rows", [(torch.float64, torch.float64), (torch.float32, torch.float32),
+                                        (torch.bfloat16, torch.float32)])
+def test_rope_rows_keep_their_precision(model, rows):
+    """The blocks get 16-bit tables as fp32 rows (the same values), and wider ones as they are: in a
+    float64 model the rotation is computed in float64."""
+    m = make().to(model)
+    seen = []
+    for b in m.blocks:
+        b.register_forward_pre_hook(lambda mod, a: seen.append((a[1], a[2])))
+    with torch.no_grad():
+        m(torch.arange(7)[None])
+    assert len(seen) == 3
+    for c, s in seen:
+        assert c.dtype == s.dtype == rows
+        assert torch.equal(c, m.rope_cos_full[:7].to(rows)) and torch.equal(s, m.rope_sin_full[:7].to(rows))
