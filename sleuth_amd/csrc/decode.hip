@@ -2574,7 +2574,7 @@ int decode_setup(SplitParams& p, int dtype, int B, int T, int H, int K, int D, c
   if (sks * (max_len + 1) * esize >= (1LL << 31))
     return set_error("forge_attn_decode: one (batch, kv head) slab of the cache must span < 2^31 bytes");
   if (max_kv_len <= 0 || max_kv_len > max_len) max_kv_len = max_len;
-  if (!row_pos && !pos_dev && (pos0 < 0 || pos0 + T > max_len))
+  if (!row_pos && !pos_dev && (pos0 < 0 || pos0 > max_len - T))
     return set_error("KV cache full: pos + T exceeds the cache length");
   if (!row_pos && !pos_dev && pos0 + T > max_kv_len) max_kv_len = pos0 + T;
   if (window < 0) return set_error("window must be >= 0");

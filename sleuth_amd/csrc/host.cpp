@@ -166,6 +166,7 @@ PyObject* decode_append_impl(PyObject* const* a) {
   }
   Rope r;
   if (!rope_ok(cos, sin, B, T, D, dev, r) || !gain_ok(qw, D, dev) || !gain_ok(kw, D, dev)) return nullptr;
+  if (pos < 0 || pos > max_len) return nullptr;
   if (max_kv < 0) max_kv = !row_pos.defined() && !pos_dev.defined() ? pos + T : max_len;
   max_kv = std::max<int64_t>(1, std::min(max_kv, max_len));
   if (window < 0 || window > INT_MAX || chunk > INT_MAX || c10::hip::current_device() != dev.index()) return nullptr;
@@ -238,7 +239,7 @@ PyObject* prefill_impl(PyObject* const* a) {
   const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3), K = k.size(1);
   const int dt = dtype_of(q);
   const c10::Device dev = q.device();
-  if (dt < 0 || K <= 0 || H % K || k.size(0) != B || k.size(3) != D || offset < 0 || k.size(2) < offset + T ||
+  if (dt < 0 || K <= 0 || H % K || k.size(0) != B || k.size(3) != D || offset < 0 || k.size(2) - T < offset ||
       window < 0 || window > INT_MAX || q.stride(3) != 1 || c10::hip::current_device() != dev.index())
     return nullptr;
   for (const Tensor* t : {&k, &v})

@@ -1430,6 +1430,9 @@ static int launch_prefill(const PrefillParams& p, int D, hipStream_t s) {
 
 using namespace forge;
 
+// Positions up to a tile past the last one fit in 31 bits (without a sum that could wrap).
+static bool positions_fit(int64_t offset, int T) { return offset < (1LL << 31) - 256 - (int64_t)T; }
+
 // fp32 (m, l) pairs and partial outputs of every part of every row
 static size_t prefill_workspace(const PrefillPlan& plan, int B, int T, int H, int D) {
   const size_t slots = (size_t)plan.nsplit * B * H * T;
@@ -1454,7 +1457,7 @@ static int prefill_setup(PrefillParams& p, int esize, int B, int T, int H, int K
   if ((sqb | sqh | sqt | skb | skh | sks) % (16 / esize))
     return set_error("forge_attn_prefill: q/k/v strides must be multiples of 16 bytes");
   if ((sob | sot | soh) % 4) return set_error("forge_attn_prefill: out strides must be multiples of 4");
-  if (offset + (int64_t)T + 256 >= (1LL << 31)) return set_error("forge_attn_prefill: positions must fit in 31 bits");
+  if (!positions_fit(offset, T)) return set_error("forge_attn_prefill: positions must fit in 31 bits");
   if (sks * esize * 256 >= (1LL << 31)) return set_error("forge_attn_prefill: k/v row stride too large");
   if (((uintptr_t)q_weight | (uintptr_t)cos | (uintptr_t)sin) % 16 || (cos && s_cos_t % 4))
     return set_error("forge_attn_prefill: gain and RoPE rows must be 16-byte aligned");
@@ -1558,7 +1561,7 @@ extern "C" int forge_attn_prefill_docs(int dtype, int B, int T, int H, int K, in
 extern "C" size_t forge_attn_prefill_workspace_bytes(int dtype, int B, int T, int H, int K, int D,
                                                      int64_t offset, int window) {
   if ((dtype != FORGE_BF16 && dtype != FORGE_F16) || (D != 64 && D != 128 && D != 256 && D != 512) || B <= 0 ||
-      T <= 0 || H <= 0 || K <= 0 || H % K || offset < 0 || window < 0 || offset + (int64_t)T + 256 >= (1LL << 31))
+      T <= 0 || H <= 0 || K <= 0 || H % K || offset < 0 || window < 0 || !positions_fit(offset, T))
     return 0;
   const PrefillPlan plan = prefill_plan(false, B, T, H, K, D, offset, window, kMaxParts);
   return plan.nsplit > 1 ? prefill_workspace(plan, B, T, H, D) : 0;
@@ -1582,7 +1585,7 @@ extern "C" int forge_attn_prefill_ws(int dtype, int B, int T, int H, int K, int 
 extern "C" size_t forge_attn_prefill_f32_workspace_bytes(int B, int T, int H, int K, int D, int64_t offset,
                                                          int window) {
   if ((D != 32 && D != 64 && D != 128) || B <= 0 || T <= 0 || H <= 0 || K <= 0 || H % K || offset < 0 ||
-      window < 0 || offset + (int64_t)T + 256 >= (1LL << 31))
+      window < 0 || !positions_fit(offset, T))
     return 0;
   const PrefillPlan plan = prefill_plan(true, B, T, H, K, D, offset, window, kMaxParts);
   return plan.nsplit > 1 ? prefill_workspace(plan, B, T, H, D) : 0;

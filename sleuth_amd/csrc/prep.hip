@@ -268,7 +268,7 @@ extern "C" int forge_kv_append(int dtype, int B, int T, int K, int D, const void
   if (!k || !v || !k_dst || !v_dst) return set_error("null tensor pointer");
   const bool rope = flags & FORGE_ROPE;
   if (rope && (!cos || !sin)) return set_error("FORGE_ROPE needs cos and sin");
-  if (!row_pos && !pos_dev && (pos0 < 0 || pos0 + T > dst_len))
+  if (!row_pos && !pos_dev && (pos0 < 0 || pos0 > dst_len - T))
     return set_error("KV cache full: pos + T exceeds the cache length");
   RowParams p{};
   p.t[0] = RowTensor{k, skb, skh, skt, k_dst, sdb, sdh, sds, k_weight, K,

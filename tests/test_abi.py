@@ -150,3 +150,24 @@ def test_ops_shape_checks_before_any_launch():
     with pytest.raises(ValueError):
         ops.kv_append(torch.zeros(1, 1, 2, 64), torch.zeros(1, 1, 3, 64), torch.zeros(1, 1, 8, 64),
                       torch.zeros(1, 1, 8, 64))
+
+
+@pytest.mark.parametrize("at", [2 ** 31, 2 ** 62, 2 ** 63 - 8, 2 ** 63 - 1])
+def test_positions_whose_end_wraps_are_rejected(at):
+    """pos + T beyond 64 bits is past the cache's end, as every other position there is."""
+    lib = _lib.lib()
+    p = 4096   # never read: the calls are rejected first
+    assert lib.forge_kv_append(_lib.BF16, 1, 20, 2, 64, p, 0, 64, 128, p, 0, 64, 128, p, p, 0, 64 * 64, 64, 64, None, None,
+                               at, None, 1e-6, 0, None, None, 0, 0, None) < 0
+    assert b"KV cache full" in lib.forge_last_error()
+    decode = [_lib.BF16, 1, 20, 4, 2, 64, p, 0, 64, 256, None, 1e-6, 0, None, None, 0, 0, p, p, 0, 64 * 64, 64, 64, None, None,
+              at, 64, 0, 1.0, 64, p, 0, 256, 64]
+    assert lib.forge_attn_decode(*decode, None, 0, None) < 0
+    assert b"KV cache full" in lib.forge_last_error()
+    for st in (lib.forge_attn_prefill(_lib.BF16, 1, 20, 4, 2, 64, p, 0, 64, 256, None, 1e-6, 0, None, None, 0, p, p, 0,
+                                      64 * 64, 64, at, 0, 1.0, p, 0, 256, 64, None),
+               lib.forge_attn_prefill_f32(1, 20, 4, 2, 64, p, 0, 64, 256, None, 1e-6, 0, None, None, 0, p, p, 0, 64 * 64, 64,
+                                          at, 0, 1.0, p, 0, 256, 64, None, 0, None)):
+        assert st < 0 and b"31 bits" in lib.forge_last_error()
+    assert lib.forge_attn_prefill_workspace_bytes(_lib.BF16, 1, 20, 4, 2, 64, at, 0) == 0
+    assert lib.forge_attn_prefill_f32_workspace_bytes(1, 20, 4, 2, 64, at, 0) == 0

@@ -101,6 +101,9 @@ def test_prefill_and_append_equal_the_python_way(monkeypatch, dtype):
             return [y, kc, vc]
         a, b = _both(monkeypatch, call)
         assert _equal(a, b), (off, extra, a, b)
+    for off in (161, 2 ** 31, 2 ** 63 - 20):     # past the keys' end, also where the end wraps
+        a, b = _both(monkeypatch, lambda: fn(q, kc0, vc0, scale=0.2, offset=off))
+        assert a == b and a[0] is ValueError, (off, a, b)
 
 
 @pytest.mark.gpu
