@@ -417,7 +417,7 @@ class Attention(nn.Module):
                                     doc_start=docs, check_doc_start=False, **q_args)
         if T > DECODE_MAX_T and offset is not None and docs is None and \
                 (q_args["cos"] is None or q_args["cos"].dim() == 2) and \
-                ops.prefill_f32_supported(q, q_args["cos"], q_args["sin"]):
+                ops.prefill_f32_supported(q, q_args["cos"], q_args["sin"], q_args.get("q_weight"), kc, offset):
             ops.kv_append(k, v, kc, vc, norm_v=norm_v, **pos_kw, **k_args)
             self.last_path = "hip-decode"   # (what fp32 prompts have always reported)
             return ops.attn_prefill_f32(q, kc, vc, scale=self.scale, offset=offset, window=self.window, **q_args)

@@ -430,11 +430,17 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: fl
 PREFILL_F32_HEAD_DIMS = (32, 64, 128)
 
 
-def prefill_f32_supported(q: torch.Tensor, cos: torch.Tensor | None = None, sin: torch.Tensor | None = None) -> bool:
-    """attn_prefill_f32 takes this q and these tables (16-byte aligned rows; attn_decode takes any)."""
-    aligned = all(t is None or (t.data_ptr() % 16 == 0 and t.dtype == torch.float32 and t.stride(-1) == 1 and
-                                all(n % 4 == 0 for n in t.stride()[:-1])) for t in (cos, sin))
-    return q.dtype == torch.float32 and q.shape[-1] in PREFILL_F32_HEAD_DIMS and aligned
+def prefill_f32_supported(q: torch.Tensor, cos: torch.Tensor | None = None, sin: torch.Tensor | None = None,
+                          q_weight: torch.Tensor | None = None, k: torch.Tensor | None = None, offset: int = 0) -> bool:
+    """attn_prefill_f32 takes this q, these tables and this gain (16-byte aligned rows; attn_decode takes
+    any), and keys k [B,K,S,D] of a slab whose rows up to a tile past the last query lie within 2^31
+    bytes (attn_decode: the cache's own rows)."""
+    if q.dtype != torch.float32 or q.shape[-1] not in PREFILL_F32_HEAD_DIMS:
+        return False
+    if k is not None and (k.stride(2) < k.shape[3] or k.stride(2) * 4 * (offset + q.shape[2] + 256) >= 2 ** 31):
+        return False
+    return all(t is None or (t.data_ptr() % 16 == 0 and t.dtype == torch.float32 and t.stride(-1) == 1 and
+                             all(n % 4 == 0 for n in t.stride()[:-1])) for t in (cos, sin, q_weight))
 
 
 def attn_prefill_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float, offset: int = 0,

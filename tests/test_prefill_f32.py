@@ -36,6 +36,20 @@ def test_rejections():
                                     None) < 0
 
 
+def test_what_it_supports():
+    """The rule sends every call that the kernel would refuse the split-K way."""
+    from sleuth_amd import ops
+
+    q, odd = torch.zeros(1, 4, 20, 32), torch.zeros(33)[1:]
+    k = torch.empty_strided((1, 2, 40, 32), (80 * 2 ** 20, 40 * 2 ** 20, 2 ** 20, 1), device="meta")
+    ok = lambda **kw: ops.prefill_f32_supported(q, **kw)  # noqa: E731
+    assert ok() and ok(q_weight=torch.zeros(32), k=torch.zeros(1, 2, 40, 32), offset=20)
+    assert not ok(q_weight=odd) and not ok(cos=odd[None].expand(20, 32))
+    assert ok(k=k, offset=20) and not ok(k=k, offset=236)         # 2^20 * 4 * (offset + 20 + 256) < 2^31 or not
+    assert not ok(k=k[..., :1, :].expand(1, 2, 40, 32))           # one row for every key
+    assert not ops.prefill_f32_supported(q.half()) and not ops.prefill_f32_supported(torch.zeros(1, 4, 20, 256))
+
+
 @pytest.mark.gpu
 @pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
 @pytest.mark.parametrize("B,T,H,K,D,offset,window", [
@@ -109,3 +123,43 @@ def test_module_takes_fp32_prompts_to_it_and_unaligned_tables_elsewhere(monkeypa
     assert [o[2] for o in outs] == [1, 1]
     assert torch.equal(outs[0][1], outs[1][1])
     assert max_abs(outs[0][0], outs[1][0]) <= 1e-5   # fp32 sums in another order
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("what", ["gain", "slab"])
+def test_module_takes_unaligned_gains_and_wide_slabs_the_split_k_way(monkeypatch, what):
+    """A q_norm weight that is a view into a flat buffer, and a cache whose rows lie so far apart that
+    only its own rows fit 2^31 bytes, give what an aligned gain and a dense cache give."""
+    from host_protocol import HostKVCache
+    from sleuth_amd import ops
+    from sleuth_amd.attention import Attention
+    from sleuth_amd.config import ModelConfig
+
+    torch.manual_seed(4)
+    cfg = ModelConfig(vocab_size=16, d_model=128, n_layers=1, n_heads=4, n_kv_heads=2, qk_norm=True, max_seq_len=64)
+    a = Attention(cfg, 0).to(DEV).eval()
+    a.q_norm.weight.data.copy_(torch.linspace(0.8, 1.2, 32))
+    x = torch.randn(1, 20, 128, device=DEV)
+    cos, sin = (t[:20].to(DEV) for t in tables(32, 64, 1e4))
+    calls, fn = [], ops.attn_prefill_f32
+    monkeypatch.setattr(ops, "attn_prefill_f32", lambda *a, **kw: calls.append(1) or fn(*a, **kw))
+
+    def run():
+        calls.clear()
+        with torch.no_grad():
+            return a(x, cos, sin, cache), cache.k[0].clone(), len(calls)
+
+    cache = HostKVCache([(2, 32)], 1, 20, DEV, F32)
+    want = run()
+    if what == "gain":
+        flat = torch.empty(33, device=DEV)
+        flat[1:] = a.q_norm.weight.detach()
+        a.q_norm.weight.data = flat[1:]
+    else:
+        row = 2 ** 21       # floats: 21 rows span 176 MB, 276 of them 2.3 GB
+        for kv in (cache.k, cache.v):
+            kv[0] = torch.zeros(20 * row, device=DEV).as_strided((1, 2, 20, 32), (64, 32, row, 1))
+    got = run()
+    assert (want[2], got[2]) == (1, 0)
+    assert torch.equal(want[1], got[1]) and max_abs(want[0], got[0]) <= 1e-5   # fp32 sums in another order
