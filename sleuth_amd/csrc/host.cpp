@@ -98,30 +98,43 @@ bool capturing() {
   return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
 }
 
-// The caller's workspace table (ops._STREAM_WS: a cleared buffer per (device, stream), the most
-// recently used last): the buffer's address if it is there and large enough.
-bool stream_workspace(PyObject* table, int dev, hipStream_t stream, size_t need, void*& ws, size_t& bytes) {
-  PyObject* key = Py_BuildValue("(iK)", dev, (unsigned long long)(uintptr_t)stream);
-  if (!key) {
-    PyErr_Clear();
-    return false;
-  }
-  bool ok = false;
-  PyObject* buf = PyDict_GetItemWithError(table, key);
-  if (buf && THPVariable_CheckExact(buf)) {
-    const Tensor& t = THPVariable_Unpack(buf);
-    bytes = (size_t)t.numel();
-    if (bytes >= need) {
-      ws = t.data_ptr();
-      Py_INCREF(buf);
-      ok = PyDict_DelItem(table, key) == 0 && PyDict_SetItem(table, key, buf) == 0;
-      Py_DECREF(buf);
+// Gives the GIL up for its scope (no Python object is touched there): an allocation may have to free
+// and synchronise, and a launch waits while the stream's queue is full.
+struct NoGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+// The buffer of (device, stream) from the caller's workspace table (ops._STREAM_WS: cleared buffers,
+// the most recently used last), taken out of the table while a call uses it, so that no other thread
+// launches on it in between, and put back once the call is launched.
+struct StreamWorkspace {
+  PyObject *table, *key = nullptr, *buf = nullptr;
+  void* ptr = nullptr;
+  size_t bytes = 0;
+
+  StreamWorkspace(PyObject* table, int dev, hipStream_t stream, size_t need) : table(table) {
+    if (!need) return;
+    key = Py_BuildValue("(iK)", dev, (unsigned long long)(uintptr_t)stream);
+    PyObject* b = key ? PyDict_GetItemWithError(table, key) : nullptr;
+    if (b && THPVariable_CheckExact(b) && (size_t)THPVariable_Unpack(b).numel() >= need) {
+      Py_INCREF(b);
+      if (PyDict_DelItem(table, key) == 0) buf = b;
+      else Py_DECREF(b);
     }
+    if (PyErr_Occurred()) PyErr_Clear();
+    if (!buf) return;
+    ptr = THPVariable_Unpack(buf).data_ptr();
+    bytes = (size_t)THPVariable_Unpack(buf).numel();
   }
-  if (PyErr_Occurred()) PyErr_Clear();
-  Py_DECREF(key);
-  return ok;
-}
+  void put_back() {
+    if (buf && PyDict_SetItem(table, key, buf) != 0) PyErr_Clear();
+  }
+  ~StreamWorkspace() {
+    Py_XDECREF(buf);
+    Py_XDECREF(key);
+  }
+};
 
 PyObject* result(int st, const Tensor& out) {
   if (st != 0) return PyLong_FromLong(st);
@@ -177,20 +190,26 @@ PyObject* decode_append_impl(PyObject* const* a) {
   }
   const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
   const size_t need = forge_attn_decode_workspace_bytes(dt, (int)B, (int)T, (int)H, (int)K, (int)D, max_kv, (int)chunk);
-  void* ws = nullptr;
-  size_t ws_bytes = 0;
-  if (need && (capturing() || !stream_workspace(a[0], dev.index(), stream, need, ws, ws_bytes))) return nullptr;
-  Tensor out = at::empty({B, T, H, D}, q.options().requires_grad(false));
+  if (need && capturing()) return nullptr;
+  StreamWorkspace ws(a[0], dev.index(), stream, need);
+  if (need && !ws.ptr) return nullptr;
   const int rope = r.cos ? FORGE_ROPE : 0;
-  const int st = forge_attn_decode_append(
-      dt, (int)B, (int)T, (int)H, (int)K, (int)D, ptr(q), q.stride(0), q.stride(1), q.stride(2),
-      norm_q ? static_cast<const float*>(ptr(qw)) : nullptr, eps, (norm_q ? FORGE_NORM_QK : 0) | rope, ptr(k),
-      k.stride(0), k.stride(1), k.stride(2), ptr(v), v.stride(0), v.stride(1), v.stride(2),
-      norm_k ? static_cast<const float*>(ptr(kw)) : nullptr,
-      (norm_k ? FORGE_NORM_QK : 0) | rope | (norm_v ? FORGE_NORM_V : 0), r.cos, r.sin, r.sb, r.st, kc.data_ptr(),
-      vc.data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), max_len, static_cast<const int32_t*>(ptr(row_pos)),
-      static_cast<const int64_t*>(ptr(pos_dev)), pos, max_kv, (int)window, scale, (int)chunk, out.data_ptr(),
-      out.stride(0), out.stride(1), out.stride(2), ws, ws_bytes, ws ? FORGE_WS_ZEROED : 0, stream);
+  Tensor out;
+  int st;
+  {
+    NoGil unlocked;
+    out = at::empty({B, T, H, D}, q.options().requires_grad(false));
+    st = forge_attn_decode_append(
+        dt, (int)B, (int)T, (int)H, (int)K, (int)D, ptr(q), q.stride(0), q.stride(1), q.stride(2),
+        norm_q ? static_cast<const float*>(ptr(qw)) : nullptr, eps, (norm_q ? FORGE_NORM_QK : 0) | rope, ptr(k),
+        k.stride(0), k.stride(1), k.stride(2), ptr(v), v.stride(0), v.stride(1), v.stride(2),
+        norm_k ? static_cast<const float*>(ptr(kw)) : nullptr,
+        (norm_k ? FORGE_NORM_QK : 0) | rope | (norm_v ? FORGE_NORM_V : 0), r.cos, r.sin, r.sb, r.st, kc.data_ptr(),
+        vc.data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), max_len, static_cast<const int32_t*>(ptr(row_pos)),
+        static_cast<const int64_t*>(ptr(pos_dev)), pos, max_kv, (int)window, scale, (int)chunk, out.data_ptr(),
+        out.stride(0), out.stride(1), out.stride(2), ws.ptr, ws.bytes, ws.ptr ? FORGE_WS_ZEROED : 0, stream);
+  }
+  if (st == 0) ws.put_back();
   return result(st, out);
 }
 
@@ -217,11 +236,16 @@ PyObject* kv_append_impl(PyObject* const* a) {
   Rope r;
   if (!rope_ok(cos, sin, B, T, D, dev, r) || !gain_ok(kw, D, dev)) return nullptr;
   const int flags = (norm_k ? FORGE_NORM_QK : 0) | (r.cos ? FORGE_ROPE : 0) | (norm_v ? FORGE_NORM_V : 0);
-  return PyLong_FromLong(forge_kv_append(
-      dt, (int)B, (int)T, (int)K, (int)D, ptr(k), k.stride(0), k.stride(1), k.stride(2), ptr(v), v.stride(0),
-      v.stride(1), v.stride(2), kc.data_ptr(), vc.data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), kc.size(2),
-      nullptr, nullptr, pos, norm_k ? static_cast<const float*>(ptr(kw)) : nullptr, eps, flags, r.cos, r.sin, r.sb,
-      r.st, c10::hip::getCurrentHIPStream(dev.index()).stream()));
+  int st;
+  {
+    NoGil unlocked;
+    st = forge_kv_append(
+        dt, (int)B, (int)T, (int)K, (int)D, ptr(k), k.stride(0), k.stride(1), k.stride(2), ptr(v), v.stride(0),
+        v.stride(1), v.stride(2), kc.data_ptr(), vc.data_ptr(), kc.stride(0), kc.stride(1), kc.stride(2), kc.size(2),
+        nullptr, nullptr, pos, norm_k ? static_cast<const float*>(ptr(kw)) : nullptr, eps, flags, r.cos, r.sin, r.sb,
+        r.st, c10::hip::getCurrentHIPStream(dev.index()).stream());
+  }
+  return PyLong_FromLong(st);
 }
 
 // prefill(q, k, v, scale, offset, window, q_weight | None, eps, norm_q, cos | None, sin | None): bf16/fp16 through
@@ -251,21 +275,26 @@ PyObject* prefill_impl(PyObject* const* a) {
   const int flags = (norm_q ? FORGE_NORM_QK : 0) | (r.cos ? FORGE_ROPE : 0);
   const float* w = norm_q ? static_cast<const float*>(ptr(qw)) : nullptr;
   const auto opts = q.options().requires_grad(false);
-  Tensor out = at::empty({B, T, H, D}, opts), ws;
-  const size_t need = f32 ? forge_attn_prefill_f32_workspace_bytes((int)B, (int)T, (int)H, (int)K, (int)D, offset, (int)window)
-                          : forge_attn_prefill_workspace_bytes(dt, (int)B, (int)T, (int)H, (int)K, (int)D, offset, (int)window);
-  if (need) ws = at::empty({(int64_t)need}, opts.dtype(at::kByte));
-  void* wp = need ? ws.data_ptr() : nullptr;
-  const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
-  const int st =
-      f32 ? forge_attn_prefill_f32((int)B, (int)T, (int)H, (int)K, (int)D, ptr(q), q.stride(0), q.stride(1), q.stride(2),
-                                   w, eps, flags, r.cos, r.sin, r.st, ptr(k), ptr(v), k.stride(0), k.stride(1),
-                                   k.stride(2), offset, (int)window, scale, out.data_ptr(), out.stride(0),
-                                   out.stride(1), out.stride(2), wp, need, stream)
-          : forge_attn_prefill_ws(dt, (int)B, (int)T, (int)H, (int)K, (int)D, ptr(q), q.stride(0), q.stride(1),
-                                  q.stride(2), w, eps, flags, r.cos, r.sin, r.st, ptr(k), ptr(v), k.stride(0),
-                                  k.stride(1), k.stride(2), offset, (int)window, scale, nullptr, 0, out.data_ptr(),
-                                  out.stride(0), out.stride(1), out.stride(2), wp, need, stream);
+  Tensor out, ws;
+  int st;
+  {
+    NoGil unlocked;
+    out = at::empty({B, T, H, D}, opts);
+    const size_t need =
+        f32 ? forge_attn_prefill_f32_workspace_bytes((int)B, (int)T, (int)H, (int)K, (int)D, offset, (int)window)
+            : forge_attn_prefill_workspace_bytes(dt, (int)B, (int)T, (int)H, (int)K, (int)D, offset, (int)window);
+    if (need) ws = at::empty({(int64_t)need}, opts.dtype(at::kByte));
+    void* wp = need ? ws.data_ptr() : nullptr;
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
+    st = f32 ? forge_attn_prefill_f32((int)B, (int)T, (int)H, (int)K, (int)D, ptr(q), q.stride(0), q.stride(1),
+                                      q.stride(2), w, eps, flags, r.cos, r.sin, r.st, ptr(k), ptr(v), k.stride(0),
+                                      k.stride(1), k.stride(2), offset, (int)window, scale, out.data_ptr(),
+                                      out.stride(0), out.stride(1), out.stride(2), wp, need, stream)
+             : forge_attn_prefill_ws(dt, (int)B, (int)T, (int)H, (int)K, (int)D, ptr(q), q.stride(0), q.stride(1),
+                                     q.stride(2), w, eps, flags, r.cos, r.sin, r.st, ptr(k), ptr(v), k.stride(0),
+                                     k.stride(1), k.stride(2), offset, (int)window, scale, nullptr, 0, out.data_ptr(),
+                                     out.stride(0), out.stride(1), out.stride(2), wp, need, stream);
+  }
   return result(st, out);
 }
 
@@ -297,10 +326,15 @@ PyObject* linear_small_impl(PyObject* const* a) {
   if (((uintptr_t)ptr(x) | (uintptr_t)ptr(w) | (uintptr_t)ptr(up) | (uintptr_t)ptr(gain)) % 16) return nullptr;
   auto shape = x.sizes().vec();
   shape.back() = N;
-  Tensor out = at::empty(shape, x.options().requires_grad(false));
-  const int st = forge_linear_small(dt, (int)M, (int)N, (int)K, ptr(x), K, ptr(w), ptr(up), K, ptr(b),
-                                    ptr(gain), gain.defined() ? dtype_of(gain) : FORGE_F32, norm, eps, ptr(res), N, out.data_ptr(), N,
-                                    c10::hip::getCurrentHIPStream(dev.index()).stream());
+  Tensor out;
+  int st;
+  {
+    NoGil unlocked;
+    out = at::empty(shape, x.options().requires_grad(false));
+    st = forge_linear_small(dt, (int)M, (int)N, (int)K, ptr(x), K, ptr(w), ptr(up), K, ptr(b), ptr(gain),
+                            gain.defined() ? dtype_of(gain) : FORGE_F32, norm, eps, ptr(res), N, out.data_ptr(), N,
+                            c10::hip::getCurrentHIPStream(dev.index()).stream());
+  }
   return result(st, out);
 }
 

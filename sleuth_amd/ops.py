@@ -245,19 +245,24 @@ _STREAM_WS: dict = {}
 _STREAM_WS_MAX = 16   # streams whose workspace is kept (the oldest is dropped beyond that)
 
 
-def _stream_workspace(dev: torch.device, need: int) -> torch.Tensor:
+def _take_stream_workspace(dev: torch.device, need: int) -> tuple[tuple, torch.Tensor]:
     """A split-K workspace per (device, stream), cleared when it is made: every call leaves
     its work ticket zero, so calls ordered on that stream may skip the ticket reset. Grown
-    (a new cleared buffer) when a call needs more. Dropping a buffer is safe while its calls
+    (a new cleared buffer) when a call needs more. It is out of the table until the call is
+    launched (_put_back_stream_workspace): another thread on the stream makes one of its own
+    rather than launch between this call's kernels. Dropping a buffer is safe while its calls
     are in flight: torch's allocator reuses the memory only in that stream's order."""
     key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
     ws = _STREAM_WS.pop(key, None)
     if ws is None or ws.numel() < need:
         ws = torch.zeros(max(need, 1 << 20), dtype=torch.uint8, device=dev)
+    return key, ws
+
+
+def _put_back_stream_workspace(key: tuple, ws: torch.Tensor) -> None:
     _STREAM_WS[key] = ws   # most recently used last
-    while len(_STREAM_WS) > _STREAM_WS_MAX:
-        _STREAM_WS.pop(next(iter(_STREAM_WS)))
-    return ws
+    for old in list(_STREAM_WS)[:-_STREAM_WS_MAX]:
+        _STREAM_WS.pop(old, None)
 
 
 def attn_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
@@ -300,9 +305,9 @@ def attn_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
     kv_flags = (NORM_QK if norm_k else 0) | (ROPE if c is not None else 0) | (NORM_V if norm_v else 0)
     kw = _weight(k_weight, D) if norm_k else None
     need = lib().forge_attn_decode_workspace_bytes(args[0], B, T, q.shape[1], K, D, max_kv_len, chunk)
-    zeroed = bool(workspace_zeroed)
+    zeroed, key = bool(workspace_zeroed), None
     if need and workspace is None and not torch.cuda.is_current_stream_capturing():
-        workspace, zeroed = _stream_workspace(dev, need), True
+        (key, workspace), zeroed = _take_stream_workspace(dev, need), True
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace, zeroed = torch.empty(need, dtype=torch.uint8, device=dev), False
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
@@ -311,6 +316,8 @@ def attn_decode_append(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
                                         *args[13:], _ptr(workspace), ws_bytes, WS_ZEROED if zeroed else 0,
                                         _stream(dev))
     check(st, "forge_attn_decode_append")
+    if key is not None:
+        _put_back_stream_workspace(key, workspace)
     return out
 
 

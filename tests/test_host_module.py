@@ -3,7 +3,9 @@ give the Python way's results bit for bit, errors included."""
 
 from __future__ import annotations
 
+import sys
 import threading
+import time
 import types
 
 import pytest
@@ -132,3 +134,66 @@ def test_streams_and_threads_have_workspaces_of_their_own():
     for t in threads:
         t.join()
     assert all(len(got[i]) == 50 and all(torch.equal(y, want[i]) for y in got[i]) for i in range(2))
+
+
+@pytest.mark.gpu
+@needs_gpu
+def test_launches_give_up_the_gil():
+    """With the interpreter's own switching all but off, a waiting thread runs only if the native calls
+    give the GIL up around their launches."""
+    k = torch.zeros(1, 1, 1, 64, dtype=torch.bfloat16, device=DEV)
+    cache, host = torch.zeros(2, 1, 1, 4, 64, dtype=torch.bfloat16, device=DEV), ops.host()
+    started, ran, interval = threading.Event(), [], sys.getswitchinterval()
+
+    def other():
+        started.set()
+        time.sleep(0.01)       # until the loop below holds the GIL
+        ran.append(1)
+
+    thread = threading.Thread(target=other)
+    try:
+        thread.start()
+        started.wait()
+        sys.setswitchinterval(1000.0)
+        for n in range(30000):
+            assert host.kv_append(k, k, cache[0], cache[1], 0, None, 0.0, False, False, None, None) == 0
+            if ran:
+                break
+        assert ran
+    finally:
+        sys.setswitchinterval(interval)
+        thread.join()
+        torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@needs_gpu
+@pytest.mark.parametrize("native", [False, True])
+def test_a_streams_workspace_is_out_of_the_table_during_a_call(monkeypatch, native):
+    """Threads on one stream: while a call launches, the table must not hand its buffer to another."""
+    g = gen(6)
+    q, k, v = (t.to(DEV) for t in qkv_proj_views(g, 1, 1, 4, 2, 64, torch.bfloat16))
+    kc, vc = (randn(g, 1, 2, 3000, 64, dtype=torch.bfloat16).to(DEV) for _ in range(2))
+    call = lambda: ops.attn_decode_append(q, k, v, kc, vc, scale=0.1, pos=2900, chunk=256)  # noqa: E731
+    key = (torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream)
+    ops._STREAM_WS.pop(key, None)
+    want = call()
+    buf = ops._STREAM_WS[key]
+    if native:
+        # the native call takes the buffer and puts it back: nothing else of the table changes
+        others = {("other", i): torch.zeros(1) for i in range(3)}
+        table = {key: buf, **others}
+        monkeypatch.setattr(ops, "_STREAM_WS", table)
+        assert torch.equal(call(), want)
+        assert list(table)[-1] == key and table[key] is buf and len(table) == 4
+    else:
+        monkeypatch.setattr(ops, "host", lambda: DECLINE)
+        fn, during = _lib.lib().forge_attn_decode_append, []
+
+        class Lib:
+            def __getattr__(self, name):
+                real = getattr(_lib.lib(), name)
+                return (lambda *a: during.append(key in ops._STREAM_WS) or fn(*a)) if name == fn.__name__ else real
+        monkeypatch.setattr(ops, "lib", Lib)
+        assert torch.equal(call(), want)
+        assert during == [False] and ops._STREAM_WS[key] is buf
