@@ -261,7 +261,11 @@ int forge_attn_prefill_f32(int B, int T, int H, int K, int D, const void* q, int
  * multiple of 32, y [M, N] with row stride so. Optional, each rounding to the dtype where the
  * eager layers do: norm != 0: RMSNorm of x's rows first (gain [K] of gain_dtype: fp32 or x's type; eps); w2 != NULL:
  * y = silu(x . W^T) * (x . w2^T); bias [N]; residual [M, N] (row stride sr): added last.
+ * forge_linear_small_rows (pure host function): up to how many rows the call of such a form is at
+ * least as fast as a library GEMM with the norm, the product or the sum in launches of their own (0:
+ * never); the call itself takes any of its shapes.
  */
+int forge_linear_small_rows(int N, int K, int norm, int gated, int residual);
 int forge_linear_small(int dtype, int M, int N, int K, const void* x, int64_t sx, const void* w,
                        const void* w2, int64_t sw, const void* bias, const void* gain,
                        int gain_dtype, int norm, float eps, const void* residual, int64_t sr,

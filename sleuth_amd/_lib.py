@@ -125,6 +125,7 @@ SIGNATURES: dict[str, tuple] = {
         _p, _i64, _i64, _i64,                # out + strides (b, t, h)
         _p, C.c_size_t,                      # workspace, bytes
         _p]),
+    "forge_linear_small_rows": (_i, [_i, _i, _i, _i, _i]),   # N, K, norm, gated, residual
     "forge_linear_small": (_i, [
         _i, _i, _i, _i,                      # dtype, M, N, K
         _p, _i64,                            # x, row stride

@@ -323,6 +323,8 @@ PyObject* linear_small_impl(PyObject* const* a) {
     return nullptr;
   const int64_t M = x.numel() / K;
   if (res.defined() && res.numel() != M * N) return nullptr;
+  if (N > INT_MAX || K > INT_MAX || M > forge_linear_small_rows((int)N, (int)K, norm, up.defined(), res.defined()))
+    return nullptr;   // torch's calls are faster there
   if (((uintptr_t)ptr(x) | (uintptr_t)ptr(w) | (uintptr_t)ptr(up) | (uintptr_t)ptr(gain)) % 16) return nullptr;
   auto shape = x.sizes().vec();
   shape.back() = N;

@@ -16,8 +16,9 @@
 // once and the norm adds one barrier: a pass over x of its own, with W's loads only in flight, took
 // 1.3 us more at K 1,024 (5.2 us against 3.9 without the norm; now 3.7 against 2.7).
 //
-// Measured (bf16, graph replays of the call alone, 1 / 5 / 16 rows, us; in brackets the form before,
-// one box each): 4096 x 1024 with norm 3.7 / 3.9 / 4.4 (5.2 / 5.4 / 6.2), hipBLASLt's product alone
+// Measured (bf16, graph replays of the call alone on one W, which the 256 MB MALL then holds up to
+// that size; 1 / 5 / 16 rows, us; in brackets the form before, one box each; on W of its own per call,
+// as in a model, see LinRule below): 4096 x 1024 with norm 3.7 / 3.9 / 4.4 (5.2 / 5.4 / 6.2), hipBLASLt's product alone
 // 6.3; 1024 x 2048 with residual 3.8 / 4.1 / 5.2 (4.3 / 4.4 / 5.2), hipBLASLt 8.2; 3072 x 1024 SwiGLU
 // with norm 4.7 / 4.9 / 5.4 (6.9 / 7.3 / 8.2); 1024 x 3072 with residual 4.9 / 5.4 / 6.9 (6.4 / 6.7 /
 // 7.8), hipBLASLt 9.4; 8192 x 1024 with norm 5.0 / 5.3 / 6.2 (7.1 / 7.4 / 8.8), hipBLASLt 6.7; 4096 x
@@ -248,6 +249,54 @@ static void launch_tiles(const LinearParams& p, hipStream_t s) {
   else launch_plain<T, false, 1, 8>(p, grid, s);
 }
 
+// Up to how many rows a caller that can make torch's calls instead should take this launch
+// (forge_linear_small_rows). Every block reads all of x, and does the norm's work on it, so the launch
+// loses to the library's GEMM as rows, K and blocks grow; what it saves are the launches around the
+// product. The lines lie where the whole of it is no slower than torch's calls. us here / torch, bf16,
+// graph replays with a W of its own per call (0.7 GB in all, so from HBM), at 1, 4, 8 and 16 rows:
+//   plain      4096 x 4096    9.3/15.7   9.4/15.7   9.7/15.6  11.1/15.7
+//              8192 x 2048   10.1/14.1   9.3/13.1  10.0/13.2  10.9/13.3
+//             12288 x 1024    6.8/9.9    6.7/9.3    7.1/9.3    8.2/9.3
+//             10240 x 768     6.3/7.8    6.6/7.9    7.0/8.0    8.1/7.9
+//       not    5120 x 3072   11.2/11.5  11.6/11.5  12.2/11.6  14.5/11.5
+//       not    5120 x 5120   18.6/14.5  19.8/14.3  22.3/14.9  27.9/15.7
+//       not   32768 x 256    10.4/8.1   11.0/8.2   11.8/8.3   13.2/8.4
+//   residual   4096 x 14336  25.2/28.7  27.3/28.6  28.4/27.4  34.7/28.0
+//              2048 x 8192   13.1/14.7  13.8/14.9  14.8/15.0  18.1/15.3
+//       not    4096 x 16384  40.6/32.5  40.9/34.1  42.4/34.6  44.4/33.1
+//       not    8192 x 28672  87.6/92.7  96.8/91.6   113/90     132/91
+//   norm       6144 x 2048   11.2/20.5  11.8/21.1  12.8/21.8  15.4/21.6
+//              6144 x 4096   19.2/25.5  20.2/25.4  22.5/25.6  27.7/25.8
+//             12288 x 4096   31.6/38.7  31.7/38.3  35.1/38.7  43.6/38.6
+//             13312 x 4096   34.8/38.2  38.3/39.6  43.0/40.5  52.8/39.0
+//             32768 x 2048   34.5/44.2  34.9/42.6  37.3/42.8  42.5/43.1
+//            151936 x 1024   62.8/72.4  66.6/72.6  69.8/73.5  74.4/75.1
+//            163840 x 2048    142/163    155/162    166/168    184/165
+//       not    7168 x 5120   24.7/29.6  27.0/28.9  29.2/29.4  37.2/29.8
+//       not  128256 x 4096    225/201    237/197    258/197    298/201
+//       not  131072 x 512      47/40      49/40      49/41      52/42
+//   norm and   9728 x 2560   35.6/53.4  37.5/50.6  40.5/51.9  45.4/49.7
+//   SwiGLU    11008 x 4096   46.7/70.9  49.7/73.1  54.6/71.9  62.4/69.0
+//             14336 x 4096   59.0/73.2  63.9/75.9  67.3/73.8  78.0/74.1
+//             28672 x 4096    106/143    114/142    125/136    138/136
+//             13824 x 5120   79.8/90.8  85.3/88.0  92.6/85.7   105/76
+//             28672 x 8192    191/262    199/238    222/241    263/242
+struct LinRule {
+  int n, k, rows;  // up to n outputs of up to k channels: up to `rows` rows
+};
+// the first line that holds a shape decides; none: 0 rows
+constexpr LinRule kLinPlainRule[] = {{4096, 4096, 16}, {8192, 2048, 16}, {16640, 512, 16}, {12288, 1024, 12}};
+constexpr LinRule kLinResidualRule[] = {{4096, 4096, 16}, {8192, 2048, 16}, {16640, 512, 16}, {12288, 1024, 12}, {4096, 16383, 4}};
+constexpr LinRule kLinNormRule[] = {{16640, 255, 16}, {1 << 30, 255, 0}, {4096, 4096, 16}, {32768, 2048, 16}, {1 << 30, 767, 0},
+                                    {155648, 1024, 16}, {155648, 2048, 8}, {163840, 2048, 4}, {12288, 4096, 8}, {16384, 4096, 4}};
+constexpr LinRule kLinGatedRule[] = {{12288, 4096, 16}, {28672, 2048, 16}, {28672, 4096, 8}, {28672, 8192, 4}};
+
+template <int COUNT> static int rule_rows(const LinRule (&rule)[COUNT], int N, int K) {
+  for (const LinRule& r : rule)
+    if (N <= r.n && K <= r.k) return r.rows;
+  return 0;
+}
+
 template <typename T>
 static int launch_linear(const LinearParams& p, hipStream_t s) {
   if (p.w2) launch_tiles<T, true, 1>(p, s);
@@ -259,6 +308,13 @@ static int launch_linear(const LinearParams& p, hipStream_t s) {
 }  // namespace forge
 
 using namespace forge;
+
+extern "C" int forge_linear_small_rows(int N, int K, int norm, int gated, int residual) {
+  if (N <= 0 || K <= 0 || K % 32) return 0;
+  return gated ? rule_rows(kLinGatedRule, N, K)
+               : norm ? rule_rows(kLinNormRule, N, K)
+                      : residual ? rule_rows(kLinResidualRule, N, K) : rule_rows(kLinPlainRule, N, K);
+}
 
 extern "C" int forge_linear_small(int dtype, int M, int N, int K, const void* x, int64_t sx, const void* w,
                                   const void* w2, int64_t sw, const void* bias, const void* gain,

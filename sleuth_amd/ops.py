@@ -497,8 +497,8 @@ def linear_small(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = N
                  norm: bool = False, residual: torch.Tensor | None = None) -> torch.Tensor | None:
     """F.linear(x, w, bias) of a decode or verify step (forge_linear_small), without autograd;
     norm: x gets RMSNorm (gain [K], fp32 or of x's type) first; w_up: silu(x . w^T) * (x . w_up^T); residual [..., N]:
-    added to the result. None where the call is not of the kernel's form (the caller then makes
-    the torch calls): it takes bf16/fp16 on one GPU, x [..., K] of at most 16 rows, K a multiple of
+    added to the result. None where the call is not of the kernel's form, or where torch's calls
+    are faster (forge_linear_small_rows), for the caller to make those: it takes bf16/fp16 on one GPU, x [..., K] of at most 16 rows, K a multiple of
     32, everything contiguous and 16-byte aligned, and nothing (autocast, tracing, a dispatch or
     function mode, a tensor subclass, a forward-mode tangent) between the call and the memory."""
     if torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or \

@@ -29,6 +29,35 @@ def test_rejections():
         assert call(**{"out": 4096 if kw else None, **kw}) < 0
 
 
+def test_rows_up_to_which_the_launch_is_taken():
+    """Shapes measured on either side of the rule's lines (N, K -> rows per form)."""
+    rows = _lib.lib().forge_linear_small_rows
+    want = {   # plain, residual, norm, gated
+        (4096, 1024): (16, 16, 16, 16), (1024, 3072): (16, 16, 16, 16), (4096, 4096): (16, 16, 16, 16),
+        (8192, 2048): (16, 16, 16, 16), (10240, 768): (12, 12, 16, 16), (6144, 4096): (0, 0, 8, 16), (5120, 5120): (0, 0, 0, 4),
+        (4096, 14336): (0, 4, 0, 0), (4096, 16384): (0, 0, 0, 0), (14336, 4096): (0, 0, 4, 8), (28672, 8192): (0, 0, 0, 4),
+        (32768, 2048): (0, 0, 16, 0), (151936, 1024): (0, 0, 16, 0), (128256, 4096): (0, 0, 0, 0),
+        (163840, 2048): (0, 0, 4, 0), (131072, 512): (0, 0, 0, 0), (65536, 128): (0, 0, 0, 0), (16403, 64): (16, 16, 16, 16)}
+    for (N, K), w in want.items():
+        assert (rows(N, K, 0, 0, 0), rows(N, K, 0, 0, 1), rows(N, K, 1, 0, 0)) == w[:3], (N, K)
+        if N < 16403:
+            assert rows(N, K, 1, 1, 0) == w[3], (N, K)
+    assert rows(0, 64, 0, 0, 0) == rows(64, 48, 0, 0, 0) == rows(64, 0, 1, 1, 0) == 0
+
+
+@pytest.mark.gpu
+@needs_gpu
+def test_torch_takes_the_shapes_that_it_is_faster_at():
+    """A layer of a wide model: the rule's rows go through the kernel, one more through torch."""
+    from sleuth_amd import ops
+
+    x, w = torch.randn(9, 4096, device=DEV).bfloat16(), torch.randn(6144, 4096, device=DEV).bfloat16()
+    gain = torch.ones(4096, device=DEV)
+    kw = dict(gain=gain, eps=1e-6, norm=True)
+    assert ops.linear_small(x[:8], w, **kw) is not None and ops.linear_small(x, w, **kw) is None
+    assert ops.linear_small(x[:1], w) is None
+
+
 @pytest.mark.gpu
 @needs_gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
