@@ -283,8 +283,13 @@ PyObject* prefill_impl(PyObject* const* a) {
     const size_t need =
         f32 ? forge_attn_prefill_f32_workspace_bytes((int)B, (int)T, (int)H, (int)K, (int)D, offset, (int)window)
             : forge_attn_prefill_workspace_bytes(dt, (int)B, (int)T, (int)H, (int)K, (int)D, offset, (int)window);
-    if (need) ws = at::empty({(int64_t)need}, opts.dtype(at::kByte));
-    void* wp = need ? ws.data_ptr() : nullptr;
+    if (need) {
+      try {
+        ws = at::empty({(int64_t)need}, opts.dtype(at::kByte));
+      } catch (const c10::OutOfMemoryError&) {   // the launch is not split then
+      }
+    }
+    void* wp = ws.defined() ? ws.data_ptr() : nullptr;
     const hipStream_t stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
     st = f32 ? forge_attn_prefill_f32((int)B, (int)T, (int)H, (int)K, (int)D, ptr(q), q.stride(0), q.stride(1),
                                       q.stride(2), w, eps, flags, r.cos, r.sin, r.st, ptr(k), ptr(v), k.stride(0),

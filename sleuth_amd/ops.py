@@ -366,6 +366,15 @@ def attn_drafter(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
 PREFILL_HEAD_DIMS = (64, 128, 256, 512)
 
 
+def _partials(need: int, dev: torch.device) -> torch.Tensor | None:
+    """Workspace of a key-split prefill launch. None where it is not split, also for want of memory: the
+    unsplit launch needs none."""
+    try:
+        return torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    except torch.OutOfMemoryError:
+        return None
+
+
 def prefill_supported(q: torch.Tensor) -> bool:
     return q.dtype in (torch.bfloat16, torch.float16) and q.shape[-1] in PREFILL_HEAD_DIMS
 
@@ -423,7 +432,7 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: fl
         doc_ptr, doc_stride = _ptr(doc_start), doc_start.stride(0)
     # partials of a key-split launch (0: the shape is not split)
     need = 0 if doc_ptr else lib().forge_attn_prefill_workspace_bytes(dtype_code(q), B, T, H, K, D, int(offset), int(window))
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    ws = _partials(need, dev)
     st = lib().forge_attn_prefill_ws(dtype_code(q), B, T, H, K, D, _ptr(q), q.stride(0), q.stride(1),
                                      q.stride(2), _ptr(w), float(eps), flags, _ptr(c), _ptr(s), s_t,
                                      _ptr(k), _ptr(v), k.stride(0), k.stride(1), k.stride(2),
@@ -480,7 +489,7 @@ def attn_prefill_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale
     w = _weight(q_weight, D) if norm_q else None
     out = torch.empty(B, T, H, D, dtype=q.dtype, device=dev)
     need = lib().forge_attn_prefill_f32_workspace_bytes(B, T, H, K, D, int(offset), int(window))
-    ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    ws = _partials(need, dev)
     st = lib().forge_attn_prefill_f32(B, T, H, K, D, _ptr(q), q.stride(0), q.stride(1), q.stride(2), _ptr(w),
                                       float(eps), flags, _ptr(c), _ptr(s), s_t, _ptr(k), _ptr(v), k.stride(0),
                                       k.stride(1), k.stride(2), int(offset), int(window), float(scale), _ptr(out),

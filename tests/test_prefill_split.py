@@ -3,6 +3,8 @@ edges of its parts, tiles and windows against the oracle and the unsplit launch.
 
 from __future__ import annotations
 
+import types
+
 import pytest
 import torch
 
@@ -139,3 +141,36 @@ def test_wide_prefill_with_four_heads_per_block(dtype, window, docs):
                            eps=1e-6, norm_q=True, cos=cos.to(DEV), sin=sin.to(DEV),
                            doc_start=starts.to(DEV) if docs else None)
     assert max_abs(got.cpu().transpose(1, 2), ref) <= tol(dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("native", [True, False])
+def test_without_memory_for_the_partials_the_launch_is_not_split(monkeypatch, native):
+    """With the process's memory limited to what it holds and room for the output, a call that would
+    split gives the unsplit launch's result (forge_attn_prefill, which has no workspace)."""
+    from sleuth_amd import ops
+
+    B, T, H, K, D, offset = 1, 1024, 16, 8, 128, 15360
+    g = gen(970)
+    q = randn(g, B, T, H, D, dtype=torch.bfloat16).transpose(1, 2).to(DEV)
+    kc, vc = (randn(g, B, K, offset + T, D, dtype=torch.bfloat16).to(DEV) for _ in range(2))
+    room = 24 << 20              # a 20 MB segment of the allocator for the output (4 MB)
+    assert _bytes(B, T, H, K, D, offset) > room
+    call = lambda: ops.attn_prefill(q, kc, vc, scale=scale_of(D), offset=offset)  # noqa: E731
+    split, want = call(), torch.empty(B, T, H, D, dtype=torch.bfloat16, device=DEV)
+    if not native:
+        monkeypatch.setattr(ops, "host", lambda: types.SimpleNamespace(prefill=lambda *a: None))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    limit = (torch.cuda.memory_reserved() + room) / torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction(limit)
+        got = call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    _lib.check(_lib.lib().forge_attn_prefill(
+        _lib.BF16, B, T, H, K, D, q.data_ptr(), *q.stride()[:3], None, 1e-6, 0, None, None, 0, kc.data_ptr(),
+        vc.data_ptr(), *kc.stride()[:3], offset, 0, scale_of(D), want.data_ptr(), *want.stride()[:3],
+        torch.cuda.current_stream().cuda_stream), "forge_attn_prefill")
+    assert torch.equal(got, want) and not torch.equal(got, split)
