@@ -1390,6 +1390,7 @@ static PrefillPlan prefill_plan(bool f32, int B, int T, int H, int K, int D, int
       if (parts > 1) split1 += parts;
       work1 += n;
     }
+    bool open = false;  // some split into more parts may still win
     for (int hpb = most_heads; hpb >= (most_heads == 4 ? 2 : most_heads); hpb /= 2) {
       double alone = hpb == 4 ? 2.55 : wide ? 2.1 : D == 256 ? 1.25 : 1.2;
       double shared = wide ? alone : D == 256 ? 1.05 : D == 128 ? 0.95 : 0.65;
@@ -1402,14 +1403,18 @@ static PrefillPlan prefill_plan(bool f32, int B, int T, int H, int K, int D, int
       const int64_t rounds = (blocks + cus - 1) / cus;
       double us = (tiles + 2.5) * alone;  // the longest block
       if (rounds > 1 && rounds * per_block * shared > us) us = rounds * per_block * shared;
-      if (split1) us += 3.0 + 2.0 * split1 * H * B * BM * D * sizeof(float) / 4e6;
+      const double partials = split1 ? 3.0 + 2.0 * split1 * H * B * BM * D * sizeof(float) / 4e6 : 0.0;
+      us += partials;
       // (splitting has to be worth more than the model's error)
       const bool first = c == 1 && hpb == most_heads;
       if (first || us < (c > 1 && best.nsplit == 1 ? 0.8 : 0.95) * best_us) {
         best = PrefillPlan{c, tiles, hpb};
         best_us = us;
       }
+      // with the CUs full, blocks and partials only grow with the parts, and the time with them
+      open = open || rounds == 1 || blocks * per_block * shared / cus + partials < 0.95 * best_us;
     }
+    if (!open) break;
   }
   if (best.nsplit > 1) best.nsplit = (longest + best.tiles - 1) / best.tiles;
   return best;
