@@ -626,10 +626,12 @@ static int launch_prefill_combine(const PrefillParams& p, int BM, int BN, hipStr
 template <typename T, int D, bool SPLIT>
 static int launch_prefill_s(PrefillParams p, hipStream_t s) {
   using TL = Tile<D>;
+  constexpr int kThreeLds = 48 * 1024;  // three blocks of it fit a CU's 160 KB, four do not
   static bool attr_set = false;  // raise the dynamic LDS limit once per kernel
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_kernel<T, D, SPLIT>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS_BYTES) != hipSuccess)
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            TL::LDS_BYTES > kThreeLds ? TL::LDS_BYTES : kThreeLds) != hipSuccess)
       return set_error("forge_attn_prefill: cannot reserve the LDS the kernel needs");
     attr_set = true;
   }
@@ -637,7 +639,19 @@ static int launch_prefill_s(PrefillParams p, hipStream_t s) {
   p.xcd_map = ((int64_t)p.B * p.K * p.nsplit) % 8 == 0 ? 1 : 0;
   const int64_t blocks = (int64_t)p.nqt * p.H * p.B * p.nsplit;
   if (blocks > 0x7fffffff) return set_error("grid too large");
-  hipLaunchKernelGGL((prefill_kernel<T, D, SPLIT>), dim3((unsigned)blocks), dim3(TL::WAVES * 64), TL::LDS_BYTES, s, p);
+  int lds = TL::LDS_BYTES;
+  if constexpr (D == 64 && !SPLIT) {
+    // A CU holds four blocks. A launch of three to four per CU would then start them all at once, on
+    // CUs that cannot even out their blocks' lengths afterwards; with three per CU the last ones go to
+    // the CUs that finish first. That pays with documents, whose blocks differ most, and otherwise
+    // while few CUs get a fourth block (three against four, us; 16 q / 16 KV heads, 12 / 4 the 792s):
+    // documents of 1,250 tokens, 896 blocks 47.5 / 48.8, 1,024 blocks 48.0 / 50.1, of 300 tokens 27.7 /
+    // 28.7 and 32.7 / 32.7; whole prompts, 792 blocks 39.6 / 40.5, 896 49.6 / 50.9, 880 39.9 / 37.4, 1,024
+    // 57.4 / 54.0; window 512, 792 blocks 29.1 / 29.4, 900 34.7 / 32.7.
+    const int64_t cus = device_cus();
+    if (blocks > 3 * cus && blocks * 4 <= (p.doc_lo ? 16 : 13) * cus) lds = kThreeLds;
+  }
+  hipLaunchKernelGGL((prefill_kernel<T, D, SPLIT>), dim3((unsigned)blocks), dim3(TL::WAVES * 64), lds, s, p);
   return check_launch();
 }
 

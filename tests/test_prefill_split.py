@@ -174,3 +174,23 @@ def test_without_memory_for_the_partials_the_launch_is_not_split(monkeypatch, na
         vc.data_ptr(), *kc.stride()[:3], offset, 0, scale_of(D), want.data_ptr(), *want.stride()[:3],
         torch.cuda.current_stream().cuda_stream), "forge_attn_prefill")
     assert torch.equal(got, want) and not torch.equal(got, split)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("B,T,window,docs", [(5, 1900, 0, True), (6, 1400, 512, False)])
+def test_rows_do_not_depend_on_the_blocks_a_cu_holds(B, T, window, docs):
+    """Head dim 64 with 900 and 792 blocks (three per CU): every row as in a call of its own."""
+    from sleuth_amd import ops
+
+    H, K, D = 12, 4, 64
+    g = gen(990)
+    q = randn(g, B, T, H, D, dtype=torch.bfloat16).transpose(1, 2).to(DEV)
+    k, v = (randn(g, B, K, T, D, dtype=torch.bfloat16).to(DEV) for _ in range(2))
+    starts = torch.tensor([0] * 700 + [700] * (T - 700), dtype=torch.int32, device=DEV)[None].expand(B, T).contiguous()
+    call = lambda r: ops.attn_prefill(q[r], k[r], v[r], scale=scale_of(D), window=window,  # noqa: E731
+                                      doc_start=starts[r] if docs else None)
+    got = call(slice(None))
+    assert docs or _bytes(1, T, H, K, D, 0, window) == 0     # a row alone is not split
+    for b in range(B):
+        assert torch.equal(call(slice(b, b + 1)), got[b:b + 1])
