@@ -15,7 +15,7 @@ of head_norm_rope + cache.update + SDPA):
       T > 16, bf16/fp16, head dim 64-512:     forge_kv_append, then forge_attn_prefill
                         (MFMA flash) with the q norm + RoPE in its q load;
       T > 16, fp32, head dim 32-128:          forge_kv_append, then forge_attn_prefill_f32
-                        (the same on fp32 MFMA);
+                        (the same on fp32 MFMA; from 49 keys on);
       otherwise         forge_attn_decode_append: the cache write and the split-K
                         attention (decode, verify, static steps, other head sizes)
                         in one launch, the q norm + RoPE fused into the q load.
@@ -415,7 +415,7 @@ class Attention(nn.Module):
             self.last_path = "hip-prefill" if docs is None else "hip-prefill-docs"
             return ops.attn_prefill(q, kc, vc, scale=self.scale, offset=offset, window=self.window,
                                     doc_start=docs, check_doc_start=False, **q_args)
-        if T > DECODE_MAX_T and offset is not None and docs is None and \
+        if T > DECODE_MAX_T and offset is not None and docs is None and offset + T >= ops.PREFILL_F32_MIN_KEYS and \
                 (q_args["cos"] is None or q_args["cos"].dim() == 2) and \
                 ops.prefill_f32_supported(q, q_args["cos"], q_args["sin"], q_args.get("q_weight"), kc, offset):
             ops.kv_append(k, v, kc, vc, norm_v=norm_v, **pos_kw, **k_args)

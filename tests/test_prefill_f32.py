@@ -140,8 +140,8 @@ def test_module_takes_unaligned_gains_and_wide_slabs_the_split_k_way(monkeypatch
     cfg = ModelConfig(vocab_size=16, d_model=128, n_layers=1, n_heads=4, n_kv_heads=2, qk_norm=True, max_seq_len=64)
     a = Attention(cfg, 0).to(DEV).eval()
     a.q_norm.weight.data.copy_(torch.linspace(0.8, 1.2, 32))
-    x = torch.randn(1, 20, 128, device=DEV)
-    cos, sin = (t[:20].to(DEV) for t in tables(32, 64, 1e4))
+    x = torch.randn(1, 60, 128, device=DEV)
+    cos, sin = (t[:60].to(DEV) for t in tables(32, 64, 1e4))
     calls, fn = [], ops.attn_prefill_f32
     monkeypatch.setattr(ops, "attn_prefill_f32", lambda *a, **kw: calls.append(1) or fn(*a, **kw))
 
@@ -150,16 +150,43 @@ def test_module_takes_unaligned_gains_and_wide_slabs_the_split_k_way(monkeypatch
         with torch.no_grad():
             return a(x, cos, sin, cache), cache.k[0].clone(), len(calls)
 
-    cache = HostKVCache([(2, 32)], 1, 20, DEV, F32)
+    cache = HostKVCache([(2, 32)], 1, 60, DEV, F32)
     want = run()
     if what == "gain":
         flat = torch.empty(33, device=DEV)
         flat[1:] = a.q_norm.weight.detach()
         a.q_norm.weight.data = flat[1:]
     else:
-        row = 2 ** 21       # floats: 21 rows span 176 MB, 276 of them 2.3 GB
+        row = 2 ** 21       # floats: 61 rows span 0.5 GB, 316 of them 2.7 GB
         for kv in (cache.k, cache.v):
-            kv[0] = torch.zeros(20 * row, device=DEV).as_strided((1, 2, 20, 32), (64, 32, row, 1))
+            kv[0] = torch.zeros(60 * row, device=DEV).as_strided((1, 2, 60, 32), (64, 32, row, 1))
     got = run()
     assert (want[2], got[2]) == (1, 0)
     assert torch.equal(want[1], got[1]) and max_abs(want[0], got[0]) <= 1e-5   # fp32 sums in another order
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("T,offset,taken", [(17, 0, 0), (20, 28, 0), (48, 0, 0), (49, 0, 1), (17, 32, 1)])
+def test_module_keeps_few_keys_on_the_split_k_path(monkeypatch, T, offset, taken):
+    """Up to 48 keys, where the matrix-core kernel's sums are no more exact: the split-K call's own bits."""
+    from sleuth_amd import ops
+    from sleuth_amd.attention import Attention
+    from sleuth_amd.config import ModelConfig
+    from sleuth_amd.kv_cache import KVCache
+
+    torch.manual_seed(5)
+    cfg = ModelConfig(vocab_size=16, d_model=128, n_layers=1, n_heads=4, n_kv_heads=2, qk_norm=True, max_seq_len=64)
+    a = Attention(cfg, 0).to(DEV).eval()
+    x = torch.randn(1, T, 128, device=DEV)
+    cos, sin = (t[offset:offset + T].to(DEV) for t in tables(32, 64, 1e4))
+    outs, calls, fn = [], [], ops.attn_prefill_f32
+    monkeypatch.setattr(ops, "attn_prefill_f32", lambda *a, **kw: calls.append(1) or fn(*a, **kw))
+    for least in (ops.PREFILL_F32_MIN_KEYS, 1000):
+        monkeypatch.setattr(ops, "PREFILL_F32_MIN_KEYS", least)
+        cache = KVCache([(2, 32)], 1, 64, DEV, F32)
+        cache.pos = offset
+        with torch.no_grad():
+            outs.append(a(x, cos, sin, cache))
+    assert len(calls) == taken
+    assert max_abs(*outs) <= 1e-5 and (taken or torch.equal(*outs))   # fp32 sums in another order, or the same
