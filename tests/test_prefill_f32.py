@@ -18,22 +18,27 @@ F32 = torch.float32
 
 
 def test_rejections():
+    """Each bad argument alone, everything else in order, is named by the error."""
     lib = _lib.lib()
     size = lib.forge_attn_prefill_f32_workspace_bytes
     assert size(1, 20, 8, 4, 32, 4000, 0) > 0 and size(8, 2048, 8, 4, 32, 0, 0) == 0
     assert size(1, 20, 8, 4, 256, 4000, 0) == 0 and size(1, 20, 8, 3, 32, 4000, 0) == 0
-    ok = dict(D=32, sks=32, q=4096, offset=0)
+    ok = dict(D=32, K=4, q=4096, w=None, sqt=256, sks=32, offset=0, window=0, out=4096, ws=None)
 
     def call(**kw):
         a = {**ok, **kw}
-        return lib.forge_attn_prefill_f32(1, 20, 8, 4, a["D"], a["q"], 0, 32, 256, None, 1e-6, 0, None, None, 0, 4096,
-                                          4096, 0, 32, a["sks"], a["offset"], 0, 1.0, None, 0, 256, 32, None, 0, None)
+        return lib.forge_attn_prefill_f32(1, 20, 8, a["K"], a["D"], a["q"], 0, 32, a["sqt"], a["w"], 1e-6, 0, None, None, 0,
+                                          4096, 4096, 0, 32, a["sks"], a["offset"], a["window"], 1.0, a["out"], 0, 256, 32,
+                                          a["ws"], 0, None)
 
-    for kw in (dict(), dict(D=256), dict(q=4100), dict(sks=34), dict(offset=-1), dict(offset=2 ** 27)):
-        assert call(**kw) < 0     # (the first: no output)
-    lib.forge_attn_prefill_ws     # bound
-    assert lib.forge_head_norm_rope(_lib.F32, None, None, 0, 0, 0, 2, 0, 0, 0, 0, 0, 0, None, 0.0, 0, None, None, 0, 0,
-                                    None) < 0
+    for kw, why in ((dict(out=None), "null"), (dict(q=None), "null"), (dict(D=256), "head dim"), (dict(K=3), "multiple of the KV"),
+                    (dict(q=4100), "16-byte aligned"), (dict(out=4104), "16-byte aligned"), (dict(w=4100), "16-byte aligned"),
+                    (dict(ws=4104), "16-byte aligned"), (dict(sks=34), "multiples of 16 bytes"),
+                    (dict(sqt=258), "multiples of 16 bytes"), (dict(offset=-1), "offset"), (dict(window=-1), "window"),
+                    (dict(offset=2 ** 31 - 276), "31 bits"), (dict(sks=28), "2^31 bytes"), (dict(offset=2 ** 24), "2^31 bytes"),
+                    (dict(sks=2 ** 21), "stride too large"), (dict(sks=2 ** 20, offset=300), "2^31 bytes")):
+        assert call(**kw) < 0, kw
+        assert why in lib.forge_last_error().decode(), (kw, lib.forge_last_error())
 
 
 def test_what_it_supports():
