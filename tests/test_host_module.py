@@ -34,17 +34,34 @@ def test_declines_what_is_no_plain_gpu_tensor():
         h.kv_append(t, i)
 
 
-def _both(monkeypatch, call):
-    """call() the Python way and the native way: results, or the errors' types and texts."""
-    out = []
+class Recorder:
+    """The native module, with what its functions returned: taken (a result or a status) or declined."""
+
+    def __init__(self):
+        self.taken = []
+
+    def __getattr__(self, name):
+        fn = getattr(_lib.host(), name)
+
+        def call(*a):
+            r = fn(*a)
+            self.taken.append(r is not None)
+            return r
+        return call
+
+
+def _both(monkeypatch, call, taken=None):
+    """call() the Python way and the native way: results, or the errors' types and texts. taken: whether the
+    native functions take the calls, one value each."""
+    out, rec = [], Recorder()
     for native in (False, True):
         with monkeypatch.context() as m:
-            if not native:
-                m.setattr(ops, "host", lambda: DECLINE)
+            m.setattr(ops, "host", (lambda: rec) if native else lambda: DECLINE)
             try:
                 out.append(call())
             except Exception as e:   # compared, not swallowed
                 out.append((type(e), str(e)))
+    assert taken is None or rec.taken == taken, (rec.taken, taken)
     return out
 
 
@@ -66,21 +83,22 @@ def test_decode_append_equals_the_python_way(monkeypatch, dtype, where, T, H, K,
     q, k, v = (t.to(DEV) for t in qkv_proj_views(g, B, T, H, K, D, dtype))
     cache = randn(g, 2, B, L, K, D, dtype=dtype).transpose(2, 3).to(DEV)     # [2, B, K, L, D], heads inside the rows
     cos, sin = (t[:B * T].view(B, T, D).to(DEV) for t in tables(D, 64, 1e4))
-    base = 250 if where == "pos" else 0
     kw = {"pos": dict(pos=250), "pos_dev": dict(pos_dev=torch.tensor([250], device=DEV)),
           "row_pos": dict(row_pos=torch.tensor([250, 3], dtype=torch.int32, device=DEV)), "none": {}}[where]
     w = torch.linspace(0.9, 1.1, D, device=DEV)
-    for tab, gain, norm in ((dict(cos=cos, sin=sin), w, True), (dict(cos=cos[0], sin=sin[0]), w.to(dtype), True),
-                            ({}, None, False), (dict(cos=cos[:, :, ::1].double(), sin=sin.double()), None, True),
-                            (dict(cos=cos), w, True), (dict(cos=cos[:, :1], sin=sin[:, :1]), w, True)):
+    f32 = dtype == torch.float32
+    # the native way takes what needs no conversion (once the stream has its workspace) and leaves the rest
+    for tab, gain, norm, plain in ((dict(cos=cos, sin=sin), w, True, True), (dict(cos=cos[0], sin=sin[0]), w.to(dtype), True, f32),
+                                   ({}, None, False, True), (dict(cos=cos[:, :, ::1].double(), sin=sin.double()), None, True, False),
+                                   (dict(cos=cos), w, True, False),
+                                   (dict(cos=cos[:, :1], sin=sin[:, :1]), w, True, T == 1)):
         def call():
             kc, vc = cache[0].clone(memory_format=torch.preserve_format), cache[1].clone(memory_format=torch.preserve_format)
             y = ops.attn_decode_append(q, k, v, kc, vc, scale=0.1, window=window, q_weight=gain, k_weight=gain, norm_q=norm,
                                        norm_k=norm, norm_v=norm, **tab, **kw)
             return [y, kc, vc]
-        a, b = _both(monkeypatch, call)
+        a, b = _both(monkeypatch, call, [plain])
         assert _equal(a, b), (a, b)
-    assert base >= 0
 
 
 @pytest.mark.gpu
@@ -94,17 +112,18 @@ def test_prefill_and_append_equal_the_python_way(monkeypatch, dtype):
     cos, sin = (t[100:100 + T].to(DEV) for t in tables(D, 200, 1e4))
     w = torch.linspace(0.9, 1.1, D, device=DEV)
     fn = ops.attn_prefill_f32 if dtype == torch.float32 else ops.attn_prefill
-    for off, kk, extra in ((100, k, {}), (100, k.to(torch.float16), {}), (190, k, {}), (100, k[..., :32], {}),
-                           (100, k, dict(window=30)), (0, k, dict(cos=cos, sin=sin)), (-1, k, {})):
+    for off, kk, extra, taken in ((100, k, {}, [True, True]), (100, k.to(torch.float16), {}, [False, True]),
+                                  (190, k, {}, [True]), (100, k[..., :32], {}, [False]), (100, k, dict(window=30), [True, True]),
+                                  (0, k, dict(cos=cos, sin=sin), [True, True]), (-1, k, {}, [True])):
         def call():
             kc, vc = kc0.clone(), vc0.clone()
             ops.kv_append(kk, v, kc, vc, pos=off, k_weight=w, norm_k=True, cos=cos, sin=sin)
             y = fn(q, kc, vc, scale=0.2, offset=off, q_weight=w, norm_q=True, **extra)
             return [y, kc, vc]
-        a, b = _both(monkeypatch, call)
+        a, b = _both(monkeypatch, call, taken)
         assert _equal(a, b), (off, extra, a, b)
     for off in (161, 2 ** 31, 2 ** 63 - 20):     # past the keys' end, also where the end wraps
-        a, b = _both(monkeypatch, lambda: fn(q, kc0, vc0, scale=0.2, offset=off))
+        a, b = _both(monkeypatch, lambda: fn(q, kc0, vc0, scale=0.2, offset=off), [False])
         assert a == b and a[0] is ValueError, (off, a, b)
 
 

@@ -194,3 +194,31 @@ def test_rows_do_not_depend_on_the_blocks_a_cu_holds(B, T, window, docs):
     assert docs or _bytes(1, T, H, K, D, 0, window) == 0     # a row alone is not split
     for b in range(B):
         assert torch.equal(call(slice(b, b + 1)), got[b:b + 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("docs", [False, True])
+def test_entry_points_without_a_workspace(docs):
+    """forge_attn_prefill at a shape that the call with a workspace splits, and forge_attn_prefill_docs, as a
+    C caller makes them, against the oracle."""
+    B, T, H, K, D, offset = 1, 200, 8, 4, 128, 0 if docs else 2500
+    S = offset + T
+    g = gen(1000)
+    q = randn(g, B, T, H, D, dtype=torch.bfloat16).transpose(1, 2)
+    k, v = (randn(g, B, K, S, D, dtype=torch.bfloat16) for _ in range(2))
+    starts = torch.tensor([0] * 70 + [70] * 130, dtype=torch.int32)[None].contiguous()
+    same = (starts[:, :, None] == starts[:, None, :])[:, None] if docs else None
+    ref = oracle.sdpa(q.float(), k.float(), v.float(), offset, 0, scale_of(D), same_doc=same)
+    dq, dk, dv, ds = (t.to(DEV) for t in (q, k, v, starts))
+    out = torch.empty(B, T, H, D, dtype=torch.bfloat16, device=DEV)
+    args = [_lib.BF16, B, T, H, K, D, dq.data_ptr(), *dq.stride()[:3], None, 1e-6, 0, None, None, 0, dk.data_ptr(), dv.data_ptr(),
+            *dk.stride()[:3], offset, 0, scale_of(D)]
+    stream = torch.cuda.current_stream().cuda_stream
+    if docs:
+        st = _lib.lib().forge_attn_prefill_docs(*args, ds.data_ptr(), T, out.data_ptr(), *out.stride()[:3], stream)
+    else:
+        assert _bytes(B, T, H, K, D, offset) > 0
+        st = _lib.lib().forge_attn_prefill(*args, out.data_ptr(), *out.stride()[:3], stream)
+    assert st == 0
+    assert max_abs(out.cpu().transpose(1, 2), ref) <= tol(torch.bfloat16)
