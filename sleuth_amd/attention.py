@@ -164,13 +164,22 @@ def plain_module(m: nn.Module, cls: type) -> bool:
     in place of forward on the module or its class, no module.compile(), and nn.Module's own call.
     Only such modules' work may be done inside a fused launch."""
     return type(m) is cls and not m._forward_hooks and not m._forward_pre_hooks and "forward" not in m.__dict__ and \
-        m._compiled_call_impl is None and _defined_in(cls.forward, cls.__module__) and \
-        _defined_in(cls.__call__, nn.Module.__module__) and _defined_in(cls._call_impl, nn.Module.__module__)
+        m._compiled_call_impl is None and \
+        (_OWN.get(cls) == (cls.forward, cls.__call__, cls._call_impl) or _runs_own_code(cls))
 
 
-def _defined_in(fn, module: str) -> bool:
-    """fn is a function written in that module (what a replacement, wrapped or not, is not)."""
-    return getattr(fn, "__globals__", None) is sys.modules[module].__dict__
+_OWN: dict[type, tuple] = {}   # class -> the functions that _runs_own_code last found to be its own
+
+
+def _runs_own_code(cls: type) -> bool:
+    """cls.forward and its call are the functions written in cls's and nn.Module's own modules (what a
+    replacement, wrapped or not, is not)."""
+    own = (cls.forward, cls.__call__, cls._call_impl)
+    for fn, module in zip(own, (cls.__module__, nn.Module.__module__, nn.Module.__module__)):
+        if getattr(fn, "__globals__", None) is not sys.modules[module].__dict__:
+            return False
+    _OWN[cls] = own
+    return True
 
 
 def no_global_hooks() -> bool:

@@ -455,12 +455,18 @@ def prefill_f32_supported(q: torch.Tensor, cos: torch.Tensor | None = None, sin:
     """attn_prefill_f32 takes this q, these tables and this gain (16-byte aligned rows; attn_decode takes
     any), and keys k [B,K,S,D] of a slab whose rows up to a tile past the last query lie within 2^31
     bytes (attn_decode: the cache's own rows)."""
-    if q.dtype != torch.float32 or q.shape[-1] not in PREFILL_F32_HEAD_DIMS:
+    _, _, T, D = q.shape
+    if q.dtype is not torch.float32 or D not in PREFILL_F32_HEAD_DIMS:
         return False
-    if k is not None and (k.stride(2) < k.shape[3] or k.stride(2) * 4 * (offset + q.shape[2] + 256) >= 2 ** 31):
+    if k is not None and not D <= k.stride(2) < 2 ** 29 / (offset + T + 256):
         return False
-    return all(t is None or (t.data_ptr() % 16 == 0 and t.dtype == torch.float32 and t.stride(-1) == 1 and
-                             all(n % 4 == 0 for n in t.stride()[:-1])) for t in (cos, sin, q_weight))
+    for t in (cos, sin, q_weight):
+        if t is None:
+            continue
+        *rows, last = t.stride()
+        if last != 1 or t.dtype is not torch.float32 or t.data_ptr() % 16 or (rows and (rows[0] % 4 or rows[-1] % 4)):
+            return False   # (a gain, or tables of up to three dimensions)
+    return True
 
 
 def attn_prefill_f32(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float, offset: int = 0,
