@@ -345,10 +345,18 @@ void prefill_kernel(PrefillParams p) {
         lds_dma16(vt_base + off, (unsigned)(lo + (lv ^ (swz_v<D>(r0) << 4))), vdst + i * 1024);
       }
     } else {
-      // last, partial tile: rows past the end are masked; they read row S - 1 instead (the
-      // wave's row is clamped first, so a lane's offset, which is unsigned, stays at least 0)
+      // last, partial tile: rows past the end are masked; they read row S - 1 instead (at head dim 256
+      // the wave's row is clamped first, so a lane's offset, which is unsigned, stays at least 0)
 #pragma unroll
       for (int i = 0; i < TL::LOADS; ++i) {
+        if constexpr (KEEP) {
+          const int row = RL * (wave * TL::LOADS + i) + ld_row, pch = lane % TL::NCH;
+          const int64_t key = key0 + row < S ? key0 + row : S - 1;
+          const unsigned rb = (unsigned)((key - key0) * p.sks * 2);
+          lds_dma16(kgb + key0 * p.sks * 2, rb + ((pch ^ swz_k<D>(row)) << 4), kdst + i * 1024);
+          lds_dma16(vgb + key0 * p.sks * 2, rb + ((pch ^ swz_v<D>(row)) << 4), vdst + i * 1024);
+          continue;
+        }
         const int r0 = RL * (wave * TL::LOADS + i);
         const int64_t key = key0 + r0 < S ? key0 + r0 : S - 1;
         const int64_t off = key * p.sks * 2;
