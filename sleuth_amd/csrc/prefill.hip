@@ -32,6 +32,8 @@
 // Q gets the per-head RMSNorm and RoPE in its load (fp32 math, one rounding), like
 // fused_ops._head_kernel (fused_ops.py:53-85); K and V come from the cache, where
 // forge_kv_append wrote them already normalised.
+#include <limits.h>
+
 #include "common.h"
 #include "forge_internal.h"
 
@@ -1405,6 +1407,25 @@ struct PrefillPlan {
 };
 constexpr int kMaxParts = 32;
 
+// Heads per block of an unsplit launch at head dim 512, from the time of its blocks: a tile of four heads
+// takes 2.55 us and one of two heads 2.1, what a block does besides (mostly its q prologue) as long as 13
+// and 7.6 tiles, and the last, partial round of blocks (the lightest: heavy ones go first) between its
+// lightest block and a mean one. Against both forms timed at 33 shapes of 17 to 4,096 queries, one to
+// eight rows, the pick is the faster one or within 1% of it (four / two heads, us): 8 x 130 52 / 49, 3 x 435
+// 76 / 65, 8 x 300 (8 q / 2 KV heads) 64 / 57, 6 x 435 108 / 112, 3 x 700 99 / 117, 2,000 199 / 179, 2,500 241 / 282.
+static int wide_heads(int B, int H, int nqt, int longest, int lightest, int64_t work, int64_t cus) {
+  double us[2];
+  for (int i = 0; i < 2; ++i) {
+    const int heads = i ? 2 : 4;
+    const double tile = i ? 2.1 : 2.55, prologue = i ? 7.6 : 13.0;
+    const int64_t blocks = (int64_t)nqt * (H / heads) * B, rest = blocks % cus;
+    const double mean = (double)work / nqt, last = rest ? lightest + prologue + (mean - lightest) * rest / cus : 0.0;
+    const double load = (blocks / cus) * (mean + prologue) + last;
+    us[i] = 5.0 + tile * (load > longest + prologue ? load : longest + prologue);
+  }
+  return us[1] < 0.95 * us[0] ? 2 : 4;  // (by more than the model's error)
+}
+
 // Picks the split with the least modelled time. Measured on calls of 1 to 32 parts (graph
 // replays, one box; the model is within 15% of each): a tile takes `alone` us in a block that has
 // its CU to itself and `shared` us of a CU that holds several (head dims 64 to 256), a block's q
@@ -1415,10 +1436,8 @@ constexpr int kMaxParts = 32;
 // 25 / 20 / 16 / 15 / 17; T 1024 at 15,360: 288 / 170 / 143 / 162 / 191; a whole prompt of
 // 2,048: 44 / 49 / 53 / 71 / 115 (not split). Head dim 256 (8 q / 4 KV), T 512 at 8,000: 352 /
 // 186 / 105 / 69 / 86.
-// At head dim 512 the same model picks the heads that share a block and its K/V tiles: four
-// take 2.55 us a tile where two take 2.1 us, so four win once the blocks fill the CUs (16 q / 1 KV
-// head, a prompt of 4,096: 384 us against 631; T 512 at 8,000, split: 211 against 301), two on
-// short calls (a prompt of 1,024: 80 us against 100).
+// At head dim 512 the same model picks the heads that share a split launch's blocks and their K/V
+// tiles (T 512 at 8,000: 211 us with four, 301 with two), and wide_heads an unsplit one's.
 static PrefillPlan prefill_plan(bool f32, int B, int T, int H, int K, int D, int64_t offset, int window,
                                 int max_parts) {
   const bool wide = D == 512;
@@ -1430,11 +1449,15 @@ static PrefillPlan prefill_plan(bool f32, int B, int T, int H, int K, int D, int
   const int nqt = (T + BM - 1) / BM;
   if ((int64_t)nqt * (H / most_heads) * B >= 4 * cus)  // several rounds of blocks already
     return PrefillPlan{1, 0, most_heads};
-  int longest = 0;
+  int longest = 0, lightest = INT_MAX;
+  int64_t work = 0;
   for (int qt = 0; qt < nqt; ++qt) {
     int begin, end;
     tile_span(offset, T, window, 0, qt, BM, BN, begin, end);
-    longest = end - begin + 1 > longest ? end - begin + 1 : longest;
+    const int n = end - begin + 1;
+    longest = n > longest ? n : longest;
+    lightest = n < lightest ? n : lightest;
+    work += n;
   }
   PrefillPlan best{1, longest, most_heads};
   double best_us = 0.0;
@@ -1478,6 +1501,7 @@ static PrefillPlan prefill_plan(bool f32, int B, int T, int H, int K, int D, int
     if (!open) break;
   }
   if (best.nsplit > 1) best.nsplit = (longest + best.tiles - 1) / best.tiles;
+  else if (most_heads == 4) best.heads_per_block = wide_heads(B, H, nqt, longest, lightest, work, cus);
   return best;
 }
 
