@@ -12,7 +12,7 @@ of head_norm_rope + cache.update + SDPA):
       k norm + RoPE (+ v norm), written into the cache at pos / pos_t / per-row
       lengths (with partial RoPE, norm and RoPE run in torch as the reference's eager
       code does, and the kernels take q and k as they are), then attention:
-      T > 16, bf16/fp16, head dim 64-512:     forge_kv_append, then forge_attn_prefill
+      T > 16, bf16/fp16, head dim 64-512:     forge_kv_append, then forge_attn_prefill_ws
                         (MFMA flash) with the q norm + RoPE in its q load;
       T > 16, fp32, head dim 32-128:          forge_kv_append, then forge_attn_prefill_f32
                         (the same on fp32 MFMA; from 49 keys on);
@@ -21,7 +21,7 @@ of head_norm_rope + cache.update + SDPA):
                         in one launch, the q norm + RoPE fused into the q load.
       A boolean document mask (transformer.py:271-275) over a whole window (no cache,
       T > 16, the prefill dtypes and head dims) whose documents are contiguous runs goes
-      to forge_attn_prefill_docs, which takes each query's first visible key.
+      to forge_attn_prefill_ws too, which takes each query's first visible key.
     The output comes back as [B, T, H, hd], the layout o_proj reads.
   * torch (CPU, training, FlexAttention block masks and other document masks, the
     pattern tap, or SLEUTH_AMD_NO_HIP=1): the reference's eager code, unchanged in meaning;
@@ -104,7 +104,7 @@ _DOC_STARTS: dict = {}   # the last mask's doc starts: one mask serves every lay
 def _doc_starts(same_doc, B: int, T: int) -> torch.Tensor | None:
     """The reference's document mask (transformer.py:271-275: [B or 1, 1, T, T] bool, True
     where query and key are in one document) as each query's first visible key, [B, T]
-    int32, for forge_attn_prefill_docs. None where it is not such a mask, or where a query's
+    int32, for forge_attn_prefill_ws. None where it is not such a mask, or where a query's
     visible keys (mask and causal) are not one run ending at the query itself, i.e. its
     document is not a contiguous run of positions."""
     m = same_doc

@@ -16,14 +16,13 @@
 // once and the norm adds one barrier: a pass over x of its own, with W's loads only in flight, took
 // 1.3 us more at K 1,024 (5.2 us against 3.9 without the norm; now 3.7 against 2.7).
 //
-// Measured (bf16, graph replays of the call alone on one W, which the 256 MB MALL then holds up to
-// that size; 1 / 5 / 16 rows, us; in brackets the form before, one box each; on W of its own per call,
-// as in a model, see LinRule below): 4096 x 1024 with norm 3.7 / 3.9 / 4.4 (5.2 / 5.4 / 6.2), hipBLASLt's product alone
-// 6.3; 1024 x 2048 with residual 3.8 / 4.1 / 5.2 (4.3 / 4.4 / 5.2), hipBLASLt 8.2; 3072 x 1024 SwiGLU
-// with norm 4.7 / 4.9 / 5.4 (6.9 / 7.3 / 8.2); 1024 x 3072 with residual 4.9 / 5.4 / 6.9 (6.4 / 6.7 /
-// 7.8), hipBLASLt 9.4; 8192 x 1024 with norm 5.0 / 5.3 / 6.2 (7.1 / 7.4 / 8.8), hipBLASLt 6.7; 4096 x
-// 14336 with residual 19.6 / 20.9 / 26.7 (27.4 / 29.1 / 32.5; 6.0 TB/s at one row); 32768 x 4096 with norm
-// 55 / 55 / 68 (60 / 63 / 83), hipBLASLt 62; 6144 x 4096 with norm 16.1 / 18.3 / 25.1 (17.0 / 17.8 / 23.5).
+// Measured: bf16, graph replays of the call alone on one W, which the 256 MB MALL then holds; 1 / 5 / 16
+// rows, us; in brackets the form before, one box each. (A W of its own per call, as in a model: LinRule
+// below. Launched one by one on idle CUs: 1 to 2 us more.) 4096 x 1024 with norm 3.7 / 3.9 / 4.4 (5.2 /
+// 5.4 / 6.2), hipBLASLt's product alone 6.3; 1024 x 2048 with residual 3.8 / 4.1 / 5.2 (4.3 / 4.4 / 5.2),
+// hipBLASLt 8.2; 3072 x 1024 SwiGLU with norm 4.7 / 4.9 / 5.4 (6.9 / 7.3 / 8.2); 1024 x 3072 with residual
+// 4.9 / 5.4 / 6.9 (6.4 / 6.7 / 7.8), hipBLASLt 9.4; 8192 x 1024 with norm 5.0 / 5.3 / 6.2 (7.1 / 7.4 / 8.8),
+// hipBLASLt 6.7; 6144 x 4096 with norm 16.1 / 18.3 / 25.1 (17.0 / 17.8 / 23.5; 16 rows go to torch).
 // A four-layer model's decode step (d 1024, hidden 3072; GraphDecoder), with the norms, residual sums
 // and SwiGLU product in these launches: 175 us (206 the form before, 411 with torch's calls).
 #include "common.h"
@@ -71,7 +70,7 @@ constexpr int kLinWaves = 8;
 constexpr int kLinRows = 16;   // rows of x
 constexpr int kLinCols = 16;   // output columns of a tile
 // Outputs from which a block takes two tiles: x's rows are then read half as often, and two blocks per
-// CU are left. 32768 x 4096 with norm at 5 rows 54 us against 63 with one tile, at 16 rows 66 against 83.
+// CU are left. On one W: 32768 x 4096 with norm at 5 rows 54 us against 63 with one tile, at 16 rows 66 against 83.
 constexpr int kLinWideN = 16384;
 
 // What the kernel does to x's rows first.

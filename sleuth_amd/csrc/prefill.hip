@@ -13,7 +13,7 @@
 //     the stages, and two blocks share a CU so that its SIMDs interleave two independent
 //     waves. At head dim 256 (128 accumulator and 64 Q^T registers of the 256 a wave may use)
 //     that needs the load and LDS addresses to come from one register each: two waves per SIMD
-//     take 284 us where one took 378 us (4 x 4096 causal, 8 q / 4 KV heads; 386 -> 514 TFLOP/s).
+//     take 311 us where one took 428 us (4 x 4096 causal, 8 q / 4 KV heads; 642 -> 884 TFLOP/s).
 //   * Scores are computed transposed, S^T = K . Q^T: K is the MFMA A operand (128-bit
 //     LDS reads), Q^T the B operand held in registers for the whole block. In the 32x32
 //     accumulator layout each lane then owns ONE query (column l % 32) and 16 keys of a
@@ -688,7 +688,7 @@ static int launch_prefill_d(const PrefillParams& p, hipStream_t s) {
 // channel c with c ^ 256, so each lane also loads its channels' partners.
 // Eight waves (four heads, two waves per SIMD) against four (two heads, one per SIMD): half the
 // tile loads per FLOP, and one wave's softmax runs beside the other's MFMAs: 16 q / 1 KV head,
-// 4,096 causal: 384 us against 631 us (716 against 435 TFLOP/s). It needs the whole 256-register
+// 4,096 causal: 432 us against 606 us (636 against 454 TFLOP/s). It needs the whole 256-register
 // budget of two waves per SIMD, hence the load and LDS addresses made from one register each and
 // the K operands held two steps ahead only: every spill reload in the tile loop would wait for
 // the tile loads in flight.
@@ -700,7 +700,7 @@ template <int NW> struct WideTile {
   static constexpr int NCH = D / 8;
   static constexpr int ROWB = 2 * D;
   static constexpr int TILEB = BN * ROWB;                // 32 KB
-  static constexpr int LOADS = TILEB / (WAVES * 1024);   // 8
+  static constexpr int LOADS = TILEB / (WAVES * 1024);   // 8 with four waves, 4 with eight
   static constexpr int STAGES = 2;
   static constexpr int PART_BYTES = WAVES * 64 * 16 * 4; // the waves' partial scores
   static constexpr int LDS_BYTES = STAGES * 2 * TILEB + PART_BYTES;
@@ -715,7 +715,7 @@ void prefill_wide_kernel(PrefillParams p) {
   constexpr int BN = TL::BN;
   // SPLIT waves share a head, each with D / SPLIT channels; the block takes WAVES / SPLIT heads
   // of one KV head, so each K/V tile is loaded once for all of them
-  static_assert(SPLIT == 4 || SPLIT == 2, "four quarter-slices of one head, or two halves of two");
+  static_assert(SPLIT == 4 || SPLIT == 2, "quarters of one head, or halves of two (four waves) or four (eight)");
   constexpr int HPB = TL::WAVES / SPLIT;     // heads per block
   constexpr int CW = D / SPLIT;              // channels per wave
   constexpr int CCH = CW / 8;                // 16-byte chunks per wave slice
@@ -991,7 +991,7 @@ void prefill_wide_kernel(PrefillParams p) {
     }
     l_run += (rs[0] + rs[1]) + (rs[2] + rs[3]);
 
-    // O^T += V^T . P^T over this wave's 128 channels
+    // O^T += V^T . P^T over this wave's CW channels
 #pragma unroll
     for (int hf = 0; hf < HALVES; ++hf) {
       V8 pb;

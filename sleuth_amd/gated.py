@@ -7,7 +7,7 @@ k_proj, v_proj, o_proj) attached by the loader, and the same forward(x, cos, sin
   (no mask for one token), and the output is multiplied by sigmoid(gate) before o_proj.
 
 On the GPU without autograd, the cache write and the attention run in the HIP kernels
-(forge_kv_append, forge_attn_prefill / forge_attn_decode); the norm and the partial RoPE stay
+(forge_kv_append, forge_attn_prefill_ws / forge_attn_decode); the norm and the partial RoPE stay
 in torch, as in the reference, which rounds after each. Everything else runs the reference's
 eager code. cfg needs n_heads, n_kv_heads, head_dim, n_rot and norm_eps (Qwen35Config,
 qwen35.py:60-65).

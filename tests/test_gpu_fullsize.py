@@ -50,7 +50,7 @@ def _gains(g, D):
 
 
 def test_c3_prefill_full_size():
-    """C3 prefill at its full size through forge_kv_append + forge_attn_prefill (q/k norm
+    """C3 prefill at its full size through forge_kv_append + forge_attn_prefill_ws (q/k norm
     and RoPE fused), every output against the oracle."""
     B, T, H, K, D = 4, 4096, 16, 8, 128
     g = torch.Generator().manual_seed(31)

@@ -1,7 +1,7 @@
 """Gemma 4's full-attention layers on the kernels: head dim 512 with one KV head (reference
 sleuth/forge/infer/kv_cache.py:12-13), values taken from the keys before their norm and RoPE
 (v_from_k, attention.py:108), values RMS-normalised without a gain (v_norm, 115-116) and
-attention scale 1.0 (attn_scale, 84). Head dim 512 runs on forge_attn_prefill's
+attention scale 1.0 (attn_scale, 84). Head dim 512 runs on forge_attn_prefill_ws's
 head-dim-split MFMA kernel, on the MFMA verify/decode kernel with 8 or more query heads per
 KV head, and on the split-K kernel below that (bf16/fp16).
 

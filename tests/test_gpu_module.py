@@ -270,7 +270,7 @@ def test_taps_on_the_hip_path():
 @pytest.mark.parametrize("hd", [64, 128])
 def test_document_mask_on_the_hip_path(hd, monkeypatch):
     """The reference's document mask (transformer.py:271-275, from doc_ids) over a scored
-    window runs forge_attn_prefill_docs when the documents are contiguous runs, and agrees
+    window runs forge_attn_prefill_ws with document starts when the documents are contiguous runs, and agrees
     with the module's own torch path (the reference's SDPA with _mask & same_doc); a mask
     whose document ids repeat after a gap stays on the torch path."""
     import oracle
