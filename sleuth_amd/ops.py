@@ -439,7 +439,7 @@ def attn_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: fl
                                      int(offset), int(window), float(scale), doc_ptr, doc_stride,
                                      _ptr(out), out.stride(0), out.stride(1), out.stride(2), _ptr(ws), need,
                                      _stream(dev))
-    check(st, "forge_attn_prefill")
+    check(st, "forge_attn_prefill" if doc_start is None else "forge_attn_prefill_docs")
     return out
 
 

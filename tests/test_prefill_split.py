@@ -36,6 +36,19 @@ def test_split_rule():
     assert _bytes(1, 512, 16, 8, 32, 15360) == 0 and _bytes(1, 512, 16, 3, 128, 15360) == 0
 
 
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a GPU")
+@pytest.mark.parametrize("docs,name", [(False, "forge_attn_prefill"), (True, "forge_attn_prefill_docs")])
+def test_a_rejected_call_names_its_entry_point(docs, name):
+    from sleuth_amd import ops
+
+    q, k = (torch.zeros(1, 2, 20, 64, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    odd = torch.zeros(1281, device=DEV)[1:].view(20, 64)       # tables the kernel refuses: not 16-byte aligned
+    starts = torch.zeros(1, 20, dtype=torch.int32, device=DEV) if docs else None
+    with pytest.raises(_lib.ForgeError, match=name + r"\b"):
+        ops.attn_prefill(q, k, k, scale=1.0, cos=odd, sin=odd, doc_start=starts)
+
+
 def test_workspace_too_small_is_rejected():
     lib = _lib.lib()
     need = _bytes(1, 512, 16, 8, 128, 15360)
