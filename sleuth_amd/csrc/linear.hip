@@ -284,8 +284,8 @@ struct LinRule {
   int n, k, rows;  // up to n outputs of up to k channels: up to `rows` rows
 };
 // the first line that holds a shape decides; none: 0 rows
-constexpr LinRule kLinPlainRule[] = {{4096, 4096, 16}, {8192, 2048, 16}, {16640, 512, 16}, {12288, 1024, 12}};
-constexpr LinRule kLinResidualRule[] = {{4096, 4096, 16}, {8192, 2048, 16}, {16640, 512, 16}, {12288, 1024, 12}, {4096, 16383, 4}};
+constexpr LinRule kLinPlainRule[] = {{4096, 4096, 16}, {8192, 2048, 16}, {16640, 512, 16}, {12288, 895, 12}, {12288, 1024, 16}};
+constexpr LinRule kLinResidualRule[] = {{4096, 4096, 16}, {8192, 2048, 16}, {16640, 512, 16}, {12288, 895, 12}, {12288, 1024, 16}, {4096, 16383, 4}};
 constexpr LinRule kLinNormRule[] = {{16640, 255, 16}, {1 << 30, 255, 0}, {4096, 4096, 16}, {32768, 2048, 16}, {1 << 30, 767, 0},
                                     {155648, 1024, 16}, {155648, 2048, 8}, {163840, 2048, 4}, {12288, 4096, 8}, {16384, 4096, 4}};
 constexpr LinRule kLinGatedRule[] = {{12288, 4096, 16}, {28672, 2048, 16}, {28672, 4096, 8}, {28672, 8192, 4}};

@@ -34,7 +34,7 @@ def test_rows_up_to_which_the_launch_is_taken():
     rows = _lib.lib().forge_linear_small_rows
     want = {   # plain, residual, norm, gated
         (4096, 1024): (16, 16, 16, 16), (1024, 3072): (16, 16, 16, 16), (4096, 4096): (16, 16, 16, 16),
-        (8192, 2048): (16, 16, 16, 16), (10240, 768): (12, 12, 16, 16), (6144, 4096): (0, 0, 8, 16), (5120, 5120): (0, 0, 0, 4),
+        (8192, 2048): (16, 16, 16, 16), (10240, 768): (12, 12, 16, 16), (9216, 1024): (16, 16, 16, 16), (12288, 1024): (16, 16, 16, 16), (6144, 4096): (0, 0, 8, 16), (5120, 5120): (0, 0, 0, 4),
         (4096, 14336): (0, 4, 0, 0), (4096, 16384): (0, 0, 0, 0), (14336, 4096): (0, 0, 4, 8), (28672, 8192): (0, 0, 0, 4),
         (32768, 2048): (0, 0, 16, 0), (151936, 1024): (0, 0, 16, 0), (128256, 4096): (0, 0, 0, 0),
         (163840, 2048): (0, 0, 4, 0), (131072, 512): (0, 0, 0, 0), (65536, 128): (0, 0, 0, 0), (16403, 64): (16, 16, 16, 16)}
